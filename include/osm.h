@@ -37,8 +37,11 @@
  *                      Chebyshev basis, damping and tanh (1722-1739), giving
  *                      dL/dx, dL/dc and dL/d ema_init from dL/dout and
  *                      dL/d ema_final.  With OSM_FLAG_FULL_JACOBIAN and
- *                      z_saved it is the per-chunk FusedChebyRKVv10.backward
- *                      (sdpc_kernel.py:2436-2515) of the full path.
+ *                      z_saved it is the FusedChebyRKVv10.backward
+ *                      (sdpc_kernel.py:2436-2515) of one chunk of the full
+ *                      path, dL/dc included.
+ *   osm_v10_bwd        dL/dx of the full path: FusedChebyRKVv10.backward on
+ *                      every chunk, in one launch.
  *   osm_v10_chunked_ttt  the full path of apply_cheby_rkv_v10: its chunk loop
  *                      (sdpc_kernel.py:2574-2606) of FusedChebyRKVv10.forward
  *                      launches (2353-2433) running _ortho_megakernel
@@ -245,6 +248,38 @@ typedef struct osm_v10_args {
 } osm_v10_args;
 
 /*
+ * Backward of the full path: dL/dx of every chunk, as
+ * FusedChebyRKVv10.backward (sdpc_kernel.py:2436-2515) gives it, from what
+ * osm_v10_chunked_ttt saved (out, z_save, coeff_hist) and dL/dout:
+ *
+ *   a[t]     = [|out[t]| < 1 - 1e-6] (dL/dout[t] + mu a[t+1]), a = 0 past the chunk of t
+ *   dL/dx[t] = (1-mu) a[t] gamma_h (1 - z[t]^2) p'(u[t]) / (1 + |x[t]|)^2,
+ *              gamma_h = 0.98 - 0.06 h/H, p the series of the chunk's coefficients
+ *
+ * Coefficients and momentum are constants of the chunk (the chunk loop
+ * detaches them, sdpc_kernel.py:2593-2594).  One launch, no workspace.
+ */
+typedef struct osm_v10_bwd_args {
+  int32_t abi_version;          /* = OSM_ABI_VERSION */
+  int32_t x_dtype;
+  int64_t B, S, H, hd, K;       /* 1 <= K <= 8 */
+  int64_t chunk;                /* tokens per Lion step, >= 1 */
+  const void* x;                /* [B,S,H*hd], x_dtype; lane stride 1, as all rows below */
+  int64_t x_stride_b, x_stride_s;
+  const float* grad_out;        /* [B,S,H*hd] dL/dout */
+  int64_t go_stride_b, go_stride_s;
+  const float* out;             /* [B,S,H*hd] the forward's output */
+  int64_t out_stride_b, out_stride_s;
+  const void* z_saved;          /* [B,S,H*hd] bf16 */
+  int64_t z_stride_b, z_stride_s;
+  const float* coeff_hist;      /* [ceil(S/chunk),B,H,K,hd] fp32 contiguous */
+  void* grad_x;                 /* [B,S,H*hd] dL/dx, x_dtype (overwritten) */
+  int64_t gx_stride_b, gx_stride_s;
+  float ema_momentum;
+  const float* ema_momentum_dev; /* optional device fp32 scalar: mu is read from it */
+} osm_v10_bwd_args;
+
+/*
  * Fixed-coefficient fused forward of the same kernel family: the reference's
  * _fused_clenshaw_ema_kernel (sdpc_kernel.py:988-1209), which
  * precision_tests.py:33-73 launches.  Per lane, over all S tokens:
@@ -343,6 +378,10 @@ int osm_cheby_ema_ttt(const osm_cheby_args* args, float* grad, int target, void*
 /* The full-path chunk loop described above osm_v10_args, in one launch on
  * `stream`.  Needs no workspace. */
 int osm_v10_chunked_ttt(const osm_v10_args* args, void* stream);
+
+/* The full path's backward described above osm_v10_bwd_args, in one launch
+ * on `stream`.  Needs no workspace. */
+int osm_v10_bwd(const osm_v10_bwd_args* args, void* stream);
 
 /* The fixed-coefficient forward described above osm_lut_fwd_args, in one
  * launch on `stream` (replaces a launch of _fused_clenshaw_ema_kernel,

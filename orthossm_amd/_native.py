@@ -56,6 +56,7 @@ EXPORTS = (
     "osm_cheby_ema_ttt",
     "osm_cheby_ema_bwd",
     "osm_v10_chunked_ttt",
+    "osm_v10_bwd",
     "osm_cheby_ema_lut_fwd",
 )
 
@@ -164,6 +165,39 @@ class V10Args(ctypes.Structure):
     ]
 
 
+class V10BwdArgs(ctypes.Structure):
+    """Mirror of ``osm_v10_bwd_args``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32),
+        ("x_dtype", ctypes.c_int32),
+        ("B", ctypes.c_int64),
+        ("S", ctypes.c_int64),
+        ("H", ctypes.c_int64),
+        ("hd", ctypes.c_int64),
+        ("K", ctypes.c_int64),
+        ("chunk", ctypes.c_int64),
+        ("x", ctypes.c_void_p),
+        ("x_stride_b", ctypes.c_int64),
+        ("x_stride_s", ctypes.c_int64),
+        ("grad_out", ctypes.c_void_p),
+        ("go_stride_b", ctypes.c_int64),
+        ("go_stride_s", ctypes.c_int64),
+        ("out", ctypes.c_void_p),
+        ("out_stride_b", ctypes.c_int64),
+        ("out_stride_s", ctypes.c_int64),
+        ("z_saved", ctypes.c_void_p),
+        ("z_stride_b", ctypes.c_int64),
+        ("z_stride_s", ctypes.c_int64),
+        ("coeff_hist", ctypes.c_void_p),
+        ("grad_x", ctypes.c_void_p),
+        ("gx_stride_b", ctypes.c_int64),
+        ("gx_stride_s", ctypes.c_int64),
+        ("ema_momentum", ctypes.c_float),
+        ("ema_momentum_dev", ctypes.c_void_p),
+    ]
+
+
 class LutFwdArgs(ctypes.Structure):
     """Mirror of ``osm_lut_fwd_args``."""
 
@@ -248,6 +282,8 @@ def load() -> ctypes.CDLL:
                                           ctypes.c_size_t, ctypes.c_void_p]
         lib.osm_v10_chunked_ttt.restype = ctypes.c_int
         lib.osm_v10_chunked_ttt.argtypes = [ctypes.POINTER(V10Args), ctypes.c_void_p]
+        lib.osm_v10_bwd.restype = ctypes.c_int
+        lib.osm_v10_bwd.argtypes = [ctypes.POINTER(V10BwdArgs), ctypes.c_void_p]
         lib.osm_cheby_ema_lut_fwd.restype = ctypes.c_int
         lib.osm_cheby_ema_lut_fwd.argtypes = [ctypes.POINTER(LutFwdArgs), ctypes.c_void_p]
         got = lib.osm_abi_version()

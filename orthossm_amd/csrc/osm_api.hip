@@ -525,6 +525,90 @@ int osm_v10_chunked_ttt(const osm_v10_args* a, void* stream) {
   return ok();
 }
 
+int osm_v10_bwd(const osm_v10_bwd_args* a, void* stream) {
+  if (!a) return fail(OSM_E_ARG, "args is NULL");
+  if (a->abi_version != OSM_ABI_VERSION)
+    return fail(OSM_E_ARG, "abi_version %d does not match library ABI %d", a->abi_version, OSM_ABI_VERSION);
+  if (a->B < 0 || a->S < 0 || a->H < 1 || a->hd < 1)
+    return fail(OSM_E_SHAPE, "need B, S >= 0, H, hd >= 1 (B=%lld S=%lld H=%lld hd=%lld)", (long long)a->B,
+                (long long)a->S, (long long)a->H, (long long)a->hd);
+  if (a->K < 1 || a->K > 8) return fail(OSM_E_SHAPE, "K=%lld outside [1, 8]", (long long)a->K);
+  if (a->chunk < 1) return fail(OSM_E_SHAPE, "chunk=%lld must be >= 1", (long long)a->chunk);
+  if (a->x_dtype != OSM_F32 && a->x_dtype != OSM_BF16) return fail(OSM_E_DTYPE, "x_dtype %d unsupported", a->x_dtype);
+  if (a->H > (int64_t(1) << 28) || a->hd > (int64_t(1) << 28)) return fail(OSM_E_SHAPE, "problem too large");
+  const int64_t D = a->H * a->hd;
+  if (D > (int64_t(1) << 28) || a->S >= (int64_t(1) << 31) || a->B >= (int64_t(1) << 31))
+    return fail(OSM_E_SHAPE, "problem too large");
+  if (a->B == 0 || a->S == 0) return ok();
+  if (!a->x || !a->grad_out || !a->out || !a->z_saved || !a->coeff_hist || !a->grad_x)
+    return fail(OSM_E_ARG, "x, grad_out, out, z_saved, coeff_hist and grad_x must be non-NULL");
+  const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
+  // Rows of one 256-token block, addressed from its first row, must fit a
+  // buffer descriptor's 31-bit offsets.
+  struct RowArg {
+    const void* p;
+    int64_t sb, ss;
+    int size;
+    const char* what;
+  };
+  const RowArg rows[5] = {{a->x, a->x_stride_b, a->x_stride_s, xs, "x"},
+                          {a->grad_out, a->go_stride_b, a->go_stride_s, 4, "grad_out"},
+                          {a->out, a->out_stride_b, a->out_stride_s, 4, "out"},
+                          {a->z_saved, a->z_stride_b, a->z_stride_s, 2, "z_saved"},
+                          {a->grad_x, a->gx_stride_b, a->gx_stride_s, xs, "grad_x"}};
+  // Two lanes per thread where every pair of lanes of every row starts on a
+  // two-element boundary; one lane per thread (any layout) otherwise.
+  bool pairs = a->hd % 2 == 0;
+  for (const RowArg& r : rows) {
+    if (!aligned1(r.p, r.size) || r.sb < 0 || r.ss < 0)
+      return fail(OSM_E_LAYOUT, "%s must be element-aligned with non-negative strides", r.what);
+    if (r.ss >= (int64_t(1) << 31) || (257 * r.ss + D) * r.size >= (int64_t(1) << 31))
+      return fail(OSM_E_LAYOUT, "%s token stride too large: 257 rows span more than 2 GiB", r.what);
+    pairs = pairs && (uintptr_t)r.p % (uintptr_t)(2 * r.size) == 0 && r.sb % 2 == 0 && r.ss % 2 == 0;
+  }
+  if (a->gx_stride_s < D || a->gx_stride_b < a->S * a->gx_stride_s)
+    return fail(OSM_E_LAYOUT, "grad_x rows/batches overlap");
+  if ((uintptr_t)a->coeff_hist % 4 || (uintptr_t)a->ema_momentum_dev % 4)
+    return fail(OSM_E_LAYOUT, "coeff_hist or ema_momentum_dev misaligned");
+  osm::V10BwdParams p{};
+  p.x = a->x;
+  p.gout = a->grad_out;
+  p.out = a->out;
+  p.z = a->z_saved;
+  p.hist = a->coeff_hist;
+  p.gx = a->grad_x;
+  p.mu_dev = a->ema_momentum_dev;
+  p.x_sb = a->x_stride_b;
+  p.x_ss = a->x_stride_s;
+  p.go_sb = a->go_stride_b;
+  p.go_ss = a->go_stride_s;
+  p.o_sb = a->out_stride_b;
+  p.o_ss = a->out_stride_s;
+  p.z_sb = a->z_stride_b;
+  p.z_ss = a->z_stride_s;
+  p.gx_sb = a->gx_stride_b;
+  p.gx_ss = a->gx_stride_s;
+  p.B = (int)a->B;
+  p.S = (int)a->S;
+  p.H = (int)a->H;
+  p.hd = (int)a->hd;
+  p.K = (int)a->K;
+  p.D = (int)D;
+  p.chunk = (int)std::min<int64_t>(a->chunk, a->S);
+  p.n_chunks = (int)((a->S + p.chunk - 1) / p.chunk);
+  p.n_lbd = (int)((D + osm::v10_bwd_lanes() - 1) / osm::v10_bwd_lanes());
+  const int64_t n_lb = a->B * (int64_t)p.n_lbd;
+  if (n_lb >= (int64_t(1) << 31) || n_lb * p.n_chunks >= (int64_t(1) << 31) - 8)
+    return fail(OSM_E_SHAPE, "problem too large");
+  p.n_items = (int)(n_lb * p.n_chunks);
+  p.items_per_xcd = (p.n_items + 7) / 8;
+  p.mu = a->ema_momentum;
+  const hipError_t e =
+      osm::launch_v10_bwd(p, a->x_dtype, pairs ? 2 : 1, a->K <= 4 ? 4 : 8, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "full-path backward launch");
+  return ok();
+}
+
 int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* a, void* stream) {
   if (!a) return fail(OSM_E_ARG, "args is NULL");
   if (a->abi_version != OSM_ABI_VERSION)

@@ -363,6 +363,21 @@ __device__ __forceinline__ double mono_coef(const float (&cm)[4]) {
   return acc;
 }
 
+// Which form a tile evaluates its series in.  The monomial form (Horner, K-1
+// FMAs) is exact in exact arithmetic, but its coefficients cancel: its fp32
+// error grows with sum_j |a_j| (a_j scaled as stored, in exp2 units), about
+// ten times faster than Clenshaw's with the size of the Chebyshev
+// coefficients.  A tile uses the monomial form while every scaled monomial
+// coefficient of its lanes satisfies |a_j| <= kMonoBound (NaN counts as
+// above), else the Chebyshev form (Clenshaw, 2(K-1) operations) on c_k
+// scaled the same way.  The bound keeps every draw of the benchmark's
+// c_k ~ N(0, 1/(k+1)^2) (largest |a_j|, a_5 = 2 log2(e) (16 c_5 - 112 c_7),
+// has a standard deviation of 41) and every coefficient set inside the
+// full path's Lion bound 8.31/(k+1)^1.5 (|a_5| <= 145) on Horner, and
+// sends coefficients of order one and larger (c_k ~ N(0, 1): |a_5| ~ 330)
+// to Clenshaw.
+constexpr float kMonoBound = 256.0f;
+
 // Horner evaluation of sum_j a[j] u^j.
 template <int KP>
 __device__ __forceinline__ float horner(float u, const float (&a)[KP]) {

@@ -224,6 +224,23 @@ struct V10FixedParams : V10Params {
   int clamp_tile;              // tokens between clamps of the carried state
 };
 
+// Backward of the full path (osm_v10_bwd): dL/dx of every chunk, one
+// workgroup per (batch row, chunk, 64-lane lane-block).  Needs no workspace.
+struct V10BwdParams {
+  const void* x;
+  const float* gout;           // dL/dout
+  const float* out;            // the saved output (the clamp mask)
+  const void* z;               // the saved z, bf16
+  const float* hist;           // [n_chunks][B,H,K,hd]
+  void* gx;                    // dL/dx, dtype of x
+  const float* mu_dev;         // device scalar overriding mu, or NULL
+  int64_t x_sb, x_ss, go_sb, go_ss, o_sb, o_ss, z_sb, z_ss, gx_sb, gx_ss;
+  int B, S, H, hd, K, D, chunk, n_chunks, n_lbd;
+  int n_items;                 // B * n_chunks * n_lbd
+  int items_per_xcd;           // ceil(n_items / 8); grid = 8 * items_per_xcd
+  float mu;
+};
+
 // Multiplier and shift that divide by v (1 <= v < 2^31) for dividends
 // 0 <= n < 2^31: s = ceil(log2 v), m = floor(2^32 (2^s - v) / v) + 1
 // (Granlund and Montgomery, "Division by invariant integers using
@@ -250,6 +267,8 @@ hipError_t launch_ttt(const FwdParams& p, float* grad, int x_dtype, int out_dtyp
 hipError_t launch_bwd(const BwdParams& p, int x_dtype, int out_dtype, bool dyn, int tile, int kpad,
                       hipStream_t stream);
 hipError_t launch_v10(const V10Params& p, int x_dtype, bool use_lut, int kpad, hipStream_t stream);
+int v10_bwd_lanes();   // lanes per lane-block of launch_v10_bwd
+hipError_t launch_v10_bwd(const V10BwdParams& p, int x_dtype, int lpt, int kpad, hipStream_t stream);
 hipError_t launch_v10_fixed(const V10FixedParams& p, int x_dtype, bool use_lut, int kpad, hipStream_t stream);
 hipError_t launch_fill_zero(void* ptr, size_t bytes, hipStream_t stream);
 hipError_t launch_copy_state(const float* src, float* dst, size_t n, hipStream_t stream);

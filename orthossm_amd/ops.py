@@ -668,44 +668,52 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     return out, x_norm, tanh_y, ema_final
 
 
+def _rows(t: torch.Tensor, dtype: torch.dtype, dev: torch.device) -> torch.Tensor:
+    """``t`` as [B,S,D] rows the kernels address: ``dtype`` on ``dev``, lane
+    stride 1, non-negative strides of at most 2^20 elements a token."""
+    if t.dtype is not dtype or t.device != dev:
+        t = t.to(device=dev, dtype=dtype)
+    if t.stride(2) != 1 or not 0 <= t.stride(1) <= 1 << 20 or t.stride(0) < 0:
+        t = t.contiguous()
+    return t
+
+
 def _v10_backward(x, out, z, hist, grad_out, n_heads, ema_momentum, chunk, need_coeffs):
     """The full path's backward (FusedChebyRKVv10.backward, sdpc_kernel.py:
     2436-2515) on every chunk: the adjoint restarts at each chunk end, the
     chunk's own coefficients enter, 1 - z^2 comes from the saved bf16 z, the
-    mask from the output, dL/dx = ... / (1+|x|)^2.  Chunks become batch rows
-    of one backward call (per batch row when S is not a multiple of chunk).
-    Returns (grad_x, grad_coeffs of the first chunk or None)."""
+    mask from the output, dL/dx = ... / (1+|x|)^2.  One osm_v10_bwd launch;
+    dL/dc (one chunk only) comes from osm_cheby_ema_bwd.  Returns (grad_x,
+    grad_coeffs of the first chunk or None)."""
     B, S, D = x.shape
     n_chunks, _, H, K, hd = hist.shape
     dev = x.device
-    h = torch.arange(H, dtype=torch.float32, device=dev)
-    damping = (0.98 - 0.06 * h / H).contiguous()
-    lam = head_momentum(ema_momentum, H, dev)
-    go = grad_out.to(dtype=torch.float32).contiguous()
-    xc = x.contiguous()
-    gx = torch.empty_like(xc)
-    kw = dict(clamp=True, nan_policy="zero_u", need_coeffs=False, full_jacobian=True)
-    n_full = S // chunk
-    if n_chunks == 1:
-        gxa, gca, _ = cheby_ema_backward(xc, hist[0], damping, lam, out, go, z_saved=z,
-                                         **dict(kw, need_coeffs=need_coeffs))
-        return gxa, gca
-    def rows(t, b0, b1, nc):
-        return t[b0:b1, :nc * chunk].reshape((b1 - b0) * nc, chunk, D)
-    if S % chunk == 0:
-        cs = hist.permute(1, 0, 2, 3, 4).reshape(B * n_chunks, H, K, hd)
-        gxa, _, _ = cheby_ema_backward(rows(xc, 0, B, n_chunks), cs, damping, lam, rows(out, 0, B, n_chunks),
-                                       rows(go, 0, B, n_chunks), z_saved=rows(z, 0, B, n_chunks), **kw)
-        return gxa.reshape(B, S, D), None
-    for b in range(B):
-        gxa, _, _ = cheby_ema_backward(rows(xc, b, b + 1, n_full), hist[:n_full, b].contiguous(), damping, lam,
-                                       rows(out, b, b + 1, n_full), rows(go, b, b + 1, n_full),
-                                       z_saved=rows(z, b, b + 1, n_full), **kw)
-        gx[b, :n_full * chunk] = gxa.reshape(n_full * chunk, D)
-    t0 = n_full * chunk
-    gxt, _, _ = cheby_ema_backward(xc[:, t0:], hist[n_full], damping, lam, out[:, t0:], go[:, t0:],
-                                   z_saved=z[:, t0:], **kw)
-    gx[:, t0:] = gxt
+    if need_coeffs:
+        h = torch.arange(H, dtype=torch.float32, device=dev)
+        damping = (0.98 - 0.06 * h / H).contiguous()
+        gx, gc, _ = cheby_ema_backward(x.contiguous(), hist[0], damping, head_momentum(ema_momentum, H, dev), out,
+                                       grad_out.to(dtype=torch.float32).contiguous(), clamp=True,
+                                       nan_policy="zero_u", z_saved=z, full_jacobian=True)
+        return gx, gc
+    lib = nat.load()
+    xr = _rows(x, x.dtype if x.dtype in (torch.float32, torch.bfloat16) else torch.float32, dev)
+    go, out, z = _rows(grad_out, torch.float32, dev), _rows(out, torch.float32, dev), _rows(z, torch.bfloat16, dev)
+    hist = hist.contiguous()
+    gx = torch.empty((B, S, D), device=dev, dtype=xr.dtype)
+    a = nat.V10BwdArgs()
+    a.abi_version, a.x_dtype = nat.ABI_VERSION, _dtype_code(xr.dtype)
+    a.B, a.S, a.H, a.hd, a.K, a.chunk = B, S, H, hd, K, int(chunk)
+    a.x, a.x_stride_b, a.x_stride_s = xr.data_ptr(), xr.stride(0), xr.stride(1)
+    a.grad_out, a.go_stride_b, a.go_stride_s = go.data_ptr(), go.stride(0), go.stride(1)
+    a.out, a.out_stride_b, a.out_stride_s = out.data_ptr(), out.stride(0), out.stride(1)
+    a.z_saved, a.z_stride_b, a.z_stride_s = z.data_ptr(), z.stride(0), z.stride(1)
+    a.coeff_hist = hist.data_ptr()
+    a.grad_x, a.gx_stride_b, a.gx_stride_s = gx.data_ptr(), gx.stride(0), gx.stride(1)
+    mu_val, mu_dev = device_momentum(ema_momentum, dev)
+    a.ema_momentum = mu_val
+    a.ema_momentum_dev = mu_dev.data_ptr() if mu_dev is not None else None
+    nat.check(lib.osm_v10_bwd(ctypes.byref(a), ctypes.c_void_p(_current_stream(dev))))
+    keep = (xr, go, out, z, hist, mu_dev)  # noqa: F841  (alive until the launch is queued)
     return gx, None
 
 

@@ -7,7 +7,7 @@ import torch
 from helpers import compare_v10 as compare
 from oracle import v10_full as V
 from orthossm_amd import apply_cheby_rkv_v10
-from orthossm_amd.ops import v10_chunked_ttt
+from orthossm_amd.ops import _v10_backward, v10_chunked_ttt
 
 pytestmark = pytest.mark.gpu
 
@@ -160,6 +160,48 @@ def test_v10_full_path_grad_x(dev, B, S, H, hd, K, chunk):
     gx, gc, wx, _ = _grads_vs_oracle(dev, B, S, H, hd, K, chunk, seed=B + S)
     assert gc is None                           # the chunk loop detaches the coefficients
     _close(gx, wx, "grad_x")
+
+
+@pytest.mark.parametrize("B,S,H,hd,K,chunk,dt,layout", [
+    (1, 1, 1, 1, 1, 256, torch.float32, ""),             # one token, one lane, one coefficient
+    (2, 300, 3, 5, 8, 64, torch.float32, ""),            # odd head size: one lane per thread; 64-token blocks
+    (1, 515, 2, 50, 8, 128, torch.bfloat16, ""),         # lane-blocks cut at D = 100; a 3-token last chunk
+    (2, 700, 2, 32, 4, 129, torch.float32, "strided"),   # just past 128: the 256-token block; x a wider tensor's view
+    (1, 1100, 4, 16, 6, 600, torch.float32, "expand"),   # chunks of three blocks; dL/dout of stride 0
+    (3, 513, 1, 66, 8, 256, torch.bfloat16, "odd"),      # rows off two-element boundaries
+    (2, 520, 2, 64, 8, 256, torch.float32, "big"),       # coefficients past the monomial bound
+])
+def test_v10_backward_every_chunk(dev, B, S, H, hd, K, chunk, dt, layout):
+    """osm_v10_bwd against the float64 restatement on its own inputs, with
+    outputs at the clamp mask's bound.  Each value passes about twenty fp32
+    roundings (2^-24 each) of terms up to ten times its own size (the
+    adjoint's sum and the series), so 1e-5 of the largest value bounds the
+    error; a bf16 result is rounded once more (2^-9 of itself)."""
+    D, n = H * hd, (S + chunk - 1) // chunk
+    gen = torch.Generator().manual_seed(S + hd)
+    x = torch.randn(B, S, D, generator=gen).to(dt)
+    out = (torch.randn(B, S, D, generator=gen) * 0.5).clamp(-1, 1)
+    z = torch.tanh(torch.randn(B, S, D, generator=gen)).bfloat16()
+    hist = torch.randn(n, B, H, K, hd, generator=gen) * (30.0 if layout == "big" else 1.0)
+    hist = hist / torch.arange(1, K + 1).view(K, 1)
+    go = torch.randn(B, S, D, generator=gen)
+    xd, god = x.to(dev), go.to(dev)
+    if layout in ("strided", "odd"):
+        pad = 3 if layout == "odd" else 4
+        wide = torch.zeros(B, S, D + pad, dtype=dt, device=dev)
+        wide[..., pad // 2:pad // 2 + D] = xd
+        xd = wide[..., pad // 2:pad // 2 + D]
+    elif layout == "expand":
+        go = torch.full_like(go, 0.7)
+        god = torch.tensor(0.7, device=dev).expand(B, S, D)
+    gx, gc = _v10_backward(xd, out.to(dev), z.to(dev), hist.to(dev), god, H, 0.9, chunk, False)
+    torch.cuda.synchronize()
+    assert gc is None and gx.dtype == dt
+    want, _ = V.v10_backward(x.float().numpy(), out.numpy(), z.float().numpy(), hist.numpy(), go.numpy(),
+                             n_heads=H, ema_momentum=float(np.float32(0.9)), chunk=chunk)
+    err = np.abs(gx.cpu().double().numpy() - want)
+    bound = 1e-5 * np.abs(want).max() + (2.0 ** -8 * np.abs(want) if dt is torch.bfloat16 else 0.0)
+    assert (err <= bound).all(), f"max error {err.max():.3e} of {np.abs(want).max():.3e}"
 
 
 def test_v10_single_chunk_grads_and_nan(dev):

@@ -388,6 +388,16 @@ int osm_v10_bwd(const osm_v10_bwd_args* args, void* stream);
  * sdpc_kernel.py:988-1209).  Needs no workspace. */
 int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* args, void* stream);
 
+/* The same forward with a workspace (as described at the head of this
+ * file): a single-pass scan over all tiles of the sequence at once instead
+ * of one workgroup walking each group of lanes.  Takes the same arguments
+ * and gives the same results up to rounding; where the scan does not apply
+ * (osm_lut_fwd_workspace_bytes gives 0: a decay outside [0.25, 1], a short
+ * sequence of few lanes, or invalid arguments) it is osm_cheby_ema_lut_fwd,
+ * and the workspace may be NULL. */
+size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* args);
+int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Backward of osm_cheby_ema_fwd: writes grad_x and, when non-NULL,
  * grad_coeffs and grad_init.  Replaces the backward listed in the header
  * comment. */

@@ -28,6 +28,7 @@ TARGET_SOFTSIGN = 1
 OP_FWD = 0
 OP_TTT = 1
 OP_BWD = 2
+OP_LUT = 3   # key of the fixed-coefficient scan's workspaces (not an osm_op)
 V10_USE_LUT = 0x1
 
 STATUS = {
@@ -58,6 +59,8 @@ EXPORTS = (
     "osm_v10_chunked_ttt",
     "osm_v10_bwd",
     "osm_cheby_ema_lut_fwd",
+    "osm_lut_fwd_workspace_bytes",
+    "osm_cheby_ema_lut_fwd_ws",
 )
 
 
@@ -286,6 +289,11 @@ def load() -> ctypes.CDLL:
         lib.osm_v10_bwd.argtypes = [ctypes.POINTER(V10BwdArgs), ctypes.c_void_p]
         lib.osm_cheby_ema_lut_fwd.restype = ctypes.c_int
         lib.osm_cheby_ema_lut_fwd.argtypes = [ctypes.POINTER(LutFwdArgs), ctypes.c_void_p]
+        lib.osm_lut_fwd_workspace_bytes.restype = ctypes.c_size_t
+        lib.osm_lut_fwd_workspace_bytes.argtypes = [ctypes.POINTER(LutFwdArgs)]
+        lib.osm_cheby_ema_lut_fwd_ws.restype = ctypes.c_int
+        lib.osm_cheby_ema_lut_fwd_ws.argtypes = [ctypes.POINTER(LutFwdArgs), ctypes.c_void_p, ctypes.c_size_t,
+                                                 ctypes.c_void_p]
         got = lib.osm_abi_version()
         if got != ABI_VERSION:
             raise ImportError(f"orthossm_amd: library ABI {got} != binding ABI {ABI_VERSION}; rebuild")

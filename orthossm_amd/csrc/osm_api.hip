@@ -222,6 +222,7 @@ struct Layout {
            kpad == o.kpad && dyn == o.dyn && op == o.op;
   }
 };
+constexpr int kLayoutLut = 3;   // Layout::op of the fixed-coefficient scan (the osm_op values are 0 to 2)
 const Layout kZeroed{-1, -1, -1, -1, -1, -1, false, -1};
 std::mutex g_ws_mu;
 std::unordered_map<uintptr_t, Layout> g_ws_layout;
@@ -293,6 +294,134 @@ int run_empty(const osm_cheby_args* a, hipStream_t stream) {
     if (e != hipSuccess) return hip_fail(e, "state copy launch");
   }
   return ok();
+}
+
+// Validates the fixed-coefficient forward's arguments without touching the
+// GPU.  Returns OSM_OK or an error; B == 0 is valid (nothing to do).
+int check_lut(const osm_lut_fwd_args* a) {
+  if (!a) return fail(OSM_E_ARG, "args is NULL");
+  if (a->abi_version != OSM_ABI_VERSION)
+    return fail(OSM_E_ARG, "abi_version %d does not match library ABI %d", a->abi_version, OSM_ABI_VERSION);
+  if (a->flags & ~OSM_V10_USE_LUT) return fail(OSM_E_ARG, "unknown flag bits 0x%x", a->flags);
+  if (a->B < 0 || a->S < 0 || a->H < 1 || a->hd < 1)
+    return fail(OSM_E_SHAPE, "need B, S >= 0, H, hd >= 1 (B=%lld S=%lld H=%lld hd=%lld)", (long long)a->B,
+                (long long)a->S, (long long)a->H, (long long)a->hd);
+  // The reference kernel loads eight coefficients at most (sdpc_kernel.py:1047-1054).
+  if (a->K < 1 || a->K > 8) return fail(OSM_E_SHAPE, "K=%lld outside [1, 8]", (long long)a->K);
+  // The carried state is clamped between waves of 16 or 32 tokens.
+  if (a->clamp_tile < 16 || a->clamp_tile % 16 || a->clamp_tile >= (int64_t(1) << 30))
+    return fail(OSM_E_SHAPE, "clamp_tile=%lld must be a multiple of 16", (long long)a->clamp_tile);
+  if (a->x_dtype != OSM_F32 && a->x_dtype != OSM_BF16) return fail(OSM_E_DTYPE, "x_dtype %d unsupported", a->x_dtype);
+  const int64_t D = a->H * a->hd;
+  if (D > (int64_t(1) << 28) || a->S >= (int64_t(1) << 31)) return fail(OSM_E_SHAPE, "problem too large");
+  if (a->B == 0) return OSM_OK;
+  // (S = 0 reads and writes no rows: only ema_final, from ema_init)
+  if (a->S > 0 && (!a->x || !a->coeffs || !a->out || ((a->flags & OSM_V10_USE_LUT) && !a->lut)))
+    return fail(OSM_E_ARG, "x, coeffs, out (and lut with OSM_V10_USE_LUT) must be non-NULL");
+  const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
+  if ((uintptr_t)a->x % xs || a->x_stride_b < 0 || a->x_stride_s < 0)
+    return fail(OSM_E_LAYOUT, "x must be element-aligned with non-negative strides");
+  // Row outputs: aligned, rows and batches not overlapping.
+  struct RowOut {
+    const float* p;
+    int64_t sb, ss;
+    const char* what;
+  };
+  const RowOut outs[3] = {{a->out, a->out_stride_b, a->out_stride_s, "out"},
+                          {a->x_norm, a->xn_stride_b, a->xn_stride_s, "x_norm"},
+                          {a->tanh_y, a->ty_stride_b, a->ty_stride_s, "tanh_y"}};
+  const int64_t lim = int64_t(1) << 31;
+  const int64_t blk_rows = osm::kV10Groups * osm::kV10Run + 1;
+  for (const RowOut& o : outs) {
+    if (!o.p) continue;
+    if ((uintptr_t)o.p % 4 || o.ss < D || o.sb < a->S * o.ss)
+      return fail(OSM_E_LAYOUT, "%s misaligned or its rows/batches overlap", o.what);
+    if ((blk_rows * o.ss + D) * 4 >= lim) return fail(OSM_E_LAYOUT, "%s token stride too large", o.what);
+  }
+  if ((blk_rows * a->x_stride_s + D) * xs >= lim)
+    return fail(OSM_E_LAYOUT, "token stride too large: 257 rows span more than 2 GiB");
+  if (a->c_stride_b < 0 || a->c_stride_h < 0 || a->c_stride_k < 0)
+    return fail(OSM_E_LAYOUT, "coeffs strides must be non-negative");
+  if (a->ema_init && ((uintptr_t)a->ema_init % 4 || a->init_stride_b < 0))
+    return fail(OSM_E_LAYOUT, "ema_init misaligned or with a negative stride");
+  if (a->ema_final && ((uintptr_t)a->ema_final % 4 || a->final_stride_b < D))
+    return fail(OSM_E_LAYOUT, "ema_final misaligned or its rows overlap");
+  return OSM_OK;
+}
+
+osm::V10FixedParams lut_params(const osm_lut_fwd_args* a) {
+  osm::V10FixedParams p{};
+  p.x = a->x;
+  p.out = a->out;
+  p.coeffs = a->coeffs;
+  p.lut = a->lut;
+  p.x_sb = a->x_stride_b;
+  p.x_ss = a->x_stride_s;
+  p.o_sb = a->out_stride_b;
+  p.o_ss = a->out_stride_s;
+  p.c_sb = a->c_stride_b;
+  p.c_sh = a->c_stride_h;
+  p.c_sk = a->c_stride_k;
+  p.B = (int)a->B;
+  p.S = (int)a->S;
+  p.H = (int)a->H;
+  p.hd = (int)a->hd;
+  p.K = (int)a->K;
+  p.D = (int)(a->H * a->hd);
+  p.chunk = (int)std::max<int64_t>(a->S, 1);   // one chunk; none when S = 0
+  p.mu = a->ema_momentum;
+  p.ema_init = a->ema_init;
+  p.init_sb = a->init_stride_b;
+  p.ema_final = a->ema_final;
+  p.final_sb = a->final_stride_b;
+  p.xnorm = a->x_norm;
+  p.xn_sb = a->xn_stride_b;
+  p.xn_ss = a->xn_stride_s;
+  p.tanhy = a->tanh_y;
+  p.ty_sb = a->ty_stride_b;
+  p.ty_ss = a->ty_stride_s;
+  p.clamp_tile = (int)a->clamp_tile;
+  return p;
+}
+
+// Geometry of the scan (osm_lut.hip) for these arguments, or n_tiles = 0
+// where the walk of osm_v10.hip serves the call: a decay outside [0.25, 1] (a
+// negative one reverses the clamp, one above 1 lets later clamps bind), or a
+// sequence the walk does in one block on one round of workgroups: at most 256
+// tokens and 2048 lanes (256 workgroups of 8).  Measured on MI355X, K=8, walk
+// against scan: 6.4 and 7.9 us at B=1 S=256 D=512, 7.2 and 8.4 at B=4, 10.1
+// and 8.6 at B=8; 8.7 and 8.0 at B=1 S=384.
+Geometry lut_scan_shape(const osm_lut_fwd_args* a) {
+  Geometry geo;
+  if (!(a->ema_momentum >= 0.25f && a->ema_momentum <= 1.0f) || a->B == 0) return geo;
+  if (a->S == 0 || (a->S <= 256 && a->B * a->H * a->hd <= 2048)) return geo;
+  const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
+  auto pairs = [](const void* p, int size, int64_t sb, int64_t ss) {
+    return !p || ((uintptr_t)p % (uintptr_t)(2 * size) == 0 && sb % 2 == 0 && ss % 2 == 0);
+  };
+  const bool two = a->hd % 2 == 0 && pairs(a->x, xs, a->x_stride_b, a->x_stride_s) &&
+                   pairs(a->out, 4, a->out_stride_b, a->out_stride_s) &&
+                   pairs(a->x_norm, 4, a->xn_stride_b, a->xn_stride_s) &&
+                   pairs(a->tanh_y, 4, a->ty_stride_b, a->ty_stride_s);
+  static_assert(osm::LutTile::TILE == osm::LutTileGeneric::TILE &&
+                    osm::LutTileSmall::TILE == osm::LutTileGenericSmall::TILE,
+                "one and two lanes per thread cut the sequence alike");
+  const int64_t n_lbd = (a->H * a->hd + 63) / 64, n_lb = a->B * n_lbd;
+  if (a->B >= (int64_t(1) << 31) || n_lb >= (int64_t(1) << 31) - 8) return geo;
+  auto tiles = [&](int64_t t) { return (a->S + t - 1) / t; };
+  constexpr int64_t kCus = 256;
+  const int tile = n_lb * tiles(osm::LutTile::TILE) >= kCus ? osm::LutTile::TILE : osm::LutTileSmall::TILE;
+  const int64_t n_tiles = tiles(tile);
+  const int64_t n_lb_pad = (n_lb + 7) / 8 * 8;
+  if (n_lb_pad * n_tiles >= (int64_t(1) << 31)) return geo;
+  geo.n_lbd = (int)n_lbd;
+  geo.n_lb = (int)n_lb;
+  geo.n_lb_pad = (int)n_lb_pad;
+  geo.n_tiles = (int)n_tiles;
+  geo.tile = tile;
+  geo.lpt = two ? 2 : 1;
+  geo.kpad = a->K <= 4 ? 4 : 8;
+  return geo;
 }
 
 }  // namespace
@@ -610,92 +739,52 @@ int osm_v10_bwd(const osm_v10_bwd_args* a, void* stream) {
 }
 
 int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* a, void* stream) {
-  if (!a) return fail(OSM_E_ARG, "args is NULL");
-  if (a->abi_version != OSM_ABI_VERSION)
-    return fail(OSM_E_ARG, "abi_version %d does not match library ABI %d", a->abi_version, OSM_ABI_VERSION);
-  if (a->flags & ~OSM_V10_USE_LUT) return fail(OSM_E_ARG, "unknown flag bits 0x%x", a->flags);
-  if (a->B < 0 || a->S < 0 || a->H < 1 || a->hd < 1)
-    return fail(OSM_E_SHAPE, "need B, S >= 0, H, hd >= 1 (B=%lld S=%lld H=%lld hd=%lld)", (long long)a->B,
-                (long long)a->S, (long long)a->H, (long long)a->hd);
-  // The reference kernel loads eight coefficients at most (sdpc_kernel.py:1047-1054).
-  if (a->K < 1 || a->K > 8) return fail(OSM_E_SHAPE, "K=%lld outside [1, 8]", (long long)a->K);
-  // The carried state is clamped between waves of 16 or 32 tokens.
-  if (a->clamp_tile < 16 || a->clamp_tile % 16 || a->clamp_tile >= (int64_t(1) << 30))
-    return fail(OSM_E_SHAPE, "clamp_tile=%lld must be a multiple of 16", (long long)a->clamp_tile);
-  if (a->x_dtype != OSM_F32 && a->x_dtype != OSM_BF16) return fail(OSM_E_DTYPE, "x_dtype %d unsupported", a->x_dtype);
-  const int64_t D = a->H * a->hd;
-  if (D > (int64_t(1) << 28) || a->S >= (int64_t(1) << 31)) return fail(OSM_E_SHAPE, "problem too large");
+  const int rc = check_lut(a);
+  if (rc != OSM_OK) return rc;
   if (a->B == 0) return ok();
-  // (S = 0 reads and writes no rows: only ema_final, from ema_init)
-  if (a->S > 0 && (!a->x || !a->coeffs || !a->out || ((a->flags & OSM_V10_USE_LUT) && !a->lut)))
-    return fail(OSM_E_ARG, "x, coeffs, out (and lut with OSM_V10_USE_LUT) must be non-NULL");
-  const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
-  if ((uintptr_t)a->x % xs || a->x_stride_b < 0 || a->x_stride_s < 0)
-    return fail(OSM_E_LAYOUT, "x must be element-aligned with non-negative strides");
-  // Row outputs: aligned, rows and batches not overlapping.
-  struct RowOut {
-    const float* p;
-    int64_t sb, ss;
-    const char* what;
-  };
-  const RowOut outs[3] = {{a->out, a->out_stride_b, a->out_stride_s, "out"},
-                          {a->x_norm, a->xn_stride_b, a->xn_stride_s, "x_norm"},
-                          {a->tanh_y, a->ty_stride_b, a->ty_stride_s, "tanh_y"}};
-  const int64_t lim = int64_t(1) << 31;
-  const int64_t blk_rows = osm::kV10Groups * osm::kV10Run + 1;
-  for (const RowOut& o : outs) {
-    if (!o.p) continue;
-    if ((uintptr_t)o.p % 4 || o.ss < D || o.sb < a->S * o.ss)
-      return fail(OSM_E_LAYOUT, "%s misaligned or its rows/batches overlap", o.what);
-    if ((blk_rows * o.ss + D) * 4 >= lim) return fail(OSM_E_LAYOUT, "%s token stride too large", o.what);
-  }
-  if ((blk_rows * a->x_stride_s + D) * xs >= lim)
-    return fail(OSM_E_LAYOUT, "token stride too large: 257 rows span more than 2 GiB");
-  if (a->c_stride_b < 0 || a->c_stride_h < 0 || a->c_stride_k < 0)
-    return fail(OSM_E_LAYOUT, "coeffs strides must be non-negative");
-  if (a->ema_init && ((uintptr_t)a->ema_init % 4 || a->init_stride_b < 0))
-    return fail(OSM_E_LAYOUT, "ema_init misaligned or with a negative stride");
-  if (a->ema_final && ((uintptr_t)a->ema_final % 4 || a->final_stride_b < D))
-    return fail(OSM_E_LAYOUT, "ema_final misaligned or its rows overlap");
-  osm::V10FixedParams p{};
-  p.x = a->x;
-  p.out = a->out;
-  p.coeffs = a->coeffs;
-  p.lut = a->lut;
-  p.x_sb = a->x_stride_b;
-  p.x_ss = a->x_stride_s;
-  p.o_sb = a->out_stride_b;
-  p.o_ss = a->out_stride_s;
-  p.c_sb = a->c_stride_b;
-  p.c_sh = a->c_stride_h;
-  p.c_sk = a->c_stride_k;
-  p.B = (int)a->B;
-  p.S = (int)a->S;
-  p.H = (int)a->H;
-  p.hd = (int)a->hd;
-  p.K = (int)a->K;
-  p.D = (int)D;
-  p.chunk = (int)std::max<int64_t>(a->S, 1);   // one chunk; none when S = 0
+  osm::V10FixedParams p = lut_params(a);
   // Waves of 32 tokens with 8 lanes per workgroup, 16 with 16 lanes: the
   // clamp boundaries fall between waves.
   p.lanes = a->clamp_tile % 32 ? 16 : osm::v10_lanes(a->B, a->H, a->hd);
   p.n_lg = (int)((a->hd + p.lanes - 1) / p.lanes);
-  p.mu = a->ema_momentum;
-  p.ema_init = a->ema_init;
-  p.init_sb = a->init_stride_b;
-  p.ema_final = a->ema_final;
-  p.final_sb = a->final_stride_b;
-  p.xnorm = a->x_norm;
-  p.xn_sb = a->xn_stride_b;
-  p.xn_ss = a->xn_stride_s;
-  p.tanhy = a->tanh_y;
-  p.ty_sb = a->ty_stride_b;
-  p.ty_ss = a->ty_stride_s;
-  p.clamp_tile = (int)a->clamp_tile;
   if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31)) return fail(OSM_E_SHAPE, "problem too large");
   const hipError_t e = osm::launch_v10_fixed(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0, a->K <= 4 ? 4 : 8,
                                              static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "fixed-coefficient forward launch");
+  return ok();
+}
+
+size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* a) {
+  if (check_lut(a) != OSM_OK) return 0;
+  const Geometry geo = lut_scan_shape(a);
+  return geo.n_tiles ? osm::fwd_workspace_bytes(geo.n_lb, geo.n_tiles, geo.lanes, false) : 0;
+}
+
+int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
+  int rc = check_lut(a);
+  if (rc != OSM_OK) return rc;
+  const Geometry geo = lut_scan_shape(a);
+  if (!geo.n_tiles) return osm_cheby_ema_lut_fwd(a, stream);
+  const size_t need = osm::fwd_workspace_bytes(geo.n_lb, geo.n_tiles, geo.lanes, false);
+  rc = check_ws(geo, OSM_OP_FWD, (int)a->K, workspace, workspace_bytes);
+  if (rc != OSM_OK) return rc;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  rc = prepare_workspace(workspace, need, geo, kLayoutLut, st);
+  if (rc != OSM_OK) return rc;
+  osm::LutScanParams p{};
+  static_cast<osm::V10FixedParams&>(p) = lut_params(a);
+  p.hdr = reinterpret_cast<unsigned*>(workspace);
+  p.slots = reinterpret_cast<unsigned long long*>(static_cast<char*>(workspace) + osm::kHeaderBytes);
+  osm::div_magic((uint32_t)a->hd, &p.hd_magic, &p.hd_shift);
+  p.n_lbd = geo.n_lbd;
+  p.n_lb = geo.n_lb;
+  p.n_lb_pad = geo.n_lb_pad;
+  p.n_tiles = geo.n_tiles;
+  p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
+  p.poll_limit = osm::kSpinLimit;
+  const hipError_t e = osm::launch_lut_scan(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0,
+                                            osm::FwdShape{geo.tile, geo.lanes, geo.lpt}, geo.kpad, st);
+  if (e != hipSuccess) return hip_fail(e, "fixed-coefficient scan launch");
   return ok();
 }
 

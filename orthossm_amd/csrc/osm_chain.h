@@ -209,9 +209,10 @@ struct LookBack {
 
 template <class G, bool DYN>
 __device__ __forceinline__ void look_back_issue(LookBack<G, DYN>& st, const ThreadPos& q, const TileInfo& ti,
-                                                const LaneSlots& ls) {
+                                                const LaneSlots& ls, int g0_min = 0) {
   const int ll = look_lane<G>(q);
-  st.g0 = (ti.tile / G::CKPT) * G::CKPT;
+  // g0_min: first tile of the group when an extra checkpoint precedes it
+  st.g0 = max((ti.tile / G::CKPT) * G::CKPT, g0_min);
   st.beg = st.g0 + (q.wave % G::WPS) * G::WPT;
   st.end = min(st.beg + G::WPT, ti.tile);
 #pragma unroll

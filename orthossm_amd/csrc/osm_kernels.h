@@ -224,6 +224,27 @@ struct V10FixedParams : V10Params {
   int clamp_tile;              // tokens between clamps of the carried state
 };
 
+// The same forward as a single-pass scan over tiles (osm_lut.hip), chained by
+// the look-back: for 0.25 <= mu <= 1 and a caller's workspace.  128-token
+// tiles where they give every CU one, else 64 (a tile of 128 tokens holds
+// its CU's VALUs ~3.8 us): on MI355X, D=512 K=8, 8.5 against 10.5 us at B=4
+// S=512 (128 tiles of 128 tokens), 12.2 against 11.9 at B=2 S=2000 D=400
+// (224), 21.0 against 16.0 at B=2 S=4096 (512).  One lane per thread where
+// rows are off two-element boundaries.
+using LutTile = TileGeo<2, 8, 8, 64, 1>;              // 128 tokens x 64 lanes
+using LutTileSmall = TileGeo<2, 8, 4, 64, 1>;         // 64 tokens
+using LutTileGeneric = TileGeo<1, 8, 16, 64, 1>;      // 128 tokens
+using LutTileGenericSmall = TileGeo<1, 8, 8, 64, 1>;  // 64 tokens
+struct LutScanParams : V10FixedParams {
+  unsigned long long* slots;   // look-back words [n_lb][n_tiles][64]
+  unsigned* hdr;               // WsHeader
+  uint32_t hd_magic;           // division by hd (div_magic)
+  int hd_shift;
+  int n_lbd, n_lb, n_lb_pad, n_tiles;
+  int clamp_at;                // tile that holds the first clamp boundary
+  unsigned poll_limit;
+};
+
 // Backward of the full path (osm_v10_bwd): dL/dx of every chunk, one
 // workgroup per (batch row, chunk, 64-lane lane-block).  Needs no workspace.
 struct V10BwdParams {
@@ -270,6 +291,8 @@ hipError_t launch_v10(const V10Params& p, int x_dtype, bool use_lut, int kpad, h
 int v10_bwd_lanes();   // lanes per lane-block of launch_v10_bwd
 hipError_t launch_v10_bwd(const V10BwdParams& p, int x_dtype, int lpt, int kpad, hipStream_t stream);
 hipError_t launch_v10_fixed(const V10FixedParams& p, int x_dtype, bool use_lut, int kpad, hipStream_t stream);
+hipError_t launch_lut_scan(const LutScanParams& p, int x_dtype, bool use_lut, FwdShape s, int kpad,
+                           hipStream_t stream);
 hipError_t launch_fill_zero(void* ptr, size_t bytes, hipStream_t stream);
 hipError_t launch_copy_state(const float* src, float* dst, size_t n, hipStream_t stream);
 hipError_t launch_ws_status(void* ws, unsigned* dst, int reset, hipStream_t stream);

@@ -24,18 +24,12 @@
 #include <type_traits>
 
 #include "osm_tile.h"
+#include "osm_v10_math.h"
 
 namespace osm {
 namespace {
 
 constexpr int kBlockTok = kV10Groups * kV10Run;      // 256 tokens per block
-constexpr float kLog2e = 1.4426950408889634f;
-// Floats per LUT row in LDS: the 8 values of T_k padded to 12, so that the
-// 16-byte reads of random rows by the lanes of a wave spread over more LDS
-// banks than with 8 (rows i and i' collide when 12 (i - i') = 0 mod the
-// bank count).  Measured at the configs[1] shape on MI355X: 221 against
-// 227 us with the XCD order below.
-constexpr int kLutStride = 12;
 // Workgroup order: the workgroups whose lanes share 128-byte lines of x go
 // to one XCD, so each line is fetched into one L2 (with consecutive indices
 // the 4 workgroups of a line sat on 4 XCDs and every line was fetched 4
@@ -67,14 +61,6 @@ __device__ __forceinline__ float load_x<float>(Rsrc r, uint32_t vo, uint32_t so)
 template <>
 __device__ __forceinline__ float load_x<__bf16>(Rsrc r, uint32_t vo, uint32_t so) {
   return __uint_as_float((unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, vo, so, 0) << 16);
-}
-
-// The megakernel's softsign on a bf16 value: |u| and sign(u); NaN reads as 0.
-__device__ __forceinline__ void v10_softsign(float xb, float& absu, float& sgn) {
-  const float xs = xb == xb ? xb : 0.0f;
-  const float ax = __builtin_fmaxf(__builtin_fabsf(xs), 1e-7f);
-  absu = 1.0f - __builtin_amdgcn_rcpf(1.0f + ax);
-  sgn = xs >= 0.0f ? 1.0f : -1.0f;
 }
 
 // The KP proxy-gradient sums of a wave's runs, reduce-scattered: the sum of

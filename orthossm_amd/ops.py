@@ -148,6 +148,12 @@ def _workspace(device: torch.device, stream: int, nbytes: int, op: int) -> torch
         return ws
 
 
+def _has_workspace(device: torch.device, stream: int, nbytes: int, op: int) -> bool:
+    with _ws_lock:
+        ws = _ws_cache.get((device.index, stream, op))
+        return ws is not None and ws.numel() >= nbytes
+
+
 def _as_param(v, H: int, device, name: str) -> torch.Tensor:
     if (isinstance(v, torch.Tensor) and v.dtype is torch.float32 and v.dim() == 1 and v.is_contiguous()
             and v.device == device):
@@ -663,7 +669,17 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     if tanh_y is not None:
         a.tanh_y, a.ty_stride_b, a.ty_stride_s = tanh_y.data_ptr(), tanh_y.stride(0), tanh_y.stride(1)
     a.ema_final, a.final_stride_b = ema_final.data_ptr(), ema_final.stride(0)
-    nat.check(lib.osm_cheby_ema_lut_fwd(ctypes.byref(a), ctypes.c_void_p(_current_stream(dev))))
+    stream = _current_stream(dev)
+    nbytes = lib.osm_lut_fwd_workspace_bytes(ctypes.byref(a))
+    if nbytes and not _has_workspace(dev, stream, nbytes, nat.OP_LUT) and torch.cuda.is_current_stream_capturing():
+        nbytes = 0   # no allocation inside a capture: the walk needs none
+    if nbytes:
+        ws = _workspace(dev, stream, nbytes, nat.OP_LUT)
+        nat.check(lib.osm_cheby_ema_lut_fwd_ws(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
+                                               ctypes.c_void_p(stream)))
+        _after_launch(ws, stream, "osm_cheby_ema_lut_fwd_ws")
+    else:
+        nat.check(lib.osm_cheby_ema_lut_fwd(ctypes.byref(a), ctypes.c_void_p(stream)))
     keep = (x, c, lut, init)  # noqa: F841  (alive until the launch is queued)
     return out, x_norm, tanh_y, ema_final
 

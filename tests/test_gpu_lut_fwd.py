@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from oracle import v10_full as V
+from orthossm_amd import _native as nat
 from orthossm_amd import apply_cheby_rkv_v10
 from orthossm_amd.ops import cheby_ema_lut_forward
 from orthossm_amd.sdpc_kernel import LUT_TABLE_SIZE, _fused_clenshaw_ema_kernel, get_chebyshev_lut
@@ -79,6 +80,78 @@ def test_carry_clamp_binds_at_tile_boundaries(dev, block_s):
     assert np.abs(wout - free).max() > 1e-2          # the case exercises the clamp
     assert rel(out, wout) <= 1e-5
     assert rel(fin, wfin) <= 1e-5
+
+
+class _WalkOnly:
+    """The library with the scan's size query answering 0: the walk serves every call."""
+
+    def __init__(self, lib):
+        self.lib = lib
+
+    def __getattr__(self, name):
+        return (lambda *a: 0) if name == "osm_lut_fwd_workspace_bytes" else getattr(self.lib, name)
+
+
+@pytest.mark.parametrize("B,S,H,hd,K,use_lut,block_s,mu,layout", [
+    (1, 257, 1, 1, 1, True, 16, 0.9, ""),             # one lane, the first clamp after one run
+    (2, 600, 3, 50, 8, True, 48, 0.25, ""),           # 64-token tiles, the smallest decay; run decays near underflow
+    (2, 600, 3, 33, 4, False, 64, 0.9, ""),           # one lane per thread; a clamp at the end of the first tile
+    (1, 1300, 2, 32, 8, True, 1024, 0.9999, ""),      # the clamp in tile 15, past a checkpoint group
+    (1, 700, 2, 32, 6, False, 2048, 0.99, ""),        # no clamp inside the sequence
+    (9, 4100, 2, 64, 8, True, 128, 1.0, ""),          # 128-token tiles; a decay of one
+    (3, 500, 2, 40, 8, True, 144, 0.95, "strided"),   # x and out views of wider rows
+])
+def test_scan_and_walk_agree_around_the_first_clamp(dev, monkeypatch, B, S, H, hd, K, use_lut, block_s, mu, layout):
+    """The scan against the float64 restatement and against the walk, with
+    initial states inside, far outside and infinitely outside [-1, 1], and
+    NaN (-1 from the clamp, in both).  1e-5 as for every output here."""
+    x, c, init = case(B, S, H, hd, K, seed=S + block_s, init_scale=0.5)
+    D = H * hd
+    odd = torch.tensor([3.0, float("inf"), -1e30, -float("inf"), -40.0])
+    for i, v in enumerate(odd):
+        init[i % B, (7 * i) % D] = v
+    xd, out = x.to(dev), None
+    if layout == "strided":
+        wide = torch.zeros(B, S, D + 2, device=dev)
+        wide[..., 2:] = xd
+        xd, out = wide[..., 2:], torch.empty(B, S, D + 6, device=dev)[..., 4:4 + D]
+
+    def call(init_):
+        return cheby_ema_lut_forward(xd, c.to(dev), n_heads=H, ema_momentum=mu, ema_init=init_.to(dev),
+                                     use_lut=use_lut, clamp_tile=block_s, out=out)
+
+    nan_init = init.clone()
+    nan_init[0, D // 2] = float("nan")
+    got = call(init)
+    wxn, wty, wout, wfin = V.fused_clenshaw_ema(x.numpy(), c.double().numpy(), n_heads=H, ema_momentum=f32(mu),
+                                                ema_init=init.numpy(), use_lut=use_lut, block_s=block_s)
+    for g, w in zip(got, (wout, wxn, wty, np.clip(wfin, -1, 1))):
+        assert rel(g, w) <= 1e-5
+    scan = [t.clone() for t in call(nan_init)]
+    real = nat.load()
+    monkeypatch.setattr(nat, "load", lambda: _WalkOnly(real))
+    walk = call(nan_init)
+    torch.cuda.synchronize()
+    for s, w in zip(scan, walk):
+        assert torch.isfinite(s).all() and rel(s, w.double().cpu().numpy()) <= 1e-5
+
+
+def test_capture_without_a_workspace(dev):
+    # a capture on a stream that has made no call yet: nothing is allocated
+    x, c, init = (t.to(dev) for t in case(2, 700, 2, 32, 8, seed=3, init_scale=0.5))
+    want = cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        got = cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
+    for _ in range(3):
+        for t in got:
+            t.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, w in zip(got, want):
+            assert rel(g, w.double().cpu().numpy()) <= 1e-6
+        cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
 
 
 def test_special_values_empty_and_optional_outputs(dev):

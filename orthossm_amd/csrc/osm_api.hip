@@ -40,7 +40,7 @@ int ok() {
 }
 
 struct Geometry {
-  int n_lbd = 0, n_lb = 0, n_lb_pad = 0, n_tiles = 0;
+  int n_lbd = 0, n_lb = 0, n_tiles = 0;
   int tile = 0;        // tokens per tile
   int lanes = 64;      // lanes per lane-block
   int lpt = 2;         // lanes per thread (forward)
@@ -128,12 +128,10 @@ int check_args(const osm_cheby_args* a, Geometry* geo, int op, bool shapes_only 
   const int64_t n_lbd = (D + shape.lanes - 1) / shape.lanes;
   const int64_t n_lb = a->B * n_lbd;
   const int64_t n_tiles = (a->S + tile - 1) / tile;
-  const int64_t n_lb_pad = (n_lb + 7) / 8 * 8;
-  if (n_lb_pad * n_tiles >= (int64_t(1) << 31) || a->S >= (int64_t(1) << 31) - tile)
+  if (n_lb * n_tiles >= (int64_t(1) << 31) || a->S >= (int64_t(1) << 31) - tile)
     return fail(OSM_E_SHAPE, "problem too large: %lld tiles", (long long)(n_lb * n_tiles));
   geo->n_lbd = (int)n_lbd;
   geo->n_lb = (int)n_lb;
-  geo->n_lb_pad = (int)n_lb_pad;
   geo->n_tiles = (int)n_tiles;
   geo->tile = (int)tile;
   geo->lanes = shape.lanes;
@@ -172,7 +170,6 @@ osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* w
   p.D = (int)(a->H * a->hd);
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
-  p.n_lb_pad = geo.n_lb_pad;
   p.n_tiles = geo.n_tiles;
   p.lam_shift = a->lam_shift;
   p.lam_min = a->lam_min;
@@ -412,11 +409,9 @@ Geometry lut_scan_shape(const osm_lut_fwd_args* a) {
   constexpr int64_t kCus = 256;
   const int tile = n_lb * tiles(osm::LutTile::TILE) >= kCus ? osm::LutTile::TILE : osm::LutTileSmall::TILE;
   const int64_t n_tiles = tiles(tile);
-  const int64_t n_lb_pad = (n_lb + 7) / 8 * 8;
-  if (n_lb_pad * n_tiles >= (int64_t(1) << 31)) return geo;
+  if (n_lb * n_tiles >= (int64_t(1) << 31)) return geo;
   geo.n_lbd = (int)n_lbd;
   geo.n_lb = (int)n_lb;
-  geo.n_lb_pad = (int)n_lb_pad;
   geo.n_tiles = (int)n_tiles;
   geo.tile = tile;
   geo.lpt = two ? 2 : 1;
@@ -778,7 +773,6 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   osm::div_magic((uint32_t)a->hd, &p.hd_magic, &p.hd_shift);
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
-  p.n_lb_pad = geo.n_lb_pad;
   p.n_tiles = geo.n_tiles;
   p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
   p.poll_limit = osm::kSpinLimit;

@@ -174,11 +174,7 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
   ThreadPos qc = q;
   qc.tg = G::NTG - 1 - q.tg;   // chain order: the tile's last run first
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lb_pad, p.n_lbd, p.n_tiles);   // tile = chain index
-  if (ti.pad) {
-    finish_block(p.hdr, tags.epoch);
-    return;
-  }
+  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);   // tile = chain index
   TileInfo tm = ti;
   tm.tile = p.n_tiles - 1 - ti.tile;   // tile in sequence order
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, tm);
@@ -393,7 +389,7 @@ __global__ void __launch_bounds__(kRedSlices * kLanes) bwd_reduce(const float* p
 template <class G, bool DYN, bool ZS, typename XT, typename OT, int KP>
 hipError_t launch_all(const BwdParams& bp, hipStream_t stream) {
   const FwdParams& p = bp.f;
-  const unsigned grid = (unsigned)p.n_lb_pad * (unsigned)p.n_tiles;
+  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   hipLaunchKernelGGL((cheby_ema_bwd_kernel<G, DYN, ZS, XT, OT, KP>), dim3(grid), dim3(G::THREADS), 0, stream, bp);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !bp.grad_coeffs) return e;

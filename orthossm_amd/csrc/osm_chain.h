@@ -17,16 +17,17 @@
 // sb*WPS .. sb*WPS+WPS-1, each reading WPT predecessor tiles, so that
 // CKPT = WPS * WPT.  Look-back words are laid out [lane-block][tile][lane].
 //
-// Tile order.  Virtual tile v covers tile v / n_lb_pad of the lane-block in
-// slot v % n_lb_pad, with n_lb_pad = n_lb rounded up to a multiple of 8
-// (tile_info maps slots to lane-blocks so that consecutive lane-blocks share
-// a class; virtual tiles with lane-block >= n_lb are padding and are
-// skipped).  A tile waits only on earlier tiles of its lane-block:
-// v - k*n_lb_pad, the same slot and class v % 8.  Block b handles v = b.  Awaited blocks have a lower index at a
-// stride that is a multiple of 8; workgroups go to the 8 XCDs round-robin by
-// index and in index order within an XCD, so each awaited block sits on the
-// same XCD and was dispatched before the waiter.  The waits are bounded
-// (kSpinLimit), so a broken assumption surfaces as a fault flag, not a hang.
+// Tile order.  Block v handles tile v / n_lb of the lane-block in slot v % n_lb
+// (tile_info maps slots to lane-blocks), so a tile waits only on blocks of
+// lower index.  Workgroups go to the 8 XCDs round-robin by index and in index
+// order within an XCD: the unfinished block of lowest index is always
+// resident or next in line on an XCD whose earlier blocks have all ended, and
+// what it waits on has ended, so the chain moves on whatever XCDs a lane-block's
+// tiles are on (the look-back words are agent-scope atomics, coherent over the
+// XCDs).  With n_lb a multiple of 8 every tile of a lane-block is on one XCD;
+// otherwise they rotate over all eight: pinning them left XCDs idle (4 of 8
+// at n_lb = 4).  The waits are bounded (kSpinLimit), so a broken
+// assumption surfaces as a fault flag, not a hang.
 #pragma once
 
 #include "osm_device.h"
@@ -46,7 +47,6 @@ struct ChainLds {
 struct TileInfo {
   int v, tile, lb, b, lbd;
   bool is_last, is_ckpt;
-  bool pad;  // padding tile: no lane-block
 };
 
 struct Tags {
@@ -93,18 +93,16 @@ __device__ __forceinline__ Tags launch_tags(unsigned* hdr_words) {
 }
 
 template <class G>
-__device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lb_pad, int n_lbd, int n_tiles) {
+__device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lbd, int n_tiles) {
   TileInfo ti;
   ti.v = v;
-  ti.tile = v / n_lb_pad;
-  // Slot s = v mod n_lb_pad (XCD class s mod 8) serves lane-block
-  // (s mod 8) * m + s / 8, m = n_lb_pad / 8: the m consecutive lane-blocks
-  // c m .. c m + m - 1 all belong to class c, so the lane-blocks of a batch
-  // row share one XCD and its L2 (they read the same lines of g, one value
-  // per head per token), and every class still holds m lane-blocks.
-  const int s = v - ti.tile * n_lb_pad;
-  ti.lb = (s & 7) * (n_lb_pad >> 3) + (s >> 3);
-  ti.pad = ti.lb >= n_lb;
+  ti.tile = v / n_lb;
+  // Slot s = v mod n_lb; the slots of one residue c = s mod 8 are on one XCD
+  // and serve consecutive lane-blocks, so the lane-blocks of a batch row share
+  // an L2 (they read the same lines of g, one value per head per token).
+  // With n_lb = 8 q + r, residues below r hold q + 1 lane-blocks.
+  const int s = v - ti.tile * n_lb, c = s & 7;
+  ti.lb = c * (n_lb >> 3) + min(c, n_lb & 7) + (s >> 3);
   ti.b = ti.lb / n_lbd;
   ti.lbd = ti.lb - ti.b * n_lbd;
   ti.is_last = ti.tile == n_tiles - 1;

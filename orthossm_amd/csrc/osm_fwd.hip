@@ -130,11 +130,7 @@ cheby_ema_fwd_kernel(const FwdParams p) {
   __builtin_amdgcn_s_setprio(3);
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lb_pad, p.n_lbd, p.n_tiles);
-  if (ti.pad) {
-    finish_block(p.hdr, tags.epoch);
-    return;
-  }
+  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
 
   // Monomial coefficients (loads first, converted after the x loads).
@@ -326,7 +322,7 @@ cheby_ema_fwd_kernel(const FwdParams p) {
 
 template <class G, bool DYN, typename XT, typename OT>
 hipError_t launch_g(const FwdParams& p, int kpad, hipStream_t stream) {
-  const unsigned grid = (unsigned)p.n_lb_pad * (unsigned)p.n_tiles;
+  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   if (kpad == 4)
     hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 4>), dim3(grid), dim3(G::THREADS), 0, stream, p);
   else if (kpad == 8)
@@ -341,7 +337,7 @@ hipError_t launch_g(const FwdParams& p, int kpad, hipStream_t stream) {
 template <bool DYN, typename XT, typename OT>
 hipError_t launch_generic(const FwdParams& p, int kpad, hipStream_t stream) {
   using G = FwdTileGeneric;
-  const unsigned grid = (unsigned)p.n_lb_pad * (unsigned)p.n_tiles;
+  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   if (kpad <= 8)
     hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 8>), dim3(grid), dim3(G::THREADS), 0, stream, p);
   else if (kpad == 16)

@@ -151,8 +151,7 @@ struct FwdParams {
   uint32_t hd_magic;           // n / hd = (umulhi(n, hd_magic) + n) >> hd_shift for 0 <= n < 2^31
   int hd_shift;
   int n_lbd;                   // lane-blocks per batch row = ceil(D / LANES)
-  int n_lb;                    // B * n_lbd
-  int n_lb_pad;                // n_lb rounded up to a multiple of 8; grid = n_lb_pad * n_tiles
+  int n_lb;                    // B * n_lbd; grid = n_lb * n_tiles
   int n_tiles;                 // ceil(S / TILE)
   float lam_shift, lam_min, lam_max;
   int clamp_out;
@@ -240,7 +239,7 @@ struct LutScanParams : V10FixedParams {
   unsigned* hdr;               // WsHeader
   uint32_t hd_magic;           // division by hd (div_magic)
   int hd_shift;
-  int n_lbd, n_lb, n_lb_pad, n_tiles;
+  int n_lbd, n_lb, n_tiles;
   int clamp_at;                // tile that holds the first clamp boundary
   unsigned poll_limit;
 };

@@ -39,11 +39,7 @@ lut_fwd_kernel(const LutScanParams p) {
 
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lb_pad, p.n_lbd, p.n_tiles);
-  if (ti.pad) {
-    finish_block(p.hdr, tags.epoch);
-    return;
-  }
+  TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
   const int t_tile = ti.tile * G::TILE;
   const int d0 = ti.lbd * kLanes + q.lt * LPT;
   const bool lane_ok = d0 < p.D;
@@ -234,7 +230,7 @@ lut_fwd_kernel(const LutScanParams p) {
 
 template <class G, typename XT, bool LUT>
 hipError_t launch_g(const LutScanParams& p, int kpad, hipStream_t stream) {
-  const dim3 grid((unsigned)p.n_lb_pad * (unsigned)p.n_tiles), block(G::THREADS);
+  const dim3 grid((unsigned)p.n_lb * (unsigned)p.n_tiles), block(G::THREADS);
   if (kpad == 4)
     hipLaunchKernelGGL((lut_fwd_kernel<G, XT, 4, LUT>), grid, block, 0, stream, p);
   else

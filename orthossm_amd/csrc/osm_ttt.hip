@@ -268,11 +268,7 @@ cheby_ema_ttt_kernel(const FwdParams p) {
 
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lb_pad, p.n_lbd, p.n_tiles);
-  if (ti.pad) {
-    finish_block(p.hdr, tags.epoch);
-    return;
-  }
+  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
   // This wave's monomial coefficient (wave w holds coefficient w of the 64
   // lanes), formed once per launch by ttt_mono_prep; loaded before x.
@@ -645,7 +641,7 @@ hipError_t launch_all(const FwdParams& p0, float* grad, hipStream_t stream) {
   hipLaunchKernelGGL((ttt_mono_prep<KP>), dim3(p.n_lb), dim3(64 * KP), 0, stream, p, p.mono_tab, form);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  const unsigned grid = (unsigned)p.n_lb_pad * (unsigned)p.n_tiles;
+  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   hipLaunchKernelGGL((cheby_ema_ttt_kernel<G, DYN, SOFT, XT, OT, KP>), dim3(grid), dim3(G::THREADS), 0, stream, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;

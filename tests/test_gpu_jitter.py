@@ -10,7 +10,8 @@ such race."""
 import pytest
 import torch
 
-from helpers import inputs, to_dev
+from helpers import (assert_close_fp32, assert_close_grad, inputs, oracle_backward, oracle_forward, oracle_ttt,
+                     to_dev)
 from orthossm_amd import cheby_ema_backward, cheby_ema_forward, cheby_ema_ttt
 from orthossm_amd import ops
 
@@ -86,3 +87,35 @@ def test_backward_bits_unchanged(dev):
     go = torch.randn(out.shape, device=dev, generator=torch.Generator(device=dev).manual_seed(73))
     a, b = twice(lambda: cheby_ema_backward(d["x"], d["coeffs"], d["damping"], d["lam"], out, go, need_init=True))
     assert_same(a, b)
+
+
+@pytest.mark.parametrize("B,S,H,hd,dyn", [
+    (1, 9000, 1, 64, False),     # one lane-block: its tiles rotate over all eight XCDs
+    (3, 5000, 1, 48, True),      # three, of 48 lanes
+    (3, 4000, 3, 64, False),     # nine: one more than the XCDs
+])
+def test_chains_across_xcds(dev, B, S, H, hd, dyn):
+    """Lane-block counts off the multiples of 8, whose tiles wait on words
+    published on other XCDs: the oracle's values, and the same bits under
+    jitter, in the forward, the TTT and the backward."""
+    inp = inputs(B, S, H, hd, 8, seed=S, dynamic=dyn)
+    d = to_dev(inp, dev)
+    go = torch.randn(B, S, H * hd, generator=torch.Generator().manual_seed(S)).to(dev)
+    args = (d["x"], d["coeffs"], d["damping"], d["lam"])
+
+    def step():
+        out, fin = cheby_ema_forward(*args, g=d.get("g"), return_state=True)
+        t_out, t_grad = cheby_ema_ttt(*args, g=d.get("g"))
+        gx, gc, _ = cheby_ema_backward(*args, out, go, g=d.get("g"))
+        return out, fin, t_out, t_grad, gx, gc
+
+    a, b = twice(step)
+    assert_same(a, b)
+    want, _ = oracle_forward(inp)
+    assert_close_fp32(a[0].cpu(), want)
+    assert_close_fp32(a[2].cpu(), want)
+    G, _, _ = oracle_ttt(inp)
+    assert_close_grad(a[3].cpu(), G, what="ttt gradient")
+    wx, wc, _ = oracle_backward(inp, go.cpu().numpy(), out_saved=a[0].cpu().numpy())
+    assert_close_grad(a[4].cpu(), wx, what="grad_x")
+    assert_close_grad(a[5].cpu(), wc, what="grad_coeffs")

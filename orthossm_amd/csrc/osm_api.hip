@@ -39,6 +39,18 @@ int ok() {
   return OSM_OK;
 }
 
+// log2 of the look-back words per thread for the geometries that hold
+// kFwdWords: 4 words (a checkpoint every 32 tiles) where few lane-blocks have
+// many tiles, so that the serial chain of checkpoints (~0.7 us each) is what
+// the launch waits for, else 1 (every 8 tiles), whose threads poll less.
+// Measured on MI355X, K=8, 1 word against 4: B=1 S=16384 D=256 16.8 and 11.0
+// us, S=65536 D=128 30.0 and 17.3, S=4096 D=256 8.5 and 7.4, S=16384 D=512 15.6
+// and 15.3 (8 lane-blocks); B=3 S=4000 D=384 (18) 11.2 and 11.4, dynamic
+// lambda B=3 S=6000 D=320 (15) 13.6 and 14.8.
+int look_back_shift(int64_t n_lb, int64_t n_tiles) {
+  return n_lb <= 8 && n_tiles >= 32 ? 2 : 0;
+}
+
 struct Geometry {
   int n_lbd = 0, n_lb = 0, n_tiles = 0;
   int tile = 0;        // tokens per tile
@@ -171,6 +183,7 @@ osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* w
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
+  p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.lam_shift = a->lam_shift;
   p.lam_min = a->lam_min;
   p.lam_max = a->lam_max;
@@ -774,6 +787,7 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
+  p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
   p.poll_limit = osm::kSpinLimit;
   const hipError_t e = osm::launch_lut_scan(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0,

@@ -15,7 +15,8 @@
 // A lane-block is G::LANES consecutive lanes of one batch row (64 or 128);
 // the look-back works on 64-lane sub-blocks: sub-block sb is served by waves
 // sb*WPS .. sb*WPS+WPS-1, each reading WPT predecessor tiles, so that
-// CKPT = WPS * WPT.  Look-back words are laid out [lane-block][tile][lane].
+// CKPT = WPS * WPT (or, where a launch chooses, fewer words: WPS << wsh).
+// Look-back words are laid out [lane-block][tile][lane].
 //
 // Tile order.  Block v handles tile v / n_lb of the lane-block in slot v % n_lb
 // (tile_info maps slots to lane-blocks), so a tile waits only on blocks of
@@ -92,8 +93,14 @@ __device__ __forceinline__ Tags launch_tags(unsigned* hdr_words) {
   return t;
 }
 
+// log2 of the look-back words per thread when a kernel always uses G::WPT.
 template <class G>
-__device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lbd, int n_tiles) {
+constexpr int kWordsShift = G::WPT == 1 ? 0 : (G::WPT == 2 ? 1 : (G::WPT == 4 ? 2 : 3));
+
+// wsh: log2 of the look-back words per thread of this launch (at most
+// G::WPT words); checkpoints lie every WPS << wsh tiles.
+template <class G>
+__device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lbd, int n_tiles, int wsh = kWordsShift<G>) {
   TileInfo ti;
   ti.v = v;
   ti.tile = v / n_lb;
@@ -106,7 +113,7 @@ __device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lbd, int n_
   ti.b = ti.lb / n_lbd;
   ti.lbd = ti.lb - ti.b * n_lbd;
   ti.is_last = ti.tile == n_tiles - 1;
-  ti.is_ckpt = (ti.tile % G::CKPT) == G::CKPT - 1;
+  ti.is_ckpt = ((ti.tile + 1) & ((G::WPS << wsh) - 1)) == 0;
   return ti;
 }
 
@@ -207,12 +214,14 @@ struct LookBack {
 
 template <class G, bool DYN>
 __device__ __forceinline__ void look_back_issue(LookBack<G, DYN>& st, const ThreadPos& q, const TileInfo& ti,
-                                                const LaneSlots& ls, int g0_min = 0) {
+                                                const LaneSlots& ls, int wsh = kWordsShift<G>, int g0_min = 0) {
+  static_assert((G::WPS & (G::WPS - 1)) == 0 && (1 << kWordsShift<G>) == G::WPT, "checkpoint groups are powers of two");
   const int ll = look_lane<G>(q);
   // g0_min: first tile of the group when an extra checkpoint precedes it
-  st.g0 = max((ti.tile / G::CKPT) * G::CKPT, g0_min);
-  st.beg = st.g0 + (q.wave % G::WPS) * G::WPT;
-  st.end = min(st.beg + G::WPT, ti.tile);
+  st.g0 = max(ti.tile & ~((G::WPS << wsh) - 1), g0_min);
+  // (wave-uniform, so the tests on it below are scalar)
+  st.beg = st.g0 + ((__builtin_amdgcn_readfirstlane(q.wave) % G::WPS) << wsh);
+  st.end = min(st.beg + (1 << wsh), ti.tile);
 #pragma unroll
   for (int i = 0; i < G::WPT; ++i) {
     if (st.beg + i < st.end) {

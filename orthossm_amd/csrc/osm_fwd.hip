@@ -130,7 +130,9 @@ cheby_ema_fwd_kernel(const FwdParams p) {
   __builtin_amdgcn_s_setprio(3);
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
+  constexpr bool kVarWords = G::WPT == kFwdWords;   // look-back words per thread chosen per launch
+  const int wsh = kVarWords ? p.wsh : kWordsShift<G>;
+  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles, wsh);
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
 
   // Monomial coefficients (loads first, converted after the x loads).
@@ -289,7 +291,7 @@ cheby_ema_fwd_kernel(const FwdParams p) {
     const int dlk = ti.lbd * G::LANES + look_lane<G>(q);
     const float a_look = DYN ? 0.0f : static_tile_A<G>(p.lam[dlk < p.D ? div_hd(dlk, p) : 0]);
     LookBack<G, DYN> lbk;
-    look_back_issue<G, DYN>(lbk, q, ti, ls);
+    look_back_issue<G, DYN>(lbk, q, ti, ls, wsh);
     jitter(p.jitter, tags.epoch, 1);
     look_back_finish<G, DYN>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
   }

@@ -22,7 +22,7 @@ constexpr int kMonoMaxK = 8;
 // reads or writes TGW rows x LANES*4 contiguous bytes (fp32).  Token groups
 // (runs) are ordered wave-major: tg = wave * TGW + lane_in_wave / TPR.  The
 // look-back serves each 64-lane sub-block with WPS waves of WPT words per
-// thread, so tiles are grouped in checkpoint runs of CKPT = WPS * WPT.
+// thread, so tiles are grouped in checkpoint runs of WPS * WPT (see osm_chain.h).
 template <int LPT_, int WAVES_, int R_, int LANES_ = 64, int WPT_ = 8>
 struct TileGeo {
   static constexpr int LPT = LPT_;            // lanes per thread
@@ -37,7 +37,6 @@ struct TileGeo {
   static constexpr int TILE = NTG * R;        // tokens per tile
   static constexpr int WPS = WAVES / NSUB;    // look-back waves per sub-block
   static constexpr int WPT = WPT_;            // look-back words per thread
-  static constexpr int CKPT = WPS * WPT;      // checkpoint interval, tiles
   static_assert(LANES % 64 == 0 && LANES % LPT == 0 && TPR <= 64 && 64 % TPR == 0, "geometry");
   static_assert(WAVES % NSUB == 0, "look-back waves");
 };
@@ -49,23 +48,25 @@ struct TileGeo {
 // tile.  Measured on MI355X at BASELINE configs[1] against 128-lane tiles
 // with 2 or 4 lanes per thread (256 and 128 tokens) and 64-lane tiles with 4
 // lanes per thread: the 64-lane, 2-lane, 512-token tile is fastest.
-// The medium and small tiles (dynamic lambda, and short sequences) read one
-// look-back word per thread (checkpoints every 8 tiles): every thread runs
-// the polling code of each of its words, and at configs[3] one word gives
-// 420 us against 429 with two and 449 with eight.  The large tile keeps
-// eight (no difference at configs[1]).
+// The medium, small and one-lane tiles read one or kFwdWords look-back words
+// per thread, chosen per launch (look_back_shift in osm_api.hip): every thread
+// runs the polling code of each of its words, and on a chip full of tiles one
+// is best (dynamic lambda, B=8 S=32768 D=1024: 420 us against 429 with two and
+// 449 with eight).  The large tile keeps eight (no difference at B=4 S=16384
+// D=512).
+constexpr int kFwdWords = 4;
 using FwdTileLarge = TileGeo<2, 8, 32>;           // 512 tokens x 64 lanes
 // Dynamic lambda at 512 tokens: the per-token lambda lives in LDS (formed
 // once per token and head), which leaves the registers for the run; one
 // look-back word per thread (two per word pair: A and B).
 using FwdTileLargeDyn = TileGeo<2, 8, 32, 64, 1>;
-using FwdTileMedium = TileGeo<2, 8, 16, 64, 1>;   // 256 tokens x 64 lanes
-using FwdTileSmall = TileGeo<2, 8, 8, 64, 1>;     // 128 tokens x 64 lanes
+using FwdTileMedium = TileGeo<2, 8, 16, 64, kFwdWords>;   // 256 tokens x 64 lanes
+using FwdTileSmall = TileGeo<2, 8, 8, 64, kFwdWords>;     // 128 tokens x 64 lanes
 // One lane per thread: any head size, rows aligned to one element, and the
 // Chebyshev form of longer series (more than kMonoMaxK coefficients), whose
 // coefficients take twice the registers.  Used only where the geometries
 // above do not apply.
-using FwdTileGeneric = TileGeo<1, 8, 16, 64, 1>;  // 128 tokens x 64 lanes
+using FwdTileGeneric = TileGeo<1, 8, 16, 64, kFwdWords>;  // 128 tokens x 64 lanes
 constexpr int kMaxTileRows = 512;              // bound on TILE (+1 row read past a tile)
 
 // Geometry of a forward launch.
@@ -157,6 +158,7 @@ struct FwdParams {
   int clamp_out;
   int nan_zero_u;              // NaN x counts as u = 0 (else z = 0)
   int jitter;                  // OSM_FLAG_TIMING_JITTER: pseudo-random delays (test aid)
+  int wsh;                     // log2 of the look-back words per thread (kFwdWords geometries)
   unsigned poll_limit;         // look-back polls before a wait gives up: kSpinLimit, or 0 under
                                // OSM_FLAG_POLL_LIMIT_ZERO (test aid)
   float ttt_scale;             // 2 / (B*(S-1)*D)
@@ -230,16 +232,17 @@ struct V10FixedParams : V10Params {
 // S=512 (128 tiles of 128 tokens), 12.2 against 11.9 at B=2 S=2000 D=400
 // (224), 21.0 against 16.0 at B=2 S=4096 (512).  One lane per thread where
 // rows are off two-element boundaries.
-using LutTile = TileGeo<2, 8, 8, 64, 1>;              // 128 tokens x 64 lanes
-using LutTileSmall = TileGeo<2, 8, 4, 64, 1>;         // 64 tokens
-using LutTileGeneric = TileGeo<1, 8, 16, 64, 1>;      // 128 tokens
-using LutTileGenericSmall = TileGeo<1, 8, 8, 64, 1>;  // 64 tokens
+using LutTile = TileGeo<2, 8, 8, 64, kFwdWords>;              // 128 tokens x 64 lanes
+using LutTileSmall = TileGeo<2, 8, 4, 64, kFwdWords>;         // 64 tokens
+using LutTileGeneric = TileGeo<1, 8, 16, 64, kFwdWords>;      // 128 tokens
+using LutTileGenericSmall = TileGeo<1, 8, 8, 64, kFwdWords>;  // 64 tokens
 struct LutScanParams : V10FixedParams {
   unsigned long long* slots;   // look-back words [n_lb][n_tiles][64]
   unsigned* hdr;               // WsHeader
   uint32_t hd_magic;           // division by hd (div_magic)
   int hd_shift;
   int n_lbd, n_lb, n_tiles;
+  int wsh;                     // log2 of the look-back words per thread
   int clamp_at;                // tile that holds the first clamp boundary
   unsigned poll_limit;
 };

@@ -39,7 +39,7 @@ lut_fwd_kernel(const LutScanParams p) {
 
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
+  TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles, p.wsh);
   const int t_tile = ti.tile * G::TILE;
   const int d0 = ti.lbd * kLanes + q.lt * LPT;
   const bool lane_ok = d0 < p.D;
@@ -169,7 +169,7 @@ lut_fwd_kernel(const LutScanParams p) {
         p.ema_init && q.wave == 0 && dc < p.D ? p.ema_init[(int64_t)ti.b * p.init_sb + dc] : 0.0f;
     const float tile_A = __builtin_fmaxf(static_tile_A<G>(mu), kTinyDecay);
     LookBack<G, false> lbk;
-    look_back_issue<G, false>(lbk, q, ti, ls, ti.tile > p.clamp_at ? p.clamp_at + 1 : 0);
+    look_back_issue<G, false>(lbk, q, ti, ls, p.wsh, ti.tile > p.clamp_at ? p.clamp_at + 1 : 0);
     ti.is_ckpt = ckpt && !at_clamp;   // the clamped tile's state is published below
     look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A, p.hdr, p.poll_limit);
   }

@@ -98,13 +98,17 @@ class _WalkOnly:
     (2, 600, 3, 33, 4, False, 64, 0.9, ""),           # one lane per thread; a clamp at the end of the first tile
     (1, 1300, 2, 32, 8, True, 1024, 0.9999, ""),      # the clamp in tile 15, past a checkpoint group
     (1, 700, 2, 32, 6, False, 2048, 0.99, ""),        # no clamp inside the sequence
+    (1, 2500, 2, 32, 8, True, 1008, 0.9995, ""),      # 40 tiles of one lane-block: groups of 32, the clamp inside one
+    (2, 4200, 1, 40, 4, True, 2064, 0.9999, ""),      # the clamp in the first tile of the second group of 32
     (9, 4100, 2, 64, 8, True, 128, 1.0, ""),          # 128-token tiles; a decay of one
     (3, 500, 2, 40, 8, True, 144, 0.95, "strided"),   # x and out views of wider rows
 ])
 def test_scan_and_walk_agree_around_the_first_clamp(dev, monkeypatch, B, S, H, hd, K, use_lut, block_s, mu, layout):
     """The scan against the float64 restatement and against the walk, with
     initial states inside, far outside and infinitely outside [-1, 1], and
-    NaN (-1 from the clamp, in both).  1e-5 as for every output here."""
+    NaN (-1 from the clamp, in both).  1e-5 as for every output here, so the
+    two may differ by 2e-5 (the walk's drift at mu = 0.9999 comes near its
+    1e-5)."""
     x, c, init = case(B, S, H, hd, K, seed=S + block_s, init_scale=0.5)
     D = H * hd
     odd = torch.tensor([3.0, float("inf"), -1e30, -float("inf"), -40.0])
@@ -133,7 +137,8 @@ def test_scan_and_walk_agree_around_the_first_clamp(dev, monkeypatch, B, S, H, h
     walk = call(nan_init)
     torch.cuda.synchronize()
     for s, w in zip(scan, walk):
-        assert torch.isfinite(s).all() and rel(s, w.double().cpu().numpy()) <= 1e-5
+        assert torch.isfinite(s).all()
+        assert rel(s, w.double().cpu().numpy()) <= 2e-5
 
 
 def test_capture_without_a_workspace(dev):

@@ -33,8 +33,7 @@ constexpr int kBlockTok = kV10Groups * kV10Run;      // 256 tokens per block
 // Workgroup order: the workgroups whose lanes share 128-byte lines of x go
 // to one XCD, so each line is fetched into one L2 (with consecutive indices
 // the 4 workgroups of a line sat on 4 XCDs and every line was fetched 4
-// times): 227 against 270 us at the configs[1] shape.
-constexpr bool kXcdLines = true;
+// times): 227 against 270 us at B=4 S=16384 D=512.
 
 // x rounded to bf16 (round to nearest even), as the reference casts on entry.
 template <typename XT>
@@ -67,10 +66,10 @@ __device__ __forceinline__ float load_x<__bf16>(Rsrc r, uint32_t vo, uint32_t so
 // v over the runs of lane l (lanes l, l + LW, l + 2 LW, .. of the wave) is
 // the butterfly v += v[lane ^ o] for o = LW, 2 LW, .. 32, and here each step
 // serves two of the sums at once, so that after the last step lane (run gw,
-// l) holds the full sum of coefficient gw (and, with LW = 16 and KP = 8,
-// of gw + 4), which it stores to ws[k][l].  The steps, with the same sums
-// (each adds a lane's partial sum and its partner's) as the butterfly:
-//   o = 8 (LW = 8): a DPP row rotate by 8 (lane ^ 8 inside each 16-lane row)
+// l) holds the full sum of one coefficient (gw with LW = 8), which it stores
+// to ws[k][l].  The steps, with the same sums (each adds a lane's partial sum
+// and its partner's) as the butterfly (LW = 4 takes o = 4 last):
+//   o = 8: a DPP row rotate by 8 (lane ^ 8 inside each 16-lane row)
 //     of the value the partner keeps (lanes with bit 3 set keep the odd one
 //     of a pair of sums, the others the even one);
 //   o = 16: v_permlane16_swap of a pair (a, b) gives (rows a0, b0, a2, b2)
@@ -107,35 +106,50 @@ __device__ __forceinline__ float pair32(float a, float b) {
 
 template <int LW, int KP>
 __device__ __forceinline__ void store_run_sums(const float (&gc)[KP], float (&ws)[8][LW], int l, int gw) {
-  static_assert(LW == 8 || LW == 16, "8 or 16 lanes per workgroup");
+  static_assert(LW == 4 || LW == 8, "4 or 8 lanes per workgroup");
   static_assert(KP == 4 || KP == 8, "4 or 8 coefficients");
-  constexpr int N1 = LW == 8 ? KP / 2 : KP;   // values left after the o = 8 step
-  float a[N1];
-  if constexpr (LW == 8) {
-    const bool odd = (threadIdx.x & 8) != 0;
+  if constexpr (LW == 4) {
+    // o = 16, o = 32, then o = 8 (lanes with bit 3 set keep the odd sum of the
+    // last pair; with KP = 4 one sum is left and all lanes add it), then o = 4
+    // on the one sum left.
+    float b[KP / 2], a[KP / 4];
 #pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const float keep = odd ? gc[2 * i + 1] : gc[2 * i];
-      const float give = odd ? gc[2 * i] : gc[2 * i + 1];
-      a[i] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xF, 0xF, false));
+    for (int i = 0; i < KP / 2; ++i) b[i] = pair16(gc[2 * i], gc[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < KP / 4; ++i) a[i] = pair32(b[2 * i], b[2 * i + 1]);
+    const int lane = threadIdx.x & 63;
+    const int hi = (lane >> 3) & 1;
+    float keep = a[0], give = a[0];
+    int k = ((lane >> 4) & 1) | (((lane >> 5) & 1) << 1);
+    if constexpr (KP == 8) {
+      keep = hi ? a[1] : a[0];
+      give = hi ? a[0] : a[1];
+      k += 4 * hi;
     }
-  } else {
+    float v = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xF, 0xF, false));
+    v += __shfl_xor(v, 4);
+    if ((lane & 4) == 0 && (KP == 8 || !hi)) ws[k][l] = v;
+    return;
+  }
+  constexpr int N1 = KP / 2;   // values left after the o = 8 step
+  float a[N1];
+  const bool odd = (threadIdx.x & 8) != 0;
 #pragma unroll
-    for (int i = 0; i < N1; ++i) a[i] = gc[i];
+  for (int i = 0; i < N1; ++i) {
+    const float keep = odd ? gc[2 * i + 1] : gc[2 * i];
+    const float give = odd ? gc[2 * i] : gc[2 * i + 1];
+    a[i] = keep + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(give), 0x128, 0xF, 0xF, false));
   }
   constexpr int N2 = N1 / 2;   // after o = 16
   float b[N2];
 #pragma unroll
   for (int i = 0; i < N2; ++i) b[i] = pair16(a[2 * i], a[2 * i + 1]);
   if constexpr (N2 == 1) {
-    // one value (LW = 8, KP = 4): lane (gw, l) holds coefficient gw & 3
+    // KP = 4: one value, lane (gw, l) holds coefficient gw & 3
     const float v = pair32(b[0], b[0]);
     if (gw < 4) ws[gw][l] = v;
   } else {
-    // N2 = 2 (LW = 8, KP = 8: coefficient gw) or N2 = 4 (LW = 16, KP = 8:
-    // coefficients gw and gw + 4) or N2 = 2 (LW = 16, KP = 4: gw)
-#pragma unroll
-    for (int i = 0; i < N2 / 2; ++i) ws[gw + 4 * i][l] = pair32(b[2 * i], b[2 * i + 1]);
+    ws[gw][l] = pair32(b[0], b[1]);   // KP = 8: coefficient gw
   }
 }
 
@@ -151,7 +165,7 @@ struct __attribute__((aligned(16))) V10Lds {
   float ws[NW][8][LW];               // each wave's proxy-gradient sums
 };
 
-// LW lanes per workgroup (8 or 16); kV10Groups runs of kV10Run tokens per
+// LW lanes per workgroup (4 or 8; 8 or 16 for the fixed forward); kV10Groups runs of kV10Run tokens per
 // 256-token block.  A wave holds 64 / LW runs of the same LW lanes: runs are
 // composed inside a wave with shuffles and across waves through LDS, both
 // in a fixed order.
@@ -174,24 +188,15 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
   const int tid = threadIdx.x;
   const int l = tid % LW, g = tid / LW;
   const int wave = tid >> 6, gw = (tid & 63) / LW;   // run inside the wave
-  int lg = blockIdx.x % p.n_lg;
-  int bh = blockIdx.x / p.n_lg;
-  if constexpr (kXcdLines) {
-    // Workgroups go to the 8 XCDs round-robin by index.  The 128 / (4 LW)
-    // consecutive lane groups of a head that share 128-byte lines of x (fp32)
-    // are given indices with the same residue mod 8, so their lines are
-    // fetched into one XCD's L2 once.
-    constexpr int kShare = 128 / (4 * LW);
-    const int grid = gridDim.x;
-    if (p.n_lg % kShare == 0 && grid % (8 * kShare) == 0) {
-      const int v = blockIdx.x, xcd = v & 7, slot = v >> 3;
-      const int line = (slot / kShare) * 8 + xcd;          // line group, global
-      const int q = slot % kShare;
-      const int lines_per_head = p.n_lg / kShare;
-      lg = (line % lines_per_head) * kShare + q;
-      bh = line / lines_per_head;
-    }
-  }
+  // Workgroups go to the 8 XCDs round-robin by index: XCD c takes the
+  // consecutive lane groups c per .. c per + per - 1, so those that share
+  // 128-byte lines of x and out are on one XCD's L2 (all but those at seven
+  // borders).
+  const int per = gridDim.x >> 3;
+  const int item = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
+  if (item >= p.B * p.H * p.n_lg) return;
+  const int lg = item % p.n_lg;
+  const int bh = item / p.n_lg;
   const int h = bh % p.H, b = bh / p.H;
   const int j = lg * LW + l;                 // lane inside the head
   const bool lane_ok = j < p.hd;
@@ -597,7 +602,7 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
     // Reduce the proxy gradient over the runs (a fixed butterfly inside each
     // wave, reduce-scattered over the coefficients, then the waves in
     // order), then Lion.
-    store_run_sums<LW, KP>(gc, L.ws[wave], l, gw);
+    if constexpr (!FIXED) store_run_sums<LW, KP>(gc, L.ws[wave], l, gw);
     // The first wave of each SIMD reaches the barrier early: it prepares its
     // token 0 of the next chunk here, the others while Lion runs.
     const bool early = wave < V10Lds<LW>::NW / 2;
@@ -644,7 +649,7 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
 
 template <typename XT, bool LUT, int LW, bool FIXED, typename P>
 hipError_t launch_w(const P& p, int kpad, hipStream_t stream) {
-  const unsigned grid = (unsigned)(p.B * p.H * p.n_lg);
+  const unsigned grid = ((unsigned)(p.B * p.H * p.n_lg) + 7u) / 8u * 8u;
   if (kpad == 4)
     hipLaunchKernelGGL((v10_chunked_kernel<XT, 4, LUT, LW, FIXED, P>), dim3(grid), dim3(kV10Groups * LW), 0, stream, p);
   else
@@ -655,15 +660,31 @@ hipError_t launch_w(const P& p, int kpad, hipStream_t stream) {
 template <typename XT, bool LUT, bool FIXED, typename P>
 hipError_t launch_x(const P& p, int kpad, hipStream_t stream) {
   if (p.lanes == 8) return launch_w<XT, LUT, 8, FIXED>(p, kpad, stream);
-  if (p.lanes == 16) return launch_w<XT, LUT, 16, FIXED>(p, kpad, stream);
+  constexpr int kOther = FIXED ? 16 : 4;
+  if (p.lanes == kOther) return launch_w<XT, LUT, kOther, FIXED>(p, kpad, stream);
   return hipErrorInvalidValue;
 }
 
 }  // namespace
 
+// The full path's chunks are a serial chain per lane, so a workgroup of 8
+// lanes (2 waves per SIMD) is taken when that gives every CU at most one
+// workgroup's worth of work or the chip is full, and 4 lanes (one wave per
+// SIMD, a shorter chunk) where 4-lane workgroups still fit one per CU, or where
+// 8-lane ones would give a few CUs a second (1 to 1.5 per CU).  Measured on
+// MI355X, K=8, 8 lanes against 4: B=1 S=4096 D=512 (64 workgroups of 8) 41.1
+// and 38.4 us, B=2 D=384 (96) 42.1 and 39.7, B=3 D=512 (192) 44.5 and 47.5, B=4
+// (256) 43.2 and 46.6, B=5 (320) 62.7 and 57.4, B=8 (512) 65.5 and 68.0.  16
+// lanes were never faster (112.6 us against 107 at B=24 S=2048, 81 against 72
+// at B=32 S=1024).
 int v10_lanes(int64_t B, int64_t H, int64_t hd) {
-  return B * H * ((hd + 15) / 16) >= 512 ? 16 : 8;
+  constexpr int64_t kCus = 256;
+  const int64_t n8 = B * H * ((hd + 7) / 8);
+  return n8 <= kCus / 2 || (n8 > kCus && n8 <= kCus + kCus / 2) ? 4 : 8;
 }
+
+// The fixed forward's walk: 16 lanes when that gives 512 workgroups.
+int v10_fixed_lanes(int64_t B, int64_t H, int64_t hd) { return B * H * ((hd + 15) / 16) >= 512 ? 16 : 8; }
 
 hipError_t launch_v10(const V10Params& p, int x_dtype, bool use_lut, int kpad, hipStream_t stream) {
   if (x_dtype == 0)

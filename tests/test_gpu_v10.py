@@ -32,7 +32,10 @@ def oracle(x, c, m, **kw):
     (2, 1300, 4, 16, 6, 512, True),     # chunks of two 256-token blocks
     (1, 700, 8, 16, 8, 700, True),      # S <= chunk: one chunk of 700
     (2, 257, 4, 16, 8, 256, True),      # a 1-token last chunk (NaN momentum, as the reference)
-    (8, 300, 8, 128, 8, 256, True),     # >= 512 workgroups of 16 lanes: the 16-lane kernel
+    (8, 300, 8, 128, 8, 256, True),     # 1024 workgroups of 8 lanes
+    (5, 300, 8, 50, 8, 256, True),      # 280 of them would be: 4-lane workgroups, the last of 2 lanes
+    (17, 260, 4, 64, 4, 128, True),     # 544, four coefficients
+    (1, 300, 1, 6, 5, 256, False),      # two workgroups of 4 lanes, on a grid padded to eight
 ])
 def test_v10_full_path_matches_oracle(dev, B, S, H, hd, K, chunk, use_lut):
     x, c, m = case(B, S, H, hd, K, seed=S + K, mom_scale=0.01)

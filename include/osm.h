@@ -318,6 +318,39 @@ typedef struct osm_lut_fwd_args {
   int64_t final_stride_b;
 } osm_lut_fwd_args;
 
+/*
+ * The engine's steps ahead of its Chebyshev path (sdpc_engine.py:163-209),
+ * fp32, without gradients:
+ *
+ *   x_normed[b,t,:] = x[b,t,:] / sqrt(mean_d x[b,t,d]^2 + eps) * norm_weight
+ *   gate[b] = sigmoid(w2 silu(w1 mean_t x_normed[b,t,:] + b1) + b2)
+ *   *tokens_seen += S
+ *   *ema_momentum = 0.7 + 0.5 (*ema_base - 0.7) (1 + cos(pi clamp(*tokens_seen / 1e8, 0, 1)))
+ *
+ * D a multiple of 4, at most OSM_ENGINE_MAX_D; rows of x, and every weight,
+ * on 16-byte boundaries.  Two launches on `stream`.
+ */
+#define OSM_ENGINE_MAX_D 1024
+
+typedef struct osm_engine_args {
+  int32_t abi_version;          /* = OSM_ABI_VERSION */
+  float eps;
+  int64_t B, S, D;              /* B, S >= 1 */
+  const float* x;               /* [B,S,D], lane stride 1 */
+  int64_t x_stride_b, x_stride_s;
+  const float* norm_weight;     /* [D] */
+  const float* w1;              /* [D/4, D] */
+  const float* b1;              /* [D/4] */
+  const float* w2;              /* [1, D/4] */
+  const float* b2;              /* [1] */
+  const float* ema_base;        /* device scalar */
+  int64_t* tokens_seen;         /* device scalar, advanced by S */
+  float* x_normed;              /* [B,S,D] contiguous */
+  float* gate;                  /* [B] */
+  float* ema_momentum;          /* device scalar */
+  float* scratch;               /* osm_engine_scratch_bytes, 16-byte aligned */
+} osm_engine_args;
+
 /* Which entry point a workspace is sized for. */
 typedef enum osm_op { OSM_OP_FWD = 0, OSM_OP_TTT = 1, OSM_OP_BWD = 2 } osm_op;
 
@@ -397,6 +430,11 @@ int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* args, void* stream);
  * and the workspace may be NULL. */
 size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* args);
 int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The engine steps described above osm_engine_args; scratch bytes for B, S
+ * and D (contents need no initialisation and are not kept). */
+size_t osm_engine_scratch_bytes(int64_t B, int64_t S, int64_t D);
+int osm_engine_prologue(const osm_engine_args* args, void* stream);
 
 /* Backward of osm_cheby_ema_fwd: writes grad_x and, when non-NULL,
  * grad_coeffs and grad_init.  Replaces the backward listed in the header

@@ -30,6 +30,7 @@ OP_TTT = 1
 OP_BWD = 2
 OP_LUT = 3   # key of the fixed-coefficient scan's workspaces (not an osm_op)
 V10_USE_LUT = 0x1
+ENGINE_MAX_D = 1024   # row length of osm_engine_prologue
 
 STATUS = {
     0: "OSM_OK",
@@ -61,6 +62,8 @@ EXPORTS = (
     "osm_cheby_ema_lut_fwd",
     "osm_lut_fwd_workspace_bytes",
     "osm_cheby_ema_lut_fwd_ws",
+    "osm_engine_scratch_bytes",
+    "osm_engine_prologue",
 )
 
 
@@ -239,6 +242,32 @@ class LutFwdArgs(ctypes.Structure):
     ]
 
 
+class EngineArgs(ctypes.Structure):
+    """Mirror of ``osm_engine_args``."""
+
+    _fields_ = [
+        ("abi_version", ctypes.c_int32),
+        ("eps", ctypes.c_float),
+        ("B", ctypes.c_int64),
+        ("S", ctypes.c_int64),
+        ("D", ctypes.c_int64),
+        ("x", ctypes.c_void_p),
+        ("x_stride_b", ctypes.c_int64),
+        ("x_stride_s", ctypes.c_int64),
+        ("norm_weight", ctypes.c_void_p),
+        ("w1", ctypes.c_void_p),
+        ("b1", ctypes.c_void_p),
+        ("w2", ctypes.c_void_p),
+        ("b2", ctypes.c_void_p),
+        ("ema_base", ctypes.c_void_p),
+        ("tokens_seen", ctypes.c_void_p),
+        ("x_normed", ctypes.c_void_p),
+        ("gate", ctypes.c_void_p),
+        ("ema_momentum", ctypes.c_void_p),
+        ("scratch", ctypes.c_void_p),
+    ]
+
+
 class OsmError(RuntimeError):
     def __init__(self, code: int, msg: str):
         super().__init__(f"{STATUS.get(code, code)}: {msg}")
@@ -294,6 +323,10 @@ def load() -> ctypes.CDLL:
         lib.osm_cheby_ema_lut_fwd_ws.restype = ctypes.c_int
         lib.osm_cheby_ema_lut_fwd_ws.argtypes = [ctypes.POINTER(LutFwdArgs), ctypes.c_void_p, ctypes.c_size_t,
                                                  ctypes.c_void_p]
+        lib.osm_engine_scratch_bytes.restype = ctypes.c_size_t
+        lib.osm_engine_scratch_bytes.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64]
+        lib.osm_engine_prologue.restype = ctypes.c_int
+        lib.osm_engine_prologue.argtypes = [ctypes.POINTER(EngineArgs), ctypes.c_void_p]
         got = lib.osm_abi_version()
         if got != ABI_VERSION:
             raise ImportError(f"orthossm_amd: library ABI {got} != binding ABI {ABI_VERSION}; rebuild")

@@ -796,6 +796,56 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   return ok();
 }
 
+size_t osm_engine_scratch_bytes(int64_t B, int64_t S, int64_t D) {
+  if (B < 1 || S < 1 || D < 1) return 0;
+  return (size_t)B * (size_t)osm::engine_tiles(S) * (size_t)D * sizeof(float);
+}
+
+int osm_engine_prologue(const osm_engine_args* a, void* stream) {
+  if (!a) return fail(OSM_E_ARG, "args is NULL");
+  if (a->abi_version != OSM_ABI_VERSION)
+    return fail(OSM_E_ARG, "abi_version %d does not match library ABI %d", a->abi_version, OSM_ABI_VERSION);
+  static_assert(OSM_ENGINE_MAX_D == osm::kEngineMaxD, "the header states the kernels' limit");
+  if (a->B < 1 || a->S < 1 || a->B > 65535 || a->S >= (int64_t(1) << 30))
+    return fail(OSM_E_SHAPE, "B=%lld outside [1, 65535] or S=%lld outside [1, 2^30)", (long long)a->B, (long long)a->S);
+  if (a->D < 4 || a->D % 4 || a->D > OSM_ENGINE_MAX_D)
+    return fail(OSM_E_SHAPE, "D=%lld must be a multiple of 4 up to %d", (long long)a->D, OSM_ENGINE_MAX_D);
+  if (!a->x || !a->norm_weight || !a->w1 || !a->b1 || !a->w2 || !a->b2 || !a->ema_base || !a->tokens_seen ||
+      !a->x_normed || !a->gate || !a->ema_momentum || !a->scratch)
+    return fail(OSM_E_ARG, "every pointer must be non-NULL");
+  const void* quads[5] = {a->x, a->norm_weight, a->w1, a->x_normed, a->scratch};
+  for (const void* q : quads)
+    if ((uintptr_t)q % 16) return fail(OSM_E_LAYOUT, "x, norm_weight, w1, x_normed and scratch must be 16-byte aligned");
+  const void* words[6] = {a->b1, a->w2, a->b2, a->ema_base, a->gate, a->ema_momentum};
+  for (const void* w : words)
+    if ((uintptr_t)w % 4) return fail(OSM_E_LAYOUT, "b1, w2, b2, ema_base, gate and ema_momentum must be 4-byte aligned");
+  if ((uintptr_t)a->tokens_seen % 8) return fail(OSM_E_LAYOUT, "tokens_seen must be 8-byte aligned");
+  if (a->x_stride_b < 0 || a->x_stride_s < 0 || a->x_stride_b % 4 || a->x_stride_s % 4)
+    return fail(OSM_E_LAYOUT, "x strides must be non-negative multiples of 4");
+  osm::EngineParams p{};
+  p.x = a->x;
+  p.norm_w = a->norm_weight;
+  p.w1 = a->w1;
+  p.b1 = a->b1;
+  p.w2 = a->w2;
+  p.b2 = a->b2;
+  p.ema_base = a->ema_base;
+  p.tokens = reinterpret_cast<long long*>(a->tokens_seen);
+  p.xn = a->x_normed;
+  p.gate = a->gate;
+  p.mu = a->ema_momentum;
+  p.part = a->scratch;
+  p.x_sb = a->x_stride_b;
+  p.x_ss = a->x_stride_s;
+  p.B = (int)a->B;
+  p.S = (int)a->S;
+  p.D = (int)a->D;
+  p.eps = a->eps;
+  const hipError_t e = osm::launch_engine(p, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "engine prologue launch");
+  return ok();
+}
+
 int osm_cheby_ema_bwd(const osm_cheby_args* args, const osm_cheby_bwd_args* bwd, void* workspace,
                       size_t workspace_bytes, void* stream) {
   Geometry geo;

@@ -265,6 +265,26 @@ struct V10BwdParams {
   float mu;
 };
 
+// The engine's input norm, complexity gate and momentum schedule (osm_engine).
+constexpr int kEngineMaxD = 1024;   // row length the kernels hold in registers and LDS
+struct EngineParams {
+  const float* x;
+  const float* norm_w;         // [D]
+  const float* w1;             // [D/4, D]
+  const float* b1;             // [D/4]
+  const float* w2;             // [D/4]
+  const float* b2;             // [1]
+  const float* ema_base;       // scalar
+  long long* tokens;           // scalar, advanced by S
+  float* xn;                   // [B,S,D] contiguous
+  float* gate;                 // [B]
+  float* mu;                   // scalar
+  float* part;                 // [B][engine_tiles(S)][D]
+  int64_t x_sb, x_ss;
+  int B, S, D;
+  float eps;
+};
+
 // Multiplier and shift that divide by v (1 <= v < 2^31) for dividends
 // 0 <= n < 2^31: s = ceil(log2 v), m = floor(2^32 (2^s - v) / v) + 1
 // (Granlund and Montgomery, "Division by invariant integers using
@@ -296,6 +316,8 @@ hipError_t launch_v10_bwd(const V10BwdParams& p, int x_dtype, int lpt, int kpad,
 hipError_t launch_v10_fixed(const V10FixedParams& p, int x_dtype, bool use_lut, int kpad, hipStream_t stream);
 hipError_t launch_lut_scan(const LutScanParams& p, int x_dtype, bool use_lut, FwdShape s, int kpad,
                            hipStream_t stream);
+int engine_tiles(int64_t S);
+hipError_t launch_engine(const EngineParams& p, hipStream_t stream);
 hipError_t launch_fill_zero(void* ptr, size_t bytes, hipStream_t stream);
 hipError_t launch_copy_state(const float* src, float* dst, size_t n, hipStream_t stream);
 hipError_t launch_ws_status(void* ws, unsigned* dst, int reset, hipStream_t stream);

@@ -51,9 +51,12 @@ from typing import NamedTuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as nn_module
+from torch.autograd import forward_ad
 from torch.utils.checkpoint import checkpoint as torch_checkpoint
 
-from .ops import cheby_ema, cheby_ema_forward, head_momentum
+from ._native import ENGINE_MAX_D
+from .ops import cheby_ema, cheby_ema_forward, engine_prologue, head_momentum
 from .sdpc_kernel import GatedComplexityPredictor, apply_cheby_rkv_v10, v10_damping
 
 # Length routing thresholds (sdpc_engine.py:51-53).
@@ -168,23 +171,75 @@ class ChebyContextPath(nn.Module):
             return cheby_ema(x_normed, coeffs, damping, lam, **kw)
         return cheby_ema_forward(x_normed, coeffs, damping, lam, **kw)
 
+    def _fused_weights(self, x: torch.Tensor):
+        """(norm weight, eps, W1, b1, W2, b2) when ``engine_prologue`` stands
+        for this call's norm, gate and schedule, else None: inference on plain
+        fp32 tensors of one device, with the submodules as __init__ makes them
+        and nothing attached that a module call would run (hooks, autocast,
+        tracing, forward-mode gradients).  Looked at afresh on every call."""
+        if (torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dtype is not torch.float32 or not x.is_cuda or
+                x.numel() == 0 or x.shape[0] > 65535 or x.shape[2] % 4 or x.shape[2] > ENGINE_MAX_D or
+                x.stride(2) != 1 or x.stride(0) % 4 or x.stride(1) % 4 or x.data_ptr() % 16):
+            return None
+        if (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling() or
+                forward_ad._current_level >= 0 or nn_module._global_forward_hooks or
+                nn_module._global_forward_pre_hooks):
+            return None
+        norm, cg = self._modules["input_norm"], self._modules["complexity_gate"]
+        if type(norm) is not nn.RMSNorm or type(cg) is not GatedComplexityPredictor:
+            return None
+        net = cg._modules["net"]
+        if type(net) is not nn.Sequential or len(net) != 4:
+            return None
+        l1, act, l2, sig = net._modules.values()
+        if type(l1) is not nn.Linear or type(act) is not nn.SiLU or type(l2) is not nn.Linear or \
+                type(sig) is not nn.Sigmoid:
+            return None
+        for m in (norm, cg, net, l1, act, l2, sig):
+            if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                return None
+        D = x.shape[2]
+        shapes = ((norm._parameters["weight"], (D,)), (l1._parameters["weight"], (D // 4, D)),
+                  (l1._parameters["bias"], (D // 4,)), (l2._parameters["weight"], (1, D // 4)),
+                  (l2._parameters["bias"], (1,)))
+        dev = x.device
+        for w, shape in shapes:
+            if type(w) is not nn.Parameter or w.dtype is not torch.float32 or w.device != dev or \
+                    w.shape != shape or not w.is_contiguous() or w.data_ptr() % 16:
+                return None
+        base, seen = self._buffers["ema_base"], self._buffers["total_tokens_seen"]
+        if base.dtype is not torch.float32 or seen.dtype is not torch.long or base.device != dev or \
+                seen.device != dev or base.numel() != 1 or seen.numel() != 1:
+            return None
+        if tuple(norm.normalized_shape) != (D,):
+            return None
+        w = [p for p, _ in shapes]
+        return w[0], torch.finfo(torch.float32).eps if norm.eps is None else norm.eps, *w[1:]
+
     def forward(self, x: torch.Tensor, cheby_state=None) -> ChebyPathOutput:
         B, S, D = x.shape
         if D != self.d_model:
             raise ValueError(f"x has D={D}, the module d_model={self.d_model}")
         n_h, hd, deg = self.n_cheby_heads, self.head_dim, self.max_degree
-        x_normed = self.input_norm(x)
-        x_mean = x_normed.mean(dim=1)
-        if cheby_state is None:
-            coeffs = self.coeff_init_proj(x_mean).view(B, n_h, deg, hd) * self.coeff_spectral_scale
-            momentum = torch.zeros(B, n_h, deg, hd, device=x.device)
-            ema = None
-        else:
+        # A call that continues from a state needs the mean of the normalised
+        # input for the gate alone, so norm, mean, gate and schedule fuse.
+        fused = self._fused_weights(x) if cheby_state is not None else None
+        if fused is not None:
             coeffs, momentum, ema = parse_cheby_state(cheby_state, deg)
-        gate = self.complexity_gate(x_mean)
-        with torch.no_grad():
-            self.total_tokens_seen.add_(S)
-            mu = ema_momentum_schedule(self.total_tokens_seen, self.ema_base).float()
+            x_normed, gate, mu = engine_prologue(x, *fused, self.ema_base, self.total_tokens_seen)
+        else:
+            x_normed = self.input_norm(x)
+            x_mean = x_normed.mean(dim=1)
+            if cheby_state is None:
+                coeffs = self.coeff_init_proj(x_mean).view(B, n_h, deg, hd) * self.coeff_spectral_scale
+                momentum = torch.zeros(B, n_h, deg, hd, device=x.device)
+                ema = None
+            else:
+                coeffs, momentum, ema = parse_cheby_state(cheby_state, deg)
+            gate = self.complexity_gate(x_mean)
+            with torch.no_grad():
+                self.total_tokens_seen.add_(S)
+                mu = ema_momentum_schedule(self.total_tokens_seen, self.ema_base).float()
 
         tier = route(S)
         if tier == "fast":

@@ -587,6 +587,31 @@ def v10_chunked_ttt(x: torch.Tensor, coeffs: torch.Tensor, momentum: torch.Tenso
     return out, c_out, m_out
 
 
+def engine_prologue(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w1: torch.Tensor, b1: torch.Tensor,
+                    w2: torch.Tensor, b2: torch.Tensor, ema_base: torch.Tensor, tokens_seen: torch.Tensor):
+    """The engine's input norm, complexity gate and momentum schedule
+    (sdpc_engine.py:163-209) in two launches, without gradients; tokens_seen
+    (int64 scalar) is advanced by S in place.  x [B,S,D] fp32 and the weights
+    fp32 contiguous on x's device, D a multiple of 4 up to ENGINE_MAX_D.
+    Returns (x_normed [B,S,D], gate [B,1], mu, a 0-d tensor)."""
+    lib = nat.load()
+    dev = x.device
+    B, S, D = x.shape
+    xn = torch.empty((B, S, D), device=dev, dtype=torch.float32)
+    scratch = torch.empty(lib.osm_engine_scratch_bytes(B, S, D) // 4, device=dev, dtype=torch.float32)
+    small = torch.empty(B + 1, device=dev, dtype=torch.float32)
+    gate, mu = small[:B].view(B, 1), small[B]
+    a = nat.EngineArgs()
+    a.abi_version, a.eps = nat.ABI_VERSION, float(eps)
+    a.B, a.S, a.D = B, S, D
+    a.x, a.x_stride_b, a.x_stride_s = x.data_ptr(), x.stride(0), x.stride(1)
+    a.norm_weight, a.w1, a.b1 = norm_weight.data_ptr(), w1.data_ptr(), b1.data_ptr()
+    a.w2, a.b2, a.ema_base, a.tokens_seen = w2.data_ptr(), b2.data_ptr(), ema_base.data_ptr(), tokens_seen.data_ptr()
+    a.x_normed, a.gate, a.ema_momentum, a.scratch = xn.data_ptr(), gate.data_ptr(), mu.data_ptr(), scratch.data_ptr()
+    nat.check(lib.osm_engine_prologue(ctypes.byref(a), ctypes.c_void_p(_current_stream(dev))))
+    return xn, gate, mu
+
+
 def _rows_dest(t: torch.Tensor | None, shape, dev, name: str) -> torch.Tensor | None:
     """A caller's [B,S,D] or [B,D] fp32 output with lane stride 1, or None."""
     if t is None:

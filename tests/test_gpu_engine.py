@@ -212,3 +212,66 @@ def test_checkpointing_keeps_gradients(dev, S):
             continue
         assert torch.isfinite(a).all() and a.abs().max() > 0
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,S,D_", [
+    (1, 1, 64),          # one row: seven of a tile's waves have none
+    (3, 9, 4),           # one float4 a row, one hidden unit, a second tile of one row
+    (2, 100, 132),       # rows of 33 pieces
+    (1, 1025, 260),      # 129 tiles' worth of rows, just past one register set
+    (2, 300, 512),
+    (5, 130, 1024),      # the longest rows
+])
+def test_prologue_matches_module_calls(dev, B, S, D_):
+    """engine_prologue against the modules in float64: the norm's mean of D
+    squares and the mean over S tokens are fp32 sums of at most eight serial
+    terms per stage (2e-6 of the largest value covers their rounding), the
+    gate's logit a dot product of D/4 + D terms (1e-5)."""
+    torch.manual_seed(S + D_)
+    m = E.ChebyContextPath(D_, n_cheby_heads=1, max_degree=K).to(dev)
+    x = torch.randn(B, S + 2, D_, generator=torch.Generator().manual_seed(S)).to(dev)[:, 1:S + 1] * 1.7
+    with torch.no_grad():
+        m.input_norm.weight.uniform_(0.5, 1.5)
+        m.total_tokens_seen.fill_(12_345_678)
+        fused = m._fused_weights(x)
+        assert fused is not None
+        xn, gate, mu = E.engine_prologue(x, *fused, m.ema_base, m.total_tokens_seen)
+        torch.cuda.synchronize()
+        assert m.total_tokens_seen.item() == 12_345_678 + S
+        want_mu = E.ema_momentum_schedule(m.total_tokens_seen, m.ema_base)
+        assert abs(float(mu) - float(want_mu)) <= 1e-7
+        xd = x.double()
+        wn = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + torch.finfo(torch.float32).eps) * \
+            m.input_norm.weight.double()
+        assert (xn - wn).abs().max() <= 2e-6 * wn.abs().max()
+        wg = m.complexity_gate.double()(wn.mean(1))
+        assert gate.shape == wg.shape and (gate - wg).abs().max() <= 1e-5
+
+
+def test_fused_and_module_prologue_agree_on_every_route(dev):
+    """A continued call with and without the fused prologue (a hook on the
+    norm takes it off), carry included; with gradients enabled the modules run."""
+    for S, carry in ((40, True), (200, False), (600, False), (1100, True)):
+        runs = []
+        for hook in (False, True):
+            m = make(dev, seed=3, carry_ema=carry)
+            m.total_tokens_seen.fill_(5_000_000)
+            x = torch.randn(2, S, D, generator=torch.Generator().manual_seed(S)).to(dev)
+            c = torch.randn(2, H, K, D // H, generator=torch.Generator().manual_seed(1)).to(dev) * 0.3
+            state = (c, torch.full_like(c, 0.02))
+            if carry:
+                state = E.ChebyState(*state, torch.full((2, D), 0.2, device=dev))
+            seen = []
+            if hook:
+                m.input_norm.register_forward_hook(lambda *a: seen.append(1))
+            with torch.no_grad():
+                assert (m._fused_weights(x) is None) == hook
+                r = m(x, state)
+            assert len(seen) == int(hook)
+            assert m._fused_weights(x) is None          # gradients enabled
+            runs.append((r.x_normed, r.gate, r.ema_momentum.reshape(1), r.out, *[s for s in r.state if s is not None]))
+        for a, b in zip(*runs):
+            # outputs of the full path are bf16 values: a last-place change of
+            # x_normed may move one by an ulp (bf16 has seven fraction bits: 2^-7
+            # of itself at most)
+            torch.testing.assert_close(a, b, rtol=2.0 ** -7, atol=2e-6)

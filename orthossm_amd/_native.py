@@ -7,6 +7,8 @@ missing, every entry point raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -332,6 +334,33 @@ def load() -> ctypes.CDLL:
             raise ImportError(f"orthossm_amd: library ABI {got} != binding ABI {ABI_VERSION}; rebuild")
         _lib = lib
         return lib
+
+
+EXT_PATH = os.path.join(os.path.dirname(LIB_PATH), "osm_torch.so")
+_ext = None
+
+
+def load_ext():
+    """The extension module ``osm_torch`` (csrc/osm_torch.cpp), imported once."""
+    global _ext
+    if _ext is None:
+        with _lock:
+            if _ext is None:
+                if not os.path.exists(EXT_PATH):
+                    raise ImportError(f"orthossm_amd: extension {EXT_PATH} is missing; build it with "
+                                      "`python -m orthossm_amd.build`.")
+                loader = importlib.machinery.ExtensionFileLoader("osm_torch", EXT_PATH)
+                spec = importlib.util.spec_from_file_location("osm_torch", EXT_PATH, loader=loader)
+                mod = importlib.util.module_from_spec(spec)
+                loader.exec_module(mod)
+                _ext = mod
+    return _ext
+
+
+# The functions osm_torch takes by address, in the order of its init().
+EXT_FUNCTIONS = ("osm_workspace_bytes", "osm_cheby_ema_fwd", "osm_cheby_ema_ttt", "osm_cheby_ema_bwd",
+                 "osm_v10_chunked_ttt", "osm_v10_bwd", "osm_lut_fwd_workspace_bytes", "osm_cheby_ema_lut_fwd_ws",
+                 "osm_engine_scratch_bytes", "osm_engine_prologue")
 
 
 def check(rc: int) -> None:

@@ -3,7 +3,9 @@
     python -m orthossm_amd.build
 
 Compiles every ``csrc/*.hip`` source with hipcc for gfx950 into one
-shared library exporting the C ABI of ``include/osm.h``.  Packed FP32 math
+shared library exporting the C ABI of ``include/osm.h``, and
+``csrc/osm_torch.cpp`` (host code) into the extension module
+``_lib/osm_torch.so`` through which the torch operators launch.  Packed FP32 math
 (v_pk_*_f32) is disabled on purpose: the kernels are written in scalar fp32.
 """
 from __future__ import annotations
@@ -64,6 +66,25 @@ def device_asm_command(src: str, out: str) -> list[str]:
     return [hipcc_path(), *common_flags(), "--offload-device-only", "-S", "-o", out, src]
 
 
+TORCH_EXT_SRC = os.path.join(CSRC, "osm_torch.cpp")
+TORCH_EXT_PATH = os.path.join(LIB_DIR, "osm_torch.so")
+
+
+def torch_ext_command(out: str) -> list[str]:
+    """The torch-facing launch path (host code only; it takes the library's
+    functions by address, so it does not link against it)."""
+    import sysconfig
+
+    import torch
+    base = os.path.dirname(os.path.abspath(torch.__file__))
+    inc = os.path.join(base, "include")
+    return [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-shared", "-o", out, TORCH_EXT_SRC,
+            "-I", INCLUDE, "-I", inc, "-I", os.path.join(inc, "torch", "csrc", "api", "include"),
+            "-I", sysconfig.get_paths()["include"], f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-L", os.path.join(base, "lib"),
+            "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10"]
+
+
 def build(verbose: bool = False) -> str:
     """Compiles the library (always, even if one exists) and returns its path."""
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -79,22 +100,29 @@ def build(verbose: bool = False) -> str:
             print(" ".join(cmd), flush=True)
         objs.append(obj)
         procs.append(subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True))
+    ext_tmp = TORCH_EXT_PATH + f".tmp{tag}"
+    cmd = torch_ext_command(ext_tmp)
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    objs.append(ext_tmp)
+    procs.append(subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True))
     errors = []
-    for src, pr in zip(sources(), procs):
+    for src, pr in zip([*sources(), TORCH_EXT_SRC], procs):
         _, err = pr.communicate()
         if pr.returncode != 0:
-            errors.append(f"{os.path.basename(src)}: hipcc failed ({pr.returncode}):\n{err[-8000:]}")
+            errors.append(f"{os.path.basename(src)}: compiler failed ({pr.returncode}):\n{err[-8000:]}")
     tmp = LIB_PATH + f".tmp{tag}"
     try:
         if errors:
             raise RuntimeError("\n".join(errors))
-        cmd = link_command(objs, tmp)
+        cmd = link_command(objs[:-1], tmp)
         if verbose:
             print(" ".join(cmd), flush=True)
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError(f"link failed ({res.returncode}):\n{res.stderr[-8000:]}")
         os.replace(tmp, LIB_PATH)
+        os.replace(ext_tmp, TORCH_EXT_PATH)
     finally:
         for f in objs + [tmp]:
             if os.path.exists(f):

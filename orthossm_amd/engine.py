@@ -56,8 +56,8 @@ from torch.autograd import forward_ad
 from torch.utils.checkpoint import checkpoint as torch_checkpoint
 
 from ._native import ENGINE_MAX_D
-from .ops import cheby_ema, cheby_ema_forward, engine_prologue, head_momentum
-from .sdpc_kernel import GatedComplexityPredictor, apply_cheby_rkv_v10, v10_damping
+from .ops import cheby_ema, cheby_ema_forward, engine_prologue
+from .sdpc_kernel import GatedComplexityPredictor, _fast_constants, apply_cheby_rkv_v10
 
 # Length routing thresholds (sdpc_engine.py:51-53).
 FAST_PATH_THRESHOLD = 384
@@ -163,8 +163,7 @@ class ChebyContextPath(nn.Module):
         dev = x_normed.device
         H = self.n_cheby_heads
         coeffs = coeffs.float()
-        damping = v10_damping(H, dev)
-        lam = head_momentum(ema_momentum, H, dev)
+        damping, lam = _fast_constants(H, dev, ema_momentum)
         kw = dict(ema_init=ema_init, out_dtype=torch.float32, return_state=True, nan_policy="zero_u")
         if torch.is_grad_enabled() and (x_normed.requires_grad or coeffs.requires_grad or
                                         (ema_init is not None and ema_init.requires_grad)):

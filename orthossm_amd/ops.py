@@ -132,6 +132,37 @@ def _current_stream(dev: torch.device) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
 
 
+# The native launch path (csrc/osm_torch.cpp) and the library it was
+# initialised for.  Its functions return None for what is not in the kernel's
+# own form; the Python code below each call then converts, or raises.
+_ext = None
+_ext_for = None
+_DTYPE_CODE = {None: None, torch.float32: nat.F32, torch.bfloat16: nat.BF16}
+
+
+def _fast():
+    """The native launch path, or None where the Python path has to run: with
+    fault checks on, or a library object that is not the loaded one."""
+    global _ext, _ext_for
+    lib = nat.load()
+    if _ext_for is not lib:
+        if _raw_stream is None or not isinstance(lib, ctypes.CDLL):
+            return None
+        ext = nat.load_ext()
+        ext.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in nat.EXT_FUNCTIONS), _raw_stream,
+                 _ws_cache, _workspace, nat.check)
+        _ext, _ext_for = ext, lib
+    return None if _check_faults else _ext
+
+
+def _flags(clamp: bool, nan_policy: str) -> int:
+    if nan_policy not in ("zero_z", "zero_u"):
+        raise ValueError("nan_policy must be 'zero_z' or 'zero_u'")
+    return ((0 if clamp else nat.FLAG_NO_CLAMP) | (nat.FLAG_NAN_ZERO_U if nan_policy == "zero_u" else 0) |
+            (nat.FLAG_TIMING_JITTER if _timing_jitter else 0) |
+            (nat.FLAG_POLL_LIMIT_ZERO if _poll_limit_zero else 0))
+
+
 def _workspace(device: torch.device, stream: int, nbytes: int, op: int) -> torch.Tensor:
     """Zero-initialised workspace reused per (device, stream, entry point).
     Calls on one stream are ordered, so they never overlap on a workspace;
@@ -217,11 +248,7 @@ def _prepare(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, ema_init, 
         raise ValueError("out must have a contiguous lane dimension and non-negative strides")
     a = nat.ChebyArgs()
     a.abi_version = nat.ABI_VERSION
-    if nan_policy not in ("zero_z", "zero_u"):
-        raise ValueError("nan_policy must be 'zero_z' or 'zero_u'")
-    a.flags = ((0 if clamp else nat.FLAG_NO_CLAMP) | (nat.FLAG_NAN_ZERO_U if nan_policy == "zero_u" else 0) |
-               (nat.FLAG_TIMING_JITTER if _timing_jitter else 0) |
-               (nat.FLAG_POLL_LIMIT_ZERO if _poll_limit_zero else 0))
+    a.flags = _flags(clamp, nan_policy)
     a.B, a.S, a.H, a.hd, a.K = B, S, H, hd, K
     a.x, a.x_dtype, a.x_stride_b, a.x_stride_s = x.data_ptr(), _dtype_code(x.dtype), x.stride(0), x.stride(1)
     a.out_dtype = _dtype_code(odt)
@@ -255,6 +282,12 @@ def cheby_ema_forward(x: torch.Tensor, coeffs: torch.Tensor, damping: Sequence[f
     NaN input gives z = 0 ('zero_z', the reference's Triton kernels) or counts
     as u = 0 ('zero_u', the reference's PyTorch fast path).
     """
+    fast = _fast()
+    if fast is not None and out_dtype in _DTYPE_CODE:
+        res = fast.forward(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, _flags(clamp, nan_policy), ema_init,
+                           _DTYPE_CODE[out_dtype], out, return_state, state_out)
+        if res is not None:
+            return res if return_state else res[0]
     lib = nat.load()
     a, out, keep = _prepare(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, ema_init, clamp,
                             out_dtype, out, nan_policy)
@@ -287,6 +320,12 @@ def cheby_ema_ttt(x: torch.Tensor, coeffs: torch.Tensor, damping, lam, *, g: tor
     tgt = {"x": nat.TARGET_X, "softsign": nat.TARGET_SOFTSIGN}.get(target)
     if tgt is None:
         raise ValueError("target must be 'x' or 'softsign'")
+    fast = _fast()
+    if fast is not None and grad_out is None and out_dtype in _DTYPE_CODE:
+        res = fast.ttt(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, _flags(clamp, nan_policy), ema_init,
+                       _DTYPE_CODE[out_dtype], out, return_state, state_out, tgt)
+        if res is not None:
+            return res if return_state else res[:2]
     a, out, keep = _prepare(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, ema_init, clamp,
                             out_dtype, out, nan_policy)
     dev = out.device
@@ -332,6 +371,14 @@ def cheby_ema_backward(x: torch.Tensor, coeffs: torch.Tensor, damping, lam, out:
     lib = nat.load()
     if out is None and clamp:
         raise ValueError("the saved forward output is needed for the clamp mask")
+    fast = _fast()
+    if fast is not None and z_saved is None and grad_x_out is None and grad_coeffs_out is None and \
+            grad_init_out is None:
+        res = fast.backward(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max,
+                            _flags(clamp, nan_policy) | (nat.FLAG_FULL_JACOBIAN if full_jacobian else 0), out, grad_out,
+                            grad_state, need_coeffs, need_init)
+        if res is not None:
+            return res
     a, _, keep = _prepare(x, coeffs, damping, lam, g, lam_shift, lam_min, lam_max, None, clamp,
                           out.dtype if out is not None else None, out, nan_policy, alloc_out=False)
     xin = keep[0]
@@ -395,6 +442,7 @@ class _ChebyEMAFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, coeffs, ema_init, damping, lam, g, lam_shift, lam_min, lam_max, clamp, out_dtype,
                 nan_policy):
+        ctx.set_materialize_grads(False)   # an unused output's gradient stays None
         out, fin = cheby_ema_forward(x, coeffs, damping, lam, g=g, lam_shift=lam_shift, lam_min=lam_min,
                                      lam_max=lam_max, ema_init=ema_init, clamp=clamp, out_dtype=out_dtype,
                                      return_state=True, nan_policy=nan_policy)
@@ -517,6 +565,14 @@ def v10_chunked_ttt(x: torch.Tensor, coeffs: torch.Tensor, momentum: torch.Tenso
     save_for_backward, also (z [B,S,D] bf16, coeff_hist [n_chunks,B,H,K,hd]).
     """
     lib = nat.load()
+    fast = _fast()
+    if fast is not None and isinstance(x, torch.Tensor) and x.is_cuda and isinstance(coeffs, torch.Tensor) and \
+            coeffs.dim() == 4:
+        lut, lion_lambda, ss, lr_scale = v10_tables(x.device, n_heads, min(coeffs.shape[2], nat.MAX_K_V10))
+        res = fast.v10(x, coeffs, momentum, n_heads, gate_global, dynamic_lambda, ema_momentum, lut, lion_lambda, ss,
+                       lr_scale, base_lr, beta1, beta2, weight_decay, chunk_size, use_lut, save_for_backward)
+        if res is not None:
+            return res
     if not isinstance(x, torch.Tensor) or x.dim() != 3:
         raise ValueError("x must be a [B,S,D] tensor")
     if x.device.type != "cuda":
@@ -594,6 +650,9 @@ def engine_prologue(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w1: 
     (int64 scalar) is advanced by S in place.  x [B,S,D] fp32 and the weights
     fp32 contiguous on x's device, D a multiple of 4 up to ENGINE_MAX_D.
     Returns (x_normed [B,S,D], gate [B,1], mu, a 0-d tensor)."""
+    fast = _fast()
+    if fast is not None:
+        return fast.engine(x, norm_weight, eps, w1, b1, w2, b2, ema_base, tokens_seen)
     lib = nat.load()
     dev = x.device
     B, S, D = x.shape
@@ -644,6 +703,13 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     if x.device.type != "cuda":
         raise RuntimeError("orthossm_amd runs on a ROCm GPU only; x is on " + str(x.device))
     dev = x.device
+    fast = _fast()
+    if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and ema_final is None:
+        table = v10_tables(dev, n_heads, LUT_TERMS)[0] if use_lut else None
+        res = fast.lut_forward(x, coeffs, n_heads, ema_momentum, ema_init, use_lut, table, clamp_tile, want_x_norm,
+                               want_tanh_y)
+        if res is not None:
+            return res
     B, S, D = x.shape
     if x.dtype not in (torch.float32, torch.bfloat16):
         x = x.float()
@@ -736,6 +802,11 @@ def _v10_backward(x, out, z, hist, grad_out, n_heads, ema_momentum, chunk, need_
                                        grad_out.to(dtype=torch.float32).contiguous(), clamp=True,
                                        nan_policy="zero_u", z_saved=z, full_jacobian=True)
         return gx, gc
+    fast = _fast()
+    if fast is not None:
+        gx = fast.v10_backward(x, out, z, hist, grad_out, ema_momentum, chunk)
+        if gx is not None:
+            return gx, None
     lib = nat.load()
     xr = _rows(x, x.dtype if x.dtype in (torch.float32, torch.bfloat16) else torch.float32, dev)
     go, out, z = _rows(grad_out, torch.float32, dev), _rows(out, torch.float32, dev), _rows(z, torch.bfloat16, dev)
@@ -765,6 +836,7 @@ class _V10FullFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, coeffs, momentum, kw):
+        ctx.set_materialize_grads(False)   # no gradient flows through the Lion state
         out, c_new, m_new, z, hist = v10_chunked_ttt(x, coeffs, momentum, save_for_backward=True, **kw)
         ctx.save_for_backward(x, out, z, hist)
         ctx.kw = kw

@@ -655,7 +655,7 @@ int osm_v10_chunked_ttt(const osm_v10_args* a, void* stream) {
   p.beta1 = a->beta1;
   p.beta2 = a->beta2;
   p.wd = a->weight_decay;
-  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 8) return fail(OSM_E_SHAPE, "problem too large");
+  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 64) return fail(OSM_E_SHAPE, "problem too large");
   const hipError_t e = osm::launch_v10(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0, a->K <= 4 ? 4 : 8,
                                        static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "full-path kernel launch");
@@ -755,7 +755,7 @@ int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* a, void* stream) {
   // clamp boundaries fall between waves.
   p.lanes = a->clamp_tile % 32 ? 16 : osm::v10_fixed_lanes(a->B, a->H, a->hd);
   p.n_lg = (int)((a->hd + p.lanes - 1) / p.lanes);
-  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 8) return fail(OSM_E_SHAPE, "problem too large");
+  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 64) return fail(OSM_E_SHAPE, "problem too large");
   const hipError_t e = osm::launch_v10_fixed(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0, a->K <= 4 ? 4 : 8,
                                              static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "fixed-coefficient forward launch");

@@ -224,11 +224,10 @@ __device__ __forceinline__ void look_back_issue(LookBack<G, DYN>& st, const Thre
   st.end = min(st.beg + (1 << wsh), ti.tile);
 #pragma unroll
   for (int i = 0; i < G::WPT; ++i) {
-    if (st.beg + i < st.end) {
-      const unsigned long long* s = ls.at(st.beg + i, ll);
-      st.vB[i] = peek(s);
-      if constexpr (DYN) st.vA[i] = peek(s + 1);
-    }
+    if (st.beg + i >= st.end) break;
+    const unsigned long long* s = ls.at(st.beg + i, ll);
+    st.vB[i] = peek(s);
+    if constexpr (DYN) st.vA[i] = peek(s + 1);
   }
   st.vck = 0;
   if (q.wave < G::NSUB && st.g0 > 0) st.vck = peek(ls.at(st.g0 - 1, carry_lane<G>(q)));
@@ -250,14 +249,13 @@ __device__ __forceinline__ void look_back_finish(LookBack<G, DYN>& st, ChainLds<
       const float Afull = DYN ? 1.0f : a_look;
 #pragma unroll
       for (int i = 0; i < G::WPT; ++i) {
-        if (st.beg + i < st.end) {
-          const unsigned long long* s = ls.at(st.beg + i, ll);
-          const float Bp = await_word(s, st.vB[i], tg.agg, hdr_words, limit);
-          float Ap = Afull;
-          if constexpr (DYN) Ap = await_word(s + 1, st.vA[i], tg.agg, hdr_words, limit);
-          mB = __builtin_fmaf(Ap, mB, Bp);
-          mA *= Ap;
-        }
+        if (st.beg + i >= st.end) break;
+        const unsigned long long* s = ls.at(st.beg + i, ll);
+        const float Bp = await_word(s, st.vB[i], tg.agg, hdr_words, limit);
+        float Ap = Afull;
+        if constexpr (DYN) Ap = await_word(s + 1, st.vA[i], tg.agg, hdr_words, limit);
+        mB = __builtin_fmaf(Ap, mB, Bp);
+        mA *= Ap;
       }
     }
     L.mA[q.wave][q.wl] = mA;

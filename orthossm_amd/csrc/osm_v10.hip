@@ -188,12 +188,12 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
   const int tid = threadIdx.x;
   const int l = tid % LW, g = tid / LW;
   const int wave = tid >> 6, gw = (tid & 63) / LW;   // run inside the wave
-  // Workgroups go to the 8 XCDs round-robin by index: XCD c takes the
-  // consecutive lane groups c per .. c per + per - 1, so those that share
-  // 128-byte lines of x and out are on one XCD's L2 (all but those at seven
-  // borders).
-  const int per = gridDim.x >> 3;
-  const int item = (int)(blockIdx.x & 7u) * per + (int)(blockIdx.x >> 3);
+  // Workgroups go to the 8 XCDs round-robin by index: each XCD takes every
+  // eighth group of the kShare consecutive workgroups whose lanes share a
+  // 128-byte line of fp32 x and out, so a line is fetched into one L2.
+  constexpr int kShare = 128 / (4 * LW);
+  const int slot = blockIdx.x >> 3;
+  const int item = ((slot / kShare) * 8 + (int)(blockIdx.x & 7u)) * kShare + slot % kShare;
   if (item >= p.B * p.H * p.n_lg) return;
   const int lg = item % p.n_lg;
   const int bh = item / p.n_lg;
@@ -649,7 +649,8 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
 
 template <typename XT, bool LUT, int LW, bool FIXED, typename P>
 hipError_t launch_w(const P& p, int kpad, hipStream_t stream) {
-  const unsigned grid = ((unsigned)(p.B * p.H * p.n_lg) + 7u) / 8u * 8u;
+  constexpr unsigned kRound = 8u * 128u / (4u * LW);   // whole rounds of line groups over the XCDs
+  const unsigned grid = ((unsigned)(p.B * p.H * p.n_lg) + kRound - 1u) / kRound * kRound;
   if (kpad == 4)
     hipLaunchKernelGGL((v10_chunked_kernel<XT, 4, LUT, LW, FIXED, P>), dim3(grid), dim3(kV10Groups * LW), 0, stream, p);
   else

@@ -27,6 +27,16 @@ namespace osm {
 namespace {
 
 constexpr int kChunk = 16;  // tiles merged per thread by the first merge kernel
+// Up to this many tiles one kernel merges a lane's tiles and writes the
+// gradient; past it the merge by chunks runs in parallel first.  Measured on
+// MI355X: 20.1 against 21.5 us at B=1 S=1000 (6 tiles), 25.0 and 27.7 at S=12000
+// with chunks (63 tiles), 34.5 and 38.3 at 105 tiles.
+constexpr int kDirectTiles = 32;
+// Up to this many tiles in the launch each tile converts its coefficients, as
+// the forward's do; past it (1-3% of a large launch) ttt_mono_prep converts
+// them once: 15.0 against 17.8 us at B=1 S=256 D=512, 57.9 against 59.7 at B=16
+// S=2048 (1408 tiles).
+constexpr int64_t kInlineMonoTiles = 4096;
 
 template <int KP>
 __host__ __device__ constexpr int n_fields() {
@@ -271,11 +281,20 @@ cheby_ema_ttt_kernel(const FwdParams p) {
   const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
   // This wave's monomial coefficient (wave w holds coefficient w of the 64
-  // lanes), formed once per launch by ttt_mono_prep; loaded before x.
+  // lanes), formed once per launch by ttt_mono_prep or, without a table
+  // (launches of few tiles), here; loaded before x.
   static_assert(G::NSUB == 1 && KP <= G::WAVES, "one coefficient per wave");
-  const float mono_w = q.wave < KP ? p.mono_tab[((size_t)ti.lb * KP + q.wave) * kLanes + q.wl] : 0.0f;
-  // the form of the table (1: Chebyshev coefficients, see ttt_mono_prep)
-  const bool cheb = __builtin_amdgcn_readfirstlane(p.mono_form[ti.lb]) != 0;
+  __shared__ unsigned mono_big[KP * G::NSUB];
+  float mono_w = 0.0f;
+  bool cheb = false;
+  if (p.mono_tab) {
+    if (q.wave < KP) mono_w = p.mono_tab[((size_t)ti.lb * KP + q.wave) * kLanes + q.wl];
+    // the form of the table (1: Chebyshev coefficients, see ttt_mono_prep)
+    cheb = __builtin_amdgcn_readfirstlane(p.mono_form[ti.lb]) != 0;
+  } else {
+    const auto ml = mono_issue<KP, G>(p, q, ti, a);
+    mono_store<KP, G>(ml, q, mono, mono_big);
+  }
 
   // x rows of the run (raw), g (dynamic lambda), and for the tile's last run
   // the row after the tile (its target y and lambda).
@@ -303,7 +322,7 @@ cheby_ema_ttt_kernel(const FwdParams p) {
     }
   }
 
-  if (q.wave < KP) mono[q.wave][q.wl] = mono_w;
+  if (p.mono_tab && q.wave < KP) mono[q.wave][q.wl] = mono_w;
   if constexpr (!DYN) {
     // lambda^R and lambda^TILE of each lane, by the last two waves
     if (q.wave >= G::WAVES - 2) {
@@ -313,6 +332,13 @@ cheby_ema_ttt_kernel(const FwdParams p) {
     }
   }
   __syncthreads();
+  if (!p.mono_tab) {
+    cheb = tile_cheb<KP, G>(mono_big);
+    if (cheb) {
+      mono_store_cheb<KP, G>(p, q, ti, a, mono);
+      __syncthreads();
+    }
+  }
   float c[LPT][KP];
   mono_read<G, KP>(mono, q, c);
 
@@ -614,15 +640,15 @@ __global__ void __launch_bounds__(64 * KP) ttt_merge_chunks(const float* partial
   }
 }
 
-// Level 2: merge the chunks of each lane from the sequence end (rho = 0) and
-// write grad[b,h,k,j] = G_k / (k+1)^2; thread (k, lane).
-template <int KP>
+// Level 2, or with few tiles the only one: merge the chunks (tiles) of each
+// lane from the sequence end (rho = 0), NB records at a time, and write grad[b,h,k,j] = G_k / (k+1)^2; thread (k, lane).
+template <int KP, int NB>
 __global__ void __launch_bounds__(64 * KP) ttt_finalize(const float* chunks, float* grad, int n_chunks, int n_lbd,
                                                         int D, int hd, int H, int K) {
   constexpr int F = n_fields<KP>();
   const int lb = blockIdx.x, l = threadIdx.x % kLanes, k = threadIdx.x / kLanes;
   float P, Q, Ar, Br;
-  merge_lane<KP, 8>(chunks + (size_t)lb * n_chunks * F * kLanes + l, (size_t)F * kLanes, n_chunks, k, P, Q, Ar, Br);
+  merge_lane<KP, NB>(chunks + (size_t)lb * n_chunks * F * kLanes + l, (size_t)F * kLanes, n_chunks, k, P, Q, Ar, Br);
   const int b = lb / n_lbd;
   const int d = (lb - b * n_lbd) * kLanes + l;
   if (d >= D || k >= K) return;
@@ -635,21 +661,30 @@ hipError_t launch_all(const FwdParams& p0, float* grad, hipStream_t stream) {
   const int n_chunks = (p0.n_tiles + kChunk - 1) / kChunk;
   float* chunks = p0.partials + (size_t)p0.n_lb * p0.n_tiles * n_fields<KP>() * kLanes;
   FwdParams p = p0;
-  p.mono_tab = chunks + (size_t)p.n_lb * n_chunks * n_fields<KP>() * kLanes;
-  unsigned* form = reinterpret_cast<unsigned*>(p.mono_tab + (size_t)p.n_lb * KP * kLanes);
-  p.mono_form = form;
-  hipLaunchKernelGGL((ttt_mono_prep<KP>), dim3(p.n_lb), dim3(64 * KP), 0, stream, p, p.mono_tab, form);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  hipError_t e = hipSuccess;
+  if ((int64_t)p.n_lb * p.n_tiles > kInlineMonoTiles) {
+    p.mono_tab = chunks + (size_t)p.n_lb * n_chunks * n_fields<KP>() * kLanes;
+    unsigned* form = reinterpret_cast<unsigned*>(p.mono_tab + (size_t)p.n_lb * KP * kLanes);
+    p.mono_form = form;
+    hipLaunchKernelGGL((ttt_mono_prep<KP>), dim3(p.n_lb), dim3(64 * KP), 0, stream, p, p.mono_tab, form);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
   const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   hipLaunchKernelGGL((cheby_ema_ttt_kernel<G, DYN, SOFT, XT, OT, KP>), dim3(grid), dim3(G::THREADS), 0, stream, p);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (p.n_tiles <= kDirectTiles) {
+    // few tiles: one kernel merges them and writes the gradient
+    hipLaunchKernelGGL((ttt_finalize<KP, 16>), dim3(p.n_lb), dim3(64 * KP), 0, stream, p.partials, grad, p.n_tiles, p.n_lbd,
+                       p.D, p.hd, p.H, p.K);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((ttt_merge_chunks<KP>), dim3(n_chunks, p.n_lb), dim3(64 * KP), 0, stream, p.partials, chunks,
                      p.n_tiles, n_chunks);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((ttt_finalize<KP>), dim3(p.n_lb), dim3(64 * KP), 0, stream, chunks, grad, n_chunks, p.n_lbd,
+  hipLaunchKernelGGL((ttt_finalize<KP, 8>), dim3(p.n_lb), dim3(64 * KP), 0, stream, chunks, grad, n_chunks, p.n_lbd,
                      p.D, p.hd, p.H, p.K);
   return hipGetLastError();
 }

@@ -40,6 +40,9 @@ def assert_grad(got, want, rtol=GRAD_RTOL):
     (2, 193, 2, 64, 4, False, "x"),           # one token into the second (192-token) tile
     (1, 64 * 128 + 33, 1, 64, 8, False, "x"),  # crosses a look-back checkpoint
     (3, 5000, 2, 16, 8, True, "softsign"),
+    (1, 32 * 192, 2, 32, 8, False, "x"),       # 32 tiles: merged by one kernel
+    (1, 32 * 192 + 1, 2, 32, 4, True, "x"),    # 33: by chunks first
+    (40, 104 * 192 - 5, 1, 6, 8, False, "x"),  # 4160 tiles in the launch: the coefficient table of its own kernel
 ])
 def test_ttt_shapes(dev, B, S, H, hd, K, dyn, target):
     inp = inputs(B, S, H, hd, K, seed=S + 7 * B, dynamic=dyn)

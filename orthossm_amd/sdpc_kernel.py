@@ -158,6 +158,8 @@ def _fast_constants(n_heads: int, device: torch.device, ema_momentum):
     with _const_lock:
         damping = _const_cache.get(dkey)
         lam = _const_cache.get(lkey) if lkey is not None else None
+    if damping is not None and lam is not None:
+        return damping, lam
     if damping is None:
         damping = v10_damping(n_heads, dev)
     if lam is None:

@@ -133,7 +133,8 @@ int check_args(const osm_cheby_args* a, Geometry* geo, int op, bool shapes_only 
         a->c_stride_k < 0 || a->c_stride_b < 0)
       return fail(OSM_E_LAYOUT, "coeffs strides must be non-negative and fit 31-bit offsets");
   }
-  osm::FwdShape shape{osm::ttt_tile_tokens(geo->dyn, a->x_dtype), osm::TttTile::LANES, 1};
+  osm::FwdShape shape{osm::ttt_tile_tokens(a->B * ((D + osm::TttTile::LANES - 1) / osm::TttTile::LANES), a->S),
+                      osm::TttTile::LANES, 1};
   if (op == OSM_OP_FWD) shape = osm::fwd_geometry(geo->dyn, a->B, D, a->S, generic);
   if (op == OSM_OP_BWD) shape = osm::FwdShape{osm::bwd_tile_tokens(geo->dyn, geo->kpad), osm::BwdTile::LANES, 1};
   const int64_t tile = shape.tile;

@@ -94,7 +94,14 @@ FwdShape fwd_geometry(bool dyn, int64_t B, int64_t D, int64_t S, bool generic);
 // (at 16-token runs 1147 us with two words against 1254 with eight and 1177
 // with four; at 20-token runs one word 1069 against 1086 with two).
 using TttTile = TileGeo<1, 8, 24, 64, 1>;   // 192 tokens
-int ttt_tile_tokens(bool dyn, int x_dtype);
+// 128-token tiles where the 192-token ones would leave CUs idle and one kernel
+// still merges them (kDirectTiles): a tile's VALU work is then a launch's
+// latency.  Measured on MI355X, 192 against 128 tokens: 15.0 and 12.3 us at B=1
+// S=256 D=512 (16 tiles of 192), 18.1 and 15.1 at B=2 S=2048 (176), 20.0 and
+// 21.4 at B=1 S=6000 (47 tiles of 128 a lane-block).  (96 tokens: 11.5, 16.7.)
+using TttTileSmall = TileGeo<1, 8, 16, 64, 1>;   // 128 tokens
+constexpr int kDirectTiles = 32;                 // tiles of a lane-block merged by one kernel (osm_ttt.hip)
+int ttt_tile_tokens(int64_t n_lb, int64_t S);
 
 // Backward: one lane per thread (the clamp mask makes the adjoint map's A
 // differ per lane); x and dL/dout of the run stay in registers between the

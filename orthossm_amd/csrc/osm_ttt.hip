@@ -27,11 +27,11 @@ namespace osm {
 namespace {
 
 constexpr int kChunk = 16;  // tiles merged per thread by the first merge kernel
-// Up to this many tiles one kernel merges a lane's tiles and writes the
+// Up to kDirectTiles tiles one kernel merges a lane's tiles and writes the
 // gradient; past it the merge by chunks runs in parallel first.  Measured on
-// MI355X: 20.1 against 21.5 us at B=1 S=1000 (6 tiles), 25.0 and 27.7 at S=12000
-// with chunks (63 tiles), 34.5 and 38.3 at 105 tiles.
-constexpr int kDirectTiles = 32;
+// MI355X: 18.7 against 21.3 us at B=1 S=1000 (6 tiles); with 105 tiles 38.3
+// against 34.5 by chunks.
+//
 // Up to this many tiles in the launch each tile converts its coefficients, as
 // the forward's do; past it (1-3% of a large launch) ttt_mono_prep converts
 // them once: 15.0 against 17.8 us at B=1 S=256 D=512, 57.9 against 59.7 at B=16
@@ -700,8 +700,9 @@ hipError_t launch_k(const FwdParams& p, float* grad, int kpad, hipStream_t strea
 // Geometry; must agree with ttt_tile_tokens.
 template <bool DYN, typename XT, typename OT>
 hipError_t launch_geo(const FwdParams& p, float* grad, int tile, int kpad, hipStream_t stream) {
-  if (tile != TttTile::TILE) return hipErrorInvalidValue;
-  return launch_k<TttTile, DYN, XT, OT>(p, grad, kpad, stream);
+  if (tile == TttTile::TILE) return launch_k<TttTile, DYN, XT, OT>(p, grad, kpad, stream);
+  if (tile == TttTileSmall::TILE) return launch_k<TttTileSmall, DYN, XT, OT>(p, grad, kpad, stream);
+  return hipErrorInvalidValue;
 }
 
 template <bool DYN>
@@ -715,7 +716,11 @@ hipError_t launch_dt(const FwdParams& p, float* grad, int x_dtype, int out_dtype
 
 }  // namespace
 
-int ttt_tile_tokens(bool, int) { return TttTile::TILE; }
+int ttt_tile_tokens(int64_t n_lb, int64_t S) {
+  constexpr int64_t kCus = 256;
+  const int64_t n_tiles = (S + TttTile::TILE - 1) / TttTile::TILE;
+  return S <= kDirectTiles * TttTileSmall::TILE && n_lb * n_tiles < kCus ? TttTileSmall::TILE : TttTile::TILE;
+}
 
 size_t ttt_workspace_bytes(int n_lb, int n_tiles, bool dyn, int K) {
   const int kpad = K <= 4 ? 4 : 8;

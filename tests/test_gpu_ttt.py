@@ -37,7 +37,10 @@ def assert_grad(got, want, rtol=GRAD_RTOL):
     (2, 1000, 8, 64, 8, True, "x"),
     (2, 777, 4, 32, 5, False, "softsign"),
     (1, 300, 3, 20, 8, True, "x"),            # partial lane-block
-    (2, 193, 2, 64, 4, False, "x"),           # one token into the second (192-token) tile
+    (2, 193, 2, 64, 4, False, "x"),           # a partial second tile of 128 tokens
+    (1, 129, 2, 64, 8, True, "softsign"),     # one token into it
+    (1, 4096, 2, 16, 8, False, "x"),          # 32 tiles of 128
+    (1, 4097, 2, 16, 8, False, "softsign"),   # one token more: 192-token tiles
     (1, 64 * 128 + 33, 1, 64, 8, False, "x"),  # crosses a look-back checkpoint
     (3, 5000, 2, 16, 8, True, "softsign"),
     (1, 32 * 192, 2, 32, 8, False, "x"),       # 32 tiles: merged by one kernel

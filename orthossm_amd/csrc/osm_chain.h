@@ -237,29 +237,37 @@ __device__ __forceinline__ void look_back_issue(LookBack<G, DYN>& st, const Thre
 // (unused when DYN); `init_carry` the initial state of carry_lane (waves <
 // NSUB); `limit` the poll limit of await_word.  A wait that gives up yields
 // NaN, so the carry (and a checkpoint published from it) is NaN.
-template <class G, bool DYN>
+// AL: the type in which a thread's words compose; double where a launch may
+// choose several per thread (rounded once; in fp32 the longer composition
+// raised the error of a long carry chain by half).
+template <class G, bool DYN, typename AL>
 __device__ __forceinline__ void look_back_finish(LookBack<G, DYN>& st, ChainLds<G>& L, const ThreadPos& q,
                                                  const TileInfo& ti, const Tags& tg, float aggA, float aggB,
-                                                 const LaneSlots& ls, float init_carry, float a_look,
-                                                 unsigned* hdr_words, unsigned limit) {
+                                                 const LaneSlots& ls, float init_carry, AL a_look,
+                                                 unsigned* hdr_words, unsigned limit, float min_a = 0.0f) {
   if (ti.tile > 0) {
     const int ll = look_lane<G>(q);
-    float mA = 1.0f, mB = 0.0f;
+    AL mA = 1, mB = 0;
     if (st.beg < st.end) {
-      const float Afull = DYN ? 1.0f : a_look;
+      const AL Afull = DYN ? AL(1) : a_look;
 #pragma unroll
       for (int i = 0; i < G::WPT; ++i) {
         if (st.beg + i >= st.end) break;
         const unsigned long long* s = ls.at(st.beg + i, ll);
         const float Bp = await_word(s, st.vB[i], tg.agg, hdr_words, limit);
-        float Ap = Afull;
+        AL Ap = Afull;
         if constexpr (DYN) Ap = await_word(s + 1, st.vA[i], tg.agg, hdr_words, limit);
-        mB = __builtin_fmaf(Ap, mB, Bp);
+        if constexpr (std::is_same_v<AL, double>)
+          mB = __builtin_fma(Ap, mB, (double)Bp);
+        else
+          mB = __builtin_fmaf(Ap, mB, Bp);
         mA *= Ap;
       }
     }
-    L.mA[q.wave][q.wl] = mA;
-    L.mB[q.wave][q.wl] = mB;
+    // min_a > 0: a composed decay does not underflow to 0 (an infinite state
+    // stays infinite)
+    L.mA[q.wave][q.wl] = min_a > 0.0f ? __builtin_fmaxf((float)mA, min_a) : (float)mA;
+    L.mB[q.wave][q.wl] = (float)mB;
     float ck = init_carry;
     if (q.wave < G::NSUB && st.g0 > 0)
       ck = await_word(ls.at(st.g0 - 1, carry_lane<G>(q)), st.vck, tg.pre, hdr_words, limit);

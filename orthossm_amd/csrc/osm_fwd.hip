@@ -289,7 +289,9 @@ cheby_ema_fwd_kernel(const FwdParams p) {
     if constexpr (!DYN)
       if (q.wave < G::NSUB) aggA = static_tile_A<G>(p.lam[dc < p.D ? div_hd(dc, p) : 0]);
     const int dlk = ti.lbd * G::LANES + look_lane<G>(q);
-    const float a_look = DYN ? 0.0f : static_tile_A<G>(p.lam[dlk < p.D ? div_hd(dlk, p) : 0]);
+    using AL = std::conditional_t<kVarWords, double, float>;
+    AL a_look = 0;
+    if constexpr (!DYN) a_look = (AL)pow_n_f64<G::TILE>((double)p.lam[dlk < p.D ? div_hd(dlk, p) : 0]);
     LookBack<G, DYN> lbk;
     look_back_issue<G, DYN>(lbk, q, ti, ls, wsh);
     jitter(p.jitter, tags.epoch, 1);
@@ -336,9 +338,8 @@ hipError_t launch_g(const FwdParams& p, int kpad, hipStream_t stream) {
 
 // The one-lane geometry also serves the Chebyshev form (kpad 16 and 32);
 // K <= 4 runs with kpad 8 there (zero coefficients), one instantiation fewer.
-template <bool DYN, typename XT, typename OT>
+template <class G, bool DYN, typename XT, typename OT>
 hipError_t launch_generic(const FwdParams& p, int kpad, hipStream_t stream) {
-  using G = FwdTileGeneric;
   const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
   if (kpad <= 8)
     hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 8>), dim3(grid), dim3(G::THREADS), 0, stream, p);
@@ -358,7 +359,9 @@ bool is_shape(FwdShape s) {
 
 template <bool DYN, typename XT, typename OT>
 hipError_t launch_k(const FwdParams& p, FwdShape s, int kpad, hipStream_t stream) {
-  if (is_shape<FwdTileGeneric>(s)) return launch_generic<DYN, XT, OT>(p, kpad, stream);
+  if (is_shape<FwdTileGeneric>(s))
+    return p.wsh > 0 ? launch_generic<FwdTileGenericFew, DYN, XT, OT>(p, kpad, stream)
+                     : launch_generic<FwdTileGeneric, DYN, XT, OT>(p, kpad, stream);
   if constexpr (!DYN) {
     if (is_shape<FwdTileLarge>(s)) return launch_g<FwdTileLarge, DYN, XT, OT>(p, kpad, stream);
   } else {

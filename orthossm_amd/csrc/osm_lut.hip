@@ -167,11 +167,13 @@ lut_fwd_kernel(const LutScanParams p) {
     const int dc = ti.lbd * kLanes + carry_lane<G>(q);
     const float init_c =
         p.ema_init && q.wave == 0 && dc < p.D ? p.ema_init[(int64_t)ti.b * p.init_sb + dc] : 0.0f;
-    const float tile_A = __builtin_fmaxf(static_tile_A<G>(mu), kTinyDecay);
+    const double tile_A64 = __builtin_fmax(pow_n_f64<G::TILE>((double)mu), (double)kTinyDecay);
+    const float tile_A = (float)tile_A64;
     LookBack<G, false> lbk;
     look_back_issue<G, false>(lbk, q, ti, ls, p.wsh, ti.tile > p.clamp_at ? p.clamp_at + 1 : 0);
     ti.is_ckpt = ckpt && !at_clamp;   // the clamped tile's state is published below
-    look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A, p.hdr, p.poll_limit);
+    look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A64, p.hdr, p.poll_limit,
+                               kTinyDecay);
   }
   finish_complete(p.hdr, tags.epoch, fin_prev);
   if (at_clamp && !ti.is_last && q.wave == 0) {

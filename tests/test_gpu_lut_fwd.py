@@ -99,6 +99,7 @@ class _WalkOnly:
     (1, 1300, 2, 32, 8, True, 1024, 0.9999, ""),      # the clamp in tile 15, past a checkpoint group
     (1, 700, 2, 32, 6, False, 2048, 0.99, ""),        # no clamp inside the sequence
     (1, 2500, 2, 32, 8, True, 1008, 0.9995, ""),      # 40 tiles of one lane-block: groups of 32, the clamp inside one
+    (1, 2500, 1, 8, 4, True, 2048, 0.25, ""),         # infinite states through decays far below fp32's smallest
     (2, 4200, 1, 40, 4, True, 2064, 0.9999, ""),      # the clamp in the first tile of the second group of 32
     (9, 4100, 2, 64, 8, True, 128, 1.0, ""),          # 128-token tiles; a decay of one
     (3, 500, 2, 40, 8, True, 144, 0.95, "strided"),   # x and out views of wider rows

@@ -534,18 +534,7 @@ PyObject* run_lut(PyObject* const* p) {
   a.ema_final = fptr(fin);
   a.final_stride_b = fin.stride(0);
   const size_t need = lib.lut_bytes(&a);
-  if (need) {
-    // A workspace that is not there yet is the Python path's to make (it
-    // makes none inside a stream capture).
-    PyObject* key = Py_BuildValue("(iOi)", (int)x.get_device(), s_obj.o, kOpLut);
-    PyObject* hit = key ? PyDict_GetItemWithError(ws_cache, key) : nullptr;
-    Py_XDECREF(key);
-    if (!hit || !THPVariable_Check(hit) || (size_t)THPVariable_Unpack(hit).numel() < need) {
-      if (PyErr_Occurred()) return nullptr;
-      Py_RETURN_NONE;
-    }
-    ws = THPVariable_Unpack(hit);
-  }
+  if (need && !get_workspace(p[0], x, s_obj.o, need, kOpLut, &ws)) return nullptr;
   int rc;
   {
     const NoGil nogil;

@@ -179,12 +179,6 @@ def _workspace(device: torch.device, stream: int, nbytes: int, op: int) -> torch
         return ws
 
 
-def _has_workspace(device: torch.device, stream: int, nbytes: int, op: int) -> bool:
-    with _ws_lock:
-        ws = _ws_cache.get((device.index, stream, op))
-        return ws is not None and ws.numel() >= nbytes
-
-
 def _as_param(v, H: int, device, name: str) -> torch.Tensor:
     if (isinstance(v, torch.Tensor) and v.dtype is torch.float32 and v.dim() == 1 and v.is_contiguous()
             and v.device == device):
@@ -703,7 +697,8 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     if x.device.type != "cuda":
         raise RuntimeError("orthossm_amd runs on a ROCm GPU only; x is on " + str(x.device))
     dev = x.device
-    fast = _fast()
+    capturing = torch.cuda.is_current_stream_capturing()
+    fast = None if capturing else _fast()
     if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and ema_final is None:
         table = v10_tables(dev, n_heads, LUT_TERMS)[0] if use_lut else None
         res = fast.lut_forward(x, coeffs, n_heads, ema_momentum, ema_init, use_lut, table, clamp_tile, want_x_norm,
@@ -761,9 +756,10 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
         a.tanh_y, a.ty_stride_b, a.ty_stride_s = tanh_y.data_ptr(), tanh_y.stride(0), tanh_y.stride(1)
     a.ema_final, a.final_stride_b = ema_final.data_ptr(), ema_final.stride(0)
     stream = _current_stream(dev)
-    nbytes = lib.osm_lut_fwd_workspace_bytes(ctypes.byref(a))
-    if nbytes and not _has_workspace(dev, stream, nbytes, nat.OP_LUT) and torch.cuda.is_current_stream_capturing():
-        nbytes = 0   # no allocation inside a capture: the walk needs none
+    # A graph would keep the address of a workspace that a later, larger call
+    # replaces, and share it with eager calls: a capture takes the walk over
+    # the tiles, which needs none.
+    nbytes = 0 if capturing else lib.osm_lut_fwd_workspace_bytes(ctypes.byref(a))
     if nbytes:
         ws = _workspace(dev, stream, nbytes, nat.OP_LUT)
         nat.check(lib.osm_cheby_ema_lut_fwd_ws(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(),

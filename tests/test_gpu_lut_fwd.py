@@ -143,7 +143,7 @@ def test_scan_and_walk_agree_around_the_first_clamp(dev, monkeypatch, B, S, H, h
 
 
 def test_capture_without_a_workspace(dev):
-    # a capture on a stream that has made no call yet: nothing is allocated
+    # a capture on a stream that has made no call yet
     x, c, init = (t.to(dev) for t in case(2, 700, 2, 32, 8, seed=3, init_scale=0.5))
     want = cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
     torch.cuda.synchronize()
@@ -158,6 +158,31 @@ def test_capture_without_a_workspace(dev):
         for g, w in zip(got, want):
             assert rel(g, w.double().cpu().numpy()) <= 1e-6
         cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
+
+
+def test_capture_outlives_the_workspace_of_its_stream(dev):
+    # the stream's workspace is there before the capture and is replaced by a
+    # larger eager call after it; the old one's memory is then given new contents
+    x, c, init = (t.to(dev) for t in case(2, 700, 2, 32, 8, seed=3, init_scale=0.5))
+    big, cbig, _ = (t if t is None else t.to(dev) for t in case(8, 8192, 8, 128, 8, seed=4))
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        want = cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            got = cheby_ema_lut_forward(x, c, n_heads=2, ema_init=init)
+        for _ in range(3):
+            cheby_ema_lut_forward(big, cbig, n_heads=8)
+            filled = torch.full((1 << 18,), 3.0, device=dev)
+            for t in got:
+                t.fill_(float("nan"))
+            graph.replay()
+            stream.synchronize()
+            assert (filled == 3.0).all()
+            for g, w in zip(got, want):
+                assert rel(g, w.double().cpu().numpy()) <= 1e-6
 
 
 def test_special_values_empty_and_optional_outputs(dev):

@@ -133,6 +133,17 @@ bool as_float(PyObject* o, float* v) {
   return true;
 }
 
+// An integer; false for what int() would have to convert (a float, say), which
+// the Python path then does or refuses.
+bool as_int(PyObject* o, int64_t* v) {
+  *v = PyLong_AsLongLong(o);
+  if (*v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    return false;
+  }
+  return true;
+}
+
 struct Common {
   const at::Tensor *x, *coeffs, *damping, *lam, *g = nullptr;
   osm_cheby_args a{};
@@ -223,6 +234,7 @@ PyObject* run_forward(PyObject* const* p, bool ttt) {
   const int dt = p[10] == Py_None ? code(x) : (int)PyLong_AsLong(p[10]);
   if (!out_rows(p[11], dt, &c, &out)) Py_RETURN_NONE;
   const bool want_state = PyObject_IsTrue(p[12]) == 1;
+  if (PyErr_Occurred()) return nullptr;
   if (p[13] != Py_None) {
     const at::Tensor* t = plain(p[13]);
     if (!t || t->dim() != 2 || t->size(0) != c.B || t->size(1) != D || !f32_flat(*t, c.B * D, x)) Py_RETURN_NONE;
@@ -279,6 +291,7 @@ PyObject* run_backward(PyObject* const* p) {
     b.grad_state = fptr(*t);
   }
   const bool need_c = PyObject_IsTrue(p[12]) == 1, need_i = PyObject_IsTrue(p[13]) == 1;
+  if (PyErr_Occurred()) return nullptr;
   c.a.out_dtype = code(*out);
   set_out(&c, *out);
   b.grad_out = go->data_ptr();
@@ -352,7 +365,7 @@ PyObject* run_v10(PyObject* const* p) {
   if (!xp || !xp->is_cuda() || !(is_f32(*xp) || is_bf16(*xp)) || !rows(*xp, *xp) || xp->size(1) == 0) Py_RETURN_NONE;
   const at::Tensor& x = *xp;
   osm_v10_args a{};
-  a.H = PyLong_AsLongLong(p[3]);
+  if (!as_int(p[3], &a.H) || !as_int(p[15], &a.chunk) || a.chunk < 1) Py_RETURN_NONE;
   if (!head_rows(cp, x, a.H) || !head_rows(mp, x, a.H) || mp->sizes() != cp->sizes() || cp->size(2) > 8) Py_RETURN_NONE;
   if (!batch_vec(p[4], x, &a.gate) || !batch_vec(p[5], x, &a.dyn_lambda)) Py_RETURN_NONE;
   if (!momentum(p[6], x, &a.ema_momentum, &a.ema_momentum_dev)) Py_RETURN_NONE;
@@ -363,10 +376,8 @@ PyObject* run_v10(PyObject* const* p) {
   for (int i = 0; i < 4; ++i) *tables[i] = fptr(THPVariable_Unpack(p[7 + i]));   // the module's own tables
   a.abi_version = OSM_ABI_VERSION;
   a.flags = PyObject_IsTrue(p[16]) == 1 ? OSM_V10_USE_LUT : 0;
-  a.chunk = PyLong_AsLongLong(p[15]);
-  if (PyErr_Occurred()) return nullptr;
-  if (a.chunk < 1) Py_RETURN_NONE;
   const bool save = PyObject_IsTrue(p[17]) == 1;
+  if (PyErr_Occurred()) return nullptr;
   a.B = x.size(0);
   a.S = x.size(1);
   a.hd = cp->size(3);
@@ -429,9 +440,7 @@ PyObject* run_v10_backward(PyObject* const* p) {
     if (!rows(*r, x) || r->stride(1) > kMost) Py_RETURN_NONE;
   if (hist.dim() != 5 || !is_f32(hist) || hist.device() != x.device() || !hist.is_contiguous()) Py_RETURN_NONE;
   osm_v10_bwd_args a{};
-  if (!momentum(p[5], x, &a.ema_momentum, &a.ema_momentum_dev)) Py_RETURN_NONE;
-  a.chunk = PyLong_AsLongLong(p[6]);
-  if (PyErr_Occurred()) return nullptr;
+  if (!momentum(p[5], x, &a.ema_momentum, &a.ema_momentum_dev) || !as_int(p[6], &a.chunk)) Py_RETURN_NONE;
   a.abi_version = OSM_ABI_VERSION;
   a.x_dtype = code(x);
   a.B = x.size(0);
@@ -478,7 +487,7 @@ PyObject* run_lut(PyObject* const* p) {
   if (!xp || !xp->is_cuda() || !(is_f32(*xp) || is_bf16(*xp)) || !rows(*xp, *xp)) Py_RETURN_NONE;
   const at::Tensor& x = *xp;
   osm_lut_fwd_args a{};
-  a.H = PyLong_AsLongLong(p[2]);
+  if (!as_int(p[2], &a.H) || !as_int(p[7], &a.clamp_tile)) Py_RETURN_NONE;
   if (!head_rows(cp, x, a.H) || cp->size(2) < 1 || cp->size(2) > 8 || !as_float(p[3], &a.ema_momentum)) Py_RETURN_NONE;
   a.B = x.size(0);
   a.S = x.size(1);
@@ -493,9 +502,8 @@ PyObject* run_lut(PyObject* const* p) {
   }
   const bool use_lut = PyObject_IsTrue(p[5]) == 1;
   if (use_lut) a.lut = fptr(THPVariable_Unpack(p[6]));   // the module's own table
-  a.clamp_tile = PyLong_AsLongLong(p[7]);
-  if (PyErr_Occurred()) return nullptr;
   const bool want_n = PyObject_IsTrue(p[8]) == 1, want_y = PyObject_IsTrue(p[9]) == 1;
+  if (PyErr_Occurred()) return nullptr;
   a.abi_version = OSM_ABI_VERSION;
   a.flags = use_lut ? OSM_V10_USE_LUT : 0;
   a.x = x.data_ptr();

@@ -561,7 +561,7 @@ def v10_chunked_ttt(x: torch.Tensor, coeffs: torch.Tensor, momentum: torch.Tenso
     lib = nat.load()
     fast = _fast()
     if fast is not None and isinstance(x, torch.Tensor) and x.is_cuda and isinstance(coeffs, torch.Tensor) and \
-            coeffs.dim() == 4:
+            coeffs.dim() == 4 and coeffs.shape[1] == n_heads:
         lut, lion_lambda, ss, lr_scale = v10_tables(x.device, n_heads, min(coeffs.shape[2], nat.MAX_K_V10))
         res = fast.v10(x, coeffs, momentum, n_heads, gate_global, dynamic_lambda, ema_momentum, lut, lion_lambda, ss,
                        lr_scale, base_lr, beta1, beta2, weight_decay, chunk_size, use_lut, save_for_backward)
@@ -699,7 +699,8 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     dev = x.device
     capturing = torch.cuda.is_current_stream_capturing()
     fast = None if capturing else _fast()
-    if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and ema_final is None:
+    if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and \
+            ema_final is None and coeffs.dim() == 4 and coeffs.shape[1] == n_heads:
         table = v10_tables(dev, n_heads, LUT_TERMS)[0] if use_lut else None
         res = fast.lut_forward(x, coeffs, n_heads, ema_momentum, ema_init, use_lut, table, clamp_tile, want_x_norm,
                                want_tanh_y)

@@ -12,7 +12,7 @@ import torch
 from oracle import v10_full as V
 from orthossm_amd import _native as nat
 from orthossm_amd import apply_cheby_rkv_v10
-from orthossm_amd.ops import cheby_ema_lut_forward
+from orthossm_amd.ops import cheby_ema_lut_forward, v10_chunked_ttt
 from orthossm_amd.sdpc_kernel import LUT_TABLE_SIZE, _fused_clenshaw_ema_kernel, get_chebyshev_lut
 
 pytestmark = pytest.mark.gpu
@@ -183,6 +183,22 @@ def test_capture_outlives_the_workspace_of_its_stream(dev):
             assert (filled == 3.0).all()
             for g, w in zip(got, want):
                 assert rel(g, w.double().cpu().numpy()) <= 1e-6
+
+
+def test_whole_numbers_as_floats_are_taken_and_wrong_head_counts_refused(dev):
+    x, c, init = (t.to(dev) for t in case(2, 300, 4, 16, 8, seed=9, init_scale=0.5))
+    want = cheby_ema_lut_forward(x, c, n_heads=4, ema_init=init, clamp_tile=128)
+    for g, w in zip(cheby_ema_lut_forward(x, c, n_heads=4, ema_init=init, clamp_tile=128.0), want):
+        assert torch.equal(g, w)
+    m = torch.zeros_like(c)
+    want = v10_chunked_ttt(x, 0.1 * c, m, n_heads=4, chunk_size=64)
+    for g, w in zip(v10_chunked_ttt(x, 0.1 * c, m, n_heads=4, chunk_size=64.0), want):
+        assert torch.equal(g, w)
+    for n in (-1, 0, 2):
+        with pytest.raises(ValueError):
+            cheby_ema_lut_forward(x, c, n_heads=n)
+        with pytest.raises(ValueError):
+            v10_chunked_ttt(x, c, m, n_heads=n)
 
 
 def test_special_values_empty_and_optional_outputs(dev):

@@ -167,7 +167,7 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
 
   // Highest wave priority while the tile's loads are issued (here and
   // before the x loads below), so that they enter the memory pipeline ahead
-  // of other workgroups' arithmetic (measured at BASELINE configs[1] on
+  // of other workgroups' arithmetic (measured at B=4 S=16384 D=512 on
   // MI355X: 121.8 against 124.0 us).
   __builtin_amdgcn_s_setprio(3);
   const ThreadPos q = thread_pos<G>();

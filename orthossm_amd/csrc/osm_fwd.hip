@@ -125,8 +125,8 @@ cheby_ema_fwd_kernel(const FwdParams p) {
 
   // Highest wave priority until the tile's loads are issued: a workgroup
   // that has just started gets its loads into the memory pipeline ahead of
-  // the arithmetic of older workgroups on the CU (measured at BASELINE
-  // configs[1] on MI355X: 52.0 against 53.5 us).
+  // the arithmetic of older workgroups on the CU (measured at B=4
+  // S=16384 D=512 on MI355X: 52.0 against 53.5 us).
   __builtin_amdgcn_s_setprio(3);
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);

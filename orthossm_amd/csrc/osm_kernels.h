@@ -45,7 +45,7 @@ struct TileGeo {
 // scan and look-back over more tokens but give fewer workgroups, so the host
 // takes the largest tile that still fills the chip (fwd_geometry).  Dynamic
 // lambda keeps a per-token lambda in registers and is limited to the medium
-// tile.  Measured on MI355X at BASELINE configs[1] against 128-lane tiles
+// tile.  Measured on MI355X at B=4 S=16384 D=512 against 128-lane tiles
 // with 2 or 4 lanes per thread (256 and 128 tokens) and 64-lane tiles with 4
 // lanes per thread: the 64-lane, 2-lane, 512-token tile is fastest.
 // The medium, small and one-lane tiles read one or kFwdWords look-back words
@@ -85,7 +85,7 @@ FwdShape fwd_geometry(bool dyn, int64_t B, int64_t D, int64_t S, bool generic);
 // TTT: keeps the raw x and w = (1-lam)(1-2r) (r = 1/(1+exp(2 damping p)))
 // of every token of the run in registers, u = softsign(x) in LDS, plus 2K
 // gradient accumulators per lane: one lane per thread (half the
-// accumulators of two).  Measured on MI355X at BASELINE configs[4] (bf16),
+// accumulators of two).  Measured on MI355X at B=16 S=65536 D=512 (bf16),
 // with u in LDS: 24-token runs 1001-1008 us against 1047-1056 with 20, 1025
 // with 28 and 1092-1095 with 16 (longer runs amortise the per-thread setup,
 // chain, composition and reduction over more tokens; at the 128-VGPR bound
@@ -112,7 +112,7 @@ int ttt_tile_tokens(int64_t n_lb, int64_t S);
 // reads two words (A, B) per predecessor.  Four look-back words per thread
 // (checkpoints every 32 tiles) instead of eight brought the static kernel from
 // 101 to 77 VGPRs, three workgroups per CU instead of two: 129 against 141 us
-// at BASELINE configs[1] on MI355X; two words (checkpoints every 16 tiles)
+// at B=4 S=16384 D=512 on MI355X; two words (checkpoints every 16 tiles)
 // 116.9 against 118.2 us with four.  24-token runs (94 VGPRs, two
 // workgroups per CU) 113.8-114.4 against 116.5-116.8 us for 16 tokens; 20
 // tokens 114.3, 28 tokens 118.2, 32 tokens 114.2; 8-token runs are slower

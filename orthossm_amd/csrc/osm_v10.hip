@@ -331,8 +331,8 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
   // Token 0 of every run is prepared ahead of its block, so that its table
   // reads are off the chunk's chain: for a chunk's first block by the first
   // wave of each SIMD while it waits for the second at the reduction
-  // barrier, and by the others while wave 0 applies Lion.  Measured at the
-  // configs[1] shape, bit-identical: one token ahead, all waves during
+  // barrier, and by the others while wave 0 applies Lion.  Measured at
+  // B=4 S=16384 D=512, bit-identical: one token ahead, all waves during
   // Lion, 152.6-153.7 against 153.9-155.0 us; two and three tokens ahead
   // 162.6 and 170.2 us (their reads outgrow the window); the first waves
   // before the barrier 150.4-150.6 against 151.1-151.6 us.
@@ -342,7 +342,7 @@ __global__ void __launch_bounds__(kV10Groups * LW) v10_chunked_kernel(const P p)
   // path with the loop's back edge, waits for the next block's prefetched
   // rows at the start of every block (vmcnt 4..1 before each row's use),
   // which exposes a full memory latency per chunk (283 against 299 us at
-  // the configs[1] shape).  s_waitcnt vmcnt(0) expcnt(7) lgkmcnt(15).
+  // B=4 S=16384 D=512).  s_waitcnt vmcnt(0) expcnt(7) lgkmcnt(15).
   __builtin_amdgcn_s_waitcnt(0xF70);
   if (!FIXED || n_chunks > 0) prep(xcur[0], f0, true);
 

@@ -1,4 +1,4 @@
-"""Synthetic workloads of the BASELINE configurations.
+"""Synthetic workloads of the headline configurations.
 
 One CPU ``torch.Generator`` seeded with ``seed`` draws, in this order:
 x ~ N(0,1) [B,S,D]; c[b,h,k,j] = N(0,1)/(k+1) [B,H,K,hd]; and, for the
@@ -34,16 +34,16 @@ class Config:
         return self.D // self.H
 
 
-# BASELINE.json configs[0..4]
+# the headline configurations
 CONFIGS = {
     "cpu_ref": Config("cpu_ref", B=1, S=2048, D=512, H=8),
     "headline": Config("headline", B=4, S=16384, D=512, H=8),
     "streaming": Config("streaming", B=1, S=262144, D=512, H=8, chunk=16384),
     "dynamic": Config("dynamic", B=8, S=32768, D=1024, H=8, dynamic=True),
     "bf16_ttt": Config("bf16_ttt", B=16, S=65536, D=512, H=8, dtype=torch.bfloat16, ttt=True),
-    # the backward of configs[1]
+    # the backward of the headline shape
     "backward": Config("backward", B=4, S=16384, D=512, H=8, bwd=True),
-    # the reference's full apply_cheby_rkv_v10 path at the configs[1] shape
+    # the reference's full apply_cheby_rkv_v10 path at the headline shape
     "v10_full": Config("v10_full", B=4, S=16384, D=512, H=8, v10=256),
 }
 

@@ -48,8 +48,10 @@ struct Rows {
   uint32_t v, s;   // this thread's byte offset, bytes per token
 };
 
-// Rows t_blk .. t_end - 1 of a [B,S,D] tensor: reads past t_end give 0 and
-// stores past it are dropped, so the tokens of the next chunk stay out.
+// Rows t_blk .. t_end - 1 of a [B,S,D] tensor: stores past t_end are dropped
+// and nothing past the last row is read.  A read of a token past t_end gives 0
+// where rows lie D or more apart; rows that share memory (dL/dout of a sum
+// over tokens has stride 0) give values of earlier tokens there.
 template <class G, typename T>
 __device__ __forceinline__ Rows chunk_rows(const void* base, int64_t sb, int64_t ss, int b, int t_blk, int t_end,
                                            int D, int tg, int d0) {
@@ -195,6 +197,15 @@ v10_bwd_kernel(const V10BwdParams p) {
         const bool over = __ballot(!(__builtin_fabs(acc * (double)(kTwoLog2e * gamma)) <= kMonoBound)) != 0;
         if (cl == 0) big[cj] = over ? 1u : 0u;
         sdm[cj][cl] = (float)((double)cj * acc * (double)gamma * (double)(1.0f - mu));
+      }
+      // The adjoint is 0 past the chunk's end: where rows of dL/dout share
+      // memory, tokens there have read another's row.
+      if (p.go_ss < p.D) {
+        const int n_valid = t1 - (t_blk + tg * R);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int i = 0; i < LPT; ++i) gv[r][i] = r < n_valid ? gv[r][i] : 0.0f;
       }
       // Pass 1, last token first: the run's map.
 #pragma unroll

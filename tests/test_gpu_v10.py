@@ -207,6 +207,43 @@ def test_v10_backward_every_chunk(dev, B, S, H, hd, K, chunk, dt, layout):
     assert (err <= bound).all(), f"max error {err.max():.3e} of {np.abs(want).max():.3e}"
 
 
+@pytest.mark.parametrize("B,S,H,hd,chunk,step", [
+    (2, 300, 2, 32, 256, 0),     # a 44-token last chunk; every token the same row of dL/dout
+    (1, 401, 3, 5, 200, 0),      # one lane per thread; every chunk short of its block
+    (2, 650, 2, 32, 600, 0),     # chunks of three blocks, the last of 88 tokens; then 50 tokens
+    (2, 130, 2, 32, 60, 7),      # rows that overlap: token t starts 7 elements after token t-1
+])
+def test_v10_backward_of_rows_that_share_memory(dev, B, S, H, hd, chunk, step):
+    """dL/dout whose token stride is below D (the gradient of a sum over
+    tokens has stride 0): tokens past a chunk's end are in the same memory as
+    tokens before it and must not enter the chunk.  Bounds as above."""
+    D, n, K = H * hd, (S + chunk - 1) // chunk, 8
+    gen = torch.Generator().manual_seed(S + chunk)
+    x = torch.randn(B, S, D, generator=gen)
+    out = torch.randn(B, S, D, generator=gen) * 0.3
+    z = torch.tanh(torch.randn(B, S, D, generator=gen)).bfloat16()
+    hist = torch.randn(n, B, H, K, hd, generator=gen) / torch.arange(1, K + 1).view(K, 1)
+    buf = torch.randn(B, D + step * (S - 1), generator=gen)
+    go = buf.as_strided((B, S, D), (buf.shape[1], step, 1))
+    god = buf.to(dev).as_strided((B, S, D), (buf.shape[1], step, 1))
+    gx, _ = _v10_backward(x.to(dev), out.to(dev), z.to(dev), hist.to(dev), god, H, 0.9, chunk, False)
+    want, _ = V.v10_backward(x.numpy(), out.numpy(), z.float().numpy(), hist.numpy(), go.numpy(),
+                             n_heads=H, ema_momentum=float(np.float32(0.9)), chunk=chunk)
+    err = np.abs(gx.cpu().double().numpy() - want)
+    assert err.max() <= 1e-5 * np.abs(want).max(), f"max error {err.max():.3e} of {np.abs(want).max():.3e}"
+
+
+def test_v10_gradient_of_a_sum_over_tokens(dev):
+    x, c, m = (t.to(dev) for t in case(2, 600, 4, 16, 8, seed=31, mom_scale=0.01))
+    grads = []
+    for reduce_ in (lambda o: (o.sum(1) * w).sum(), lambda o: (o * w[:, None, :]).sum()):
+        w = torch.randn(2, 64, generator=torch.Generator().manual_seed(5)).to(dev)
+        xr = x.clone().requires_grad_(True)
+        reduce_(apply_cheby_rkv_v10(xr, c, m, n_heads=4, seq_threshold=0)[0]).backward()
+        grads.append(xr.grad)
+    assert torch.equal(*grads)
+
+
 def test_v10_single_chunk_grads_and_nan(dev):
     gx, gc, wx, wc = _grads_vs_oracle(dev, 2, 200, 4, 16, 8, 256, seed=77, nan=True)
     assert torch.isnan(gx[0, 5, 2])

@@ -246,6 +246,12 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
     }
     if constexpr (!DYN) A = pow_n<R>(lam_h);
   } else {
+    // dL/dout reads 0 past S only where its rows lie D or more apart; rows
+    // that share memory, as a sum over tokens gives, read earlier tokens.
+    if (tail && bp.go_ss < p.D) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) gv[r] = r < n_valid ? gv[r] : 0.0f;
+    }
     // Tokens >= S (last tile) are the identity; a zero mask cuts the chain.
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {

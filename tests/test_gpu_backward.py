@@ -63,6 +63,32 @@ def test_backward_shapes(dev, B, S, H, hd, K, dyn):
     check(inp, out, gx, gc, gi, go, gs, init)
 
 
+@pytest.mark.parametrize("B,S,H,hd,K,dyn,step", [
+    (2, 300, 2, 32, 8, False, 0),    # every token the same row, S off the 192-token tiles
+    (1, 193, 3, 20, 4, True, 0),     # one token past a tile, dynamic lambda
+    (2, 100, 2, 32, 12, False, 5),   # rows that overlap, the long-series kernel
+    (1, 1, 1, 8, 8, False, 0),
+])
+def test_backward_of_rows_that_share_memory(dev, B, S, H, hd, K, dyn, step):
+    """dL/dout with a token stride below D, as a sum over tokens gives it:
+    memory past the last token's row start belongs to earlier tokens."""
+    inp, _, gs, init = grads_case(B, S, H, hd, K, seed=S, dynamic=dyn)
+    D = H * hd
+    buf = torch.randn(B, D + step * (S - 1), generator=torch.Generator().manual_seed(S))
+    shape, strides = (B, S, D), (buf.shape[1], step, 1)
+    d = to_dev(inp, dev)
+    out = cheby_ema_forward(d["x"], d["coeffs"], d["damping"], d["lam"], g=d.get("g"),
+                            ema_init=torch.from_numpy(init).to(dev))
+    args = (d["x"], d["coeffs"], d["damping"], d["lam"], out, buf.to(dev).as_strided(shape, strides))
+    kw = dict(g=d.get("g"), grad_state=torch.from_numpy(gs).to(dev), need_init=True)
+    grads = cheby_ema_backward(*args, **kw)
+    check(inp, out, *grads, buf.as_strided(shape, strides).numpy(), gs, init)
+    # with a caller's buffer (the Python launch)
+    again = cheby_ema_backward(*args, grad_x_out=torch.empty_like(d["x"]), **kw)
+    for a, b in zip(grads, again):
+        assert torch.equal(a, b)
+
+
 def test_backward_without_state_gradient(dev):
     inp, go, _, _ = grads_case(2, 2000, 8, 64, 8, seed=5)
     out, gx, gc, gi = fwd_bwd(inp, dev, go)

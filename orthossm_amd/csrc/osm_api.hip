@@ -184,6 +184,7 @@ osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* w
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
+  p.order = osm::tile_order(geo.n_lb, geo.n_tiles);
   p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.lam_shift = a->lam_shift;
   p.lam_min = a->lam_min;
@@ -788,6 +789,7 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
+  p.order = osm::tile_order(geo.n_lb, geo.n_tiles);
   p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
   p.poll_limit = osm::kSpinLimit;

@@ -155,7 +155,7 @@ __device__ __forceinline__ void bwd_pass2(float& v, float (&Gk)[KP], const float
 }
 
 // Two workgroups (4 waves per SIMD) per CU: at most 128 VGPRs.
-template <class G, bool DYN, bool ZS, typename XT, typename OT, int KP>
+template <class G, bool DYN, bool ZS, typename XT, typename OT, int KP, bool SPREAD>
 __global__ void __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 cheby_ema_bwd_kernel(const BwdParams bp) {
   constexpr int R = G::R;
@@ -174,7 +174,11 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
   ThreadPos qc = q;
   qc.tg = G::NTG - 1 - q.tg;   // chain order: the tile's last run first
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);   // tile = chain index
+  const TileInfo ti = tile_info<G, SPREAD>(p.order, p.hdr, p.n_lb, p.n_lbd, p.n_tiles);   // tile = chain index
+  if (SPREAD && ti.pad) {
+    skip_block(p.hdr, tags, ti);
+    return;
+  }
   TileInfo tm = ti;
   tm.tile = p.n_tiles - 1 - ti.tile;   // tile in sequence order
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, tm);
@@ -358,7 +362,7 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
     for (int w = 0; w < G::WAVES; ++w) acc += sh_red[w][k][q.wl];
     part[(size_t)k * kLanes + q.wl] = acc;
   }
-  finish_block(p.hdr, tags.epoch);
+  finish_block<SPREAD>(p.hdr, tags.epoch);
 }
 
 // dL/dc[b,h,k,j] = 4 damping_h (1 - lam_h if static) * sum over the tiles of
@@ -395,8 +399,10 @@ __global__ void __launch_bounds__(kRedSlices * kLanes) bwd_reduce(const float* p
 template <class G, bool DYN, bool ZS, typename XT, typename OT, int KP>
 hipError_t launch_all(const BwdParams& bp, hipStream_t stream) {
   const FwdParams& p = bp.f;
-  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
-  hipLaunchKernelGGL((cheby_ema_bwd_kernel<G, DYN, ZS, XT, OT, KP>), dim3(grid), dim3(G::THREADS), 0, stream, bp);
+  with_order(p.order, [&](auto spread) {
+    hipLaunchKernelGGL((cheby_ema_bwd_kernel<G, DYN, ZS, XT, OT, KP, decltype(spread)::value>), dim3(p.order.grid),
+                       dim3(G::THREADS), 0, stream, bp);
+  });
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !bp.grad_coeffs) return e;
   hipLaunchKernelGGL((bwd_reduce<KP>), dim3(KP, p.n_lb), dim3(kRedSlices * kLanes), 0, stream, p.partials,

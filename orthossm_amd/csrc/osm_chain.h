@@ -18,17 +18,21 @@
 // CKPT = WPS * WPT (or, where a launch chooses, fewer words: WPS << wsh).
 // Look-back words are laid out [lane-block][tile][lane].
 //
-// Tile order.  Block v handles tile v / n_lb of the lane-block in slot v % n_lb
-// (tile_info maps slots to lane-blocks), so a tile waits only on blocks of
-// lower index.  Workgroups go to the 8 XCDs round-robin by index and in index
-// order within an XCD: the unfinished block of lowest index is always
-// resident or next in line on an XCD whose earlier blocks have all ended, and
-// what it waits on has ended, so the chain moves on whatever XCDs a lane-block's
-// tiles are on (the look-back words are agent-scope atomics, coherent over the
-// XCDs).  With n_lb a multiple of 8 every tile of a lane-block is on one XCD;
-// otherwise they rotate over all eight: pinning them left XCDs idle (4 of 8
-// at n_lb = 4).  The waits are bounded (kSpinLimit), so a broken
-// assumption surfaces as a fault flag, not a hang.
+// Tile order (tile_order, tile_info).  A tile waits on earlier tiles of its
+// lane-block, and blocks that wait may fill every place that another launch's
+// blocks need, on any XCD.  So an awaited block has to be running already
+// whenever the waiting one is:
+//   - by index over a multiple of 8 slots: workgroups go to the 8 XCDs
+//     round-robin by index and in index order within an XCD, and the tiles of
+//     a lane-block are on blocks of one residue mod 8, ascending: those
+//     awaited were dispatched to the same XCD before.
+//   - by ticket: a block draws its tile from its lane-block's counter when it
+//     starts, so those awaited have started, whatever XCD they are on.
+//   - with one tile nothing waits.
+// (By index over several XCDs holds for one launch alone; two of them could
+// wait for each other, each holding the XCD that the other needs.)  The waits
+// are bounded (kSpinLimit), so a broken assumption surfaces as a fault flag,
+// not a hang.
 #pragma once
 
 #include "osm_device.h"
@@ -46,8 +50,9 @@ struct ChainLds {
 };
 
 struct TileInfo {
-  int v, tile, lb, b, lbd;
+  int tile, lb, b, lbd;
   bool is_last, is_ckpt;
+  bool pad;   // no tile: a slot without a lane-block
 };
 
 struct Tags {
@@ -97,19 +102,32 @@ __device__ __forceinline__ Tags launch_tags(unsigned* hdr_words) {
 template <class G>
 constexpr int kWordsShift = G::WPT == 1 ? 0 : (G::WPT == 2 ? 1 : (G::WPT == 4 ? 2 : 3));
 
-// wsh: log2 of the look-back words per thread of this launch (at most
-// G::WPT words); checkpoints lie every WPS << wsh tiles.
-template <class G>
-__device__ __forceinline__ TileInfo tile_info(int v, int n_lb, int n_lbd, int n_tiles, int wsh = kWordsShift<G>) {
+// The block's tile.  wsh: log2 of the look-back words per thread of this
+// launch (at most G::WPT words); checkpoints lie every WPS << wsh tiles.
+template <class G, bool SPREAD>
+__device__ __forceinline__ TileInfo tile_info(const TileOrder& order, unsigned* hdr_words, int n_lb, int n_lbd,
+                                              int n_tiles, int wsh = kWordsShift<G>) {
   TileInfo ti;
-  ti.v = v;
-  ti.tile = v / n_lb;
-  // Slot s = v mod n_lb; the slots of one residue c = s mod 8 are on one XCD
-  // and serve consecutive lane-blocks, so the lane-blocks of a batch row share
-  // an L2 (they read the same lines of g, one value per head per token).
-  // With n_lb = 8 q + r, residues below r hold q + 1 lane-blocks.
-  const int s = v - ti.tile * n_lb, c = s & 7;
-  ti.lb = c * (n_lb >> 3) + min(c, n_lb & 7) + (s >> 3);
+  ti.pad = false;
+  if constexpr (!SPREAD) {
+    const int v = blockIdx.x;
+    ti.tile = v / n_lb;
+    ti.lb = slot_lane_block(v - ti.tile * n_lb, n_lb);
+  } else {
+    const TileSlot slot = spread_slot(order, blockIdx.x, n_lb, n_tiles);
+    ti.tile = slot.tile;
+    ti.lb = slot.lb;
+    if (ti.tile < 0 && ti.lb >= 0) {
+      __shared__ unsigned drawn;
+      if (threadIdx.x == 0)
+        drawn = __hip_atomic_fetch_add(&reinterpret_cast<WsHeader*>(hdr_words)->ticket[ti.lb & 7].next, 1u,
+                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      ti.tile = (int)__builtin_amdgcn_readfirstlane(drawn);
+    }
+    // (a drawn tile past the last: only where two launches share a workspace)
+    ti.pad = ti.lb < 0 || (unsigned)ti.tile >= (unsigned)n_tiles;
+  }
   ti.b = ti.lb / n_lbd;
   ti.lbd = ti.lb - ti.b * n_lbd;
   ti.is_last = ti.tile == n_tiles - 1;
@@ -309,6 +327,8 @@ __device__ __forceinline__ unsigned finish_issue(unsigned* hdr_words, unsigned e
   return prev;
 }
 
+// (SPREAD: and the ticket counters, from which every block has drawn.)
+template <bool SPREAD>
 __device__ __forceinline__ void finish_complete(unsigned* hdr_words, unsigned epoch, unsigned prev) {
   if (threadIdx.x == 0) {
     WsHeader* hdr = reinterpret_cast<WsHeader*>(hdr_words);
@@ -321,6 +341,11 @@ __device__ __forceinline__ void finish_complete(unsigned* hdr_words, unsigned ep
                                                        __HIP_MEMORY_SCOPE_AGENT);
       if (prev_all == n_cls - 1u) {
         __hip_atomic_store(&hdr->done_all, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if constexpr (SPREAD) {
+#pragma unroll 1
+          for (int i = 0; i < 7; ++i)
+            __hip_atomic_store(&hdr->ticket[i].next, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         __hip_atomic_store(&hdr->epoch, epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
@@ -328,8 +353,26 @@ __device__ __forceinline__ void finish_complete(unsigned* hdr_words, unsigned ep
 }
 
 // Both halves at once (blocks without a tile, and the end of a kernel).
+template <bool SPREAD>
 __device__ __forceinline__ void finish_block(unsigned* hdr_words, unsigned epoch) {
-  finish_complete(hdr_words, epoch, finish_issue(hdr_words, epoch));
+  finish_complete<SPREAD>(hdr_words, epoch, finish_issue(hdr_words, epoch));
+}
+
+// A block without a tile.  (Also one whose drawn tile is past the last, which
+// takes another launch drawing from the same workspace: a fault of both.)
+__device__ __forceinline__ void skip_block(unsigned* hdr_words, const Tags& tg, const TileInfo& ti) {
+  if (ti.lb >= 0 && threadIdx.x == 0) raise_fault(hdr_words, fault_tag_of(tg.agg));
+  finish_block<true>(hdr_words, tg.epoch);
+}
+
+// Launches a kernel in the version of the launch's tile order: f gets
+// std::true_type for a spread order.
+template <class F>
+void with_order(const TileOrder& o, F f) {
+  if (o.spread)
+    f(std::true_type{});
+  else
+    f(std::false_type{});
 }
 
 }  // namespace osm

@@ -32,6 +32,8 @@ constexpr float kTwoLog2e = 2.8853900817779268f;  // 2*log2(e): tanh via exp2
 //              dispatch): `done` counts its finished blocks; the last block
 //              of the class resets it.  One 128-byte line per class: no
 //              cross-class contention.
+//   ticket[i]  next tile of lane-block 8 q + i, where the running launch's
+//              blocks draw them (TileOrder); reset by the last block
 struct WsHeader {
   unsigned epoch;
   unsigned reserved0[2];
@@ -43,6 +45,10 @@ struct WsHeader {
     unsigned done;
     unsigned reserved[31];
   } cls[8];                // byte offsets 128 + 128 c
+  struct {
+    unsigned next;
+    unsigned reserved[31];
+  } ticket[7];             // byte offsets 1152 + 128 i
 };
 static_assert(sizeof(WsHeader) <= kHeaderBytes, "header fits");
 static_assert(offsetof(WsHeader, fault) < kHeaderKeepBytes && offsetof(WsHeader, done_all) == kHeaderKeepBytes,

@@ -116,7 +116,7 @@ __device__ __forceinline__ void pass2(float (&s)[G::LPT], const float (&w)[G::R]
 }
 
 // Two workgroups (4 waves per SIMD) per CU: at most 128 VGPRs.
-template <class G, bool DYN, typename XT, typename OT, int KP>
+template <class G, bool DYN, typename XT, typename OT, int KP, bool SPREAD>
 __global__ void __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 cheby_ema_fwd_kernel(const FwdParams p) {
   constexpr int R = G::R;
@@ -132,7 +132,11 @@ cheby_ema_fwd_kernel(const FwdParams p) {
   const Tags tags = launch_tags(p.hdr);
   constexpr bool kVarWords = G::WPT == kFwdWords;   // look-back words per thread chosen per launch
   const int wsh = kVarWords ? p.wsh : kWordsShift<G>;
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles, wsh);
+  const TileInfo ti = tile_info<G, SPREAD>(p.order, p.hdr, p.n_lb, p.n_lbd, p.n_tiles, wsh);
+  if (SPREAD && ti.pad) {
+    skip_block(p.hdr, tags, ti);
+    return;
+  }
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
 
   // Monomial coefficients (loads first, converted after the x loads).
@@ -297,7 +301,7 @@ cheby_ema_fwd_kernel(const FwdParams p) {
     jitter(p.jitter, tags.epoch, 1);
     look_back_finish<G, DYN>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
   }
-  finish_complete(p.hdr, tags.epoch, fin_prev);
+  finish_complete<SPREAD>(p.hdr, tags.epoch, fin_prev);
 
   // Pass 2: replay the recurrence from the true carry and store out.
   float s[LPT];
@@ -324,32 +328,30 @@ cheby_ema_fwd_kernel(const FwdParams p) {
   }
 }
 
+template <class G, bool DYN, typename XT, typename OT, int KP>
+hipError_t launch_kp(const FwdParams& p, hipStream_t stream) {
+  with_order(p.order, [&](auto spread) {
+    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, KP, decltype(spread)::value>), dim3(p.order.grid),
+                       dim3(G::THREADS), 0, stream, p);
+  });
+  return hipGetLastError();
+}
+
 template <class G, bool DYN, typename XT, typename OT>
 hipError_t launch_g(const FwdParams& p, int kpad, hipStream_t stream) {
-  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
-  if (kpad == 4)
-    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 4>), dim3(grid), dim3(G::THREADS), 0, stream, p);
-  else if (kpad == 8)
-    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 8>), dim3(grid), dim3(G::THREADS), 0, stream, p);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (kpad == 4) return launch_kp<G, DYN, XT, OT, 4>(p, stream);
+  if (kpad == 8) return launch_kp<G, DYN, XT, OT, 8>(p, stream);
+  return hipErrorInvalidValue;
 }
 
 // The one-lane geometry also serves the Chebyshev form (kpad 16 and 32);
 // K <= 4 runs with kpad 8 there (zero coefficients), one instantiation fewer.
 template <class G, bool DYN, typename XT, typename OT>
 hipError_t launch_generic(const FwdParams& p, int kpad, hipStream_t stream) {
-  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
-  if (kpad <= 8)
-    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 8>), dim3(grid), dim3(G::THREADS), 0, stream, p);
-  else if (kpad == 16)
-    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 16>), dim3(grid), dim3(G::THREADS), 0, stream, p);
-  else if (kpad == 32)
-    hipLaunchKernelGGL((cheby_ema_fwd_kernel<G, DYN, XT, OT, 32>), dim3(grid), dim3(G::THREADS), 0, stream, p);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
+  if (kpad <= 8) return launch_kp<G, DYN, XT, OT, 8>(p, stream);
+  if (kpad == 16) return launch_kp<G, DYN, XT, OT, 16>(p, stream);
+  if (kpad == 32) return launch_kp<G, DYN, XT, OT, 32>(p, stream);
+  return hipErrorInvalidValue;
 }
 
 template <class G>

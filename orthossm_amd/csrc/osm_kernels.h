@@ -141,6 +141,115 @@ constexpr size_t kHeaderBytes = 2048;
 // cleared with the look-back words).
 constexpr size_t kHeaderKeepBytes = 64;
 
+// Multiplier and shift that divide by v (1 <= v < 2^31) for dividends
+// 0 <= n < 2^31: s = ceil(log2 v), m = floor(2^32 (2^s - v) / v) + 1
+// (Granlund and Montgomery, "Division by invariant integers using
+// multiplication", 1994, the round-up variant).
+inline void div_magic(uint32_t v, uint32_t* magic, int* shift) {
+  int s = 0;
+  while ((uint64_t(1) << s) < v) ++s;
+  *shift = s;
+  *magic = (uint32_t)((((uint64_t(1) << s) - v) << 32) / v + 1);
+}
+
+__host__ __device__ __forceinline__ unsigned mul_hi(unsigned a, unsigned b) {
+  return (unsigned)(((unsigned long long)a * b) >> 32);
+}
+
+struct Divisor {
+  uint32_t mul;
+  int shift;
+  __host__ __device__ __forceinline__ unsigned of(unsigned n) const { return (mul_hi(n, mul) + n) >> shift; }
+};
+inline Divisor divisor(int64_t v) {
+  Divisor d;
+  div_magic((uint32_t)v, &d.mul, &d.shift);
+  return d;
+}
+
+// Tile order of a launch with a look-back (see osm_chain.h): which tile of
+// which lane-block a block takes.
+struct TileOrder {
+  unsigned grid;
+  bool spread;       // false: block v takes tile v / n_lb of slot v % n_lb
+  unsigned ticket;   // spread: 0, or with tickets the share of ticket blocks as a fraction of 2^32
+  int n_slots;       // spread, by index: blocks per tile row, a multiple of 8
+  Divisor by_slots, by_whole, by_rest;   // n_slots; with tickets n_lb / 8 and n_lb % 8
+};
+struct TileSlot {
+  int tile;   // >= n_tiles: none; -1: the next of the lane-block, by its ticket counter
+  int lb;     // < 0: none
+};
+
+// Lane-block of slot s: the slots of one residue mod 8 (an XCD) serve
+// consecutive lane-blocks, so the lane-blocks of a batch row share an L2 (they
+// read the same lines of g, one value per head per token).  With n_lb = 8 q + r,
+// residues below r hold q + 1.
+__host__ __device__ __forceinline__ int slot_lane_block(int s, int n_lb) {
+  const int c = s & 7, r = n_lb & 7;
+  return c * (n_lb >> 3) + (c < r ? c : r) + (s >> 3);
+}
+
+// Spread orders.  By index, block v takes tile v / n_slots of slot v %
+// n_slots, which is empty where its residue holds no such lane-block.
+// With tickets, an XCD walks q whole lane-blocks by index and, spread evenly
+// among their tiles, takes its eighth of the tiles of the r others.
+__host__ __device__ __forceinline__ TileSlot spread_slot(const TileOrder& o, unsigned block, int n_lb, int n_tiles) {
+  const int q = n_lb >> 3, r = n_lb & 7;
+  if (!o.ticket) {
+    const unsigned tile = o.by_slots.of(block), s = block - tile * (unsigned)o.n_slots;
+    const bool held = (int)(s >> 3) < q + ((int)(s & 7u) < r ? 1 : 0);
+    return {(int)tile, held ? slot_lane_block((int)s, n_lb) : -1};
+  }
+  const unsigned c = block & 7u, k = block >> 3;
+  const unsigned e = q ? mul_hi(k, o.ticket) : k;   // ticket blocks of this XCD before block k
+  if (q && mul_hi(k + 1, o.ticket) == e) {
+    const unsigned tile = o.by_whole.of(k - e);
+    return {(int)tile, (int)(c * (unsigned)q + (k - e - tile * (unsigned)q))};
+  }
+  const unsigned t = e * 8u + c;
+  return {-1, t < (unsigned)r * (unsigned)n_tiles ? 8 * q + (int)(t - o.by_rest.of(t) * (unsigned)r) : -1};
+}
+
+// With n_lb off the multiples of 8, the order by index pads the slots and gives
+// some XCDs a lane-block more than others; tickets balance them, but a block
+// then waits for an atomic on memory before its first load.  By index where the
+// fullest XCD has at most one tile for each of its CUs, or its surplus over the
+// mean is at most 12 tiles or a sixteenth of its tiles.  Measured on MI355X, by
+// index against tickets (fp32 unless noted):
+//   forward B=1 S=4096 D=256 (32 tiles on the fullest XCD) 7.0 and 7.7 us, B=3
+//   S=1000 D=400 (24) 6.9 and 7.5, TTT B=1 S=4000 D=256 (32) 15.5 and 16.2;
+//   backward B=3 S=5000 D=448 (81, surplus 10) 31.5 and 32.6; forward B=9 S=8192
+//   D=448 (128, surplus 2) 46.5 and 52.1;
+//   forward B=3 S=5001 D=400 bf16 (120, surplus 15) 13.0 and 12.9, S=20000 fp32
+//   52.4 and 49.2, B=5 S=5000 D=320 (160, surplus 35) 16.6 and 14.1, B=1 S=65536
+//   D=128 37.9 and 19.7; TTT B=5 S=16384 D=448 bf16 (430, surplus 54) 94.8 and 90.1;
+//   backward B=1 S=65536 D=128 91.6 and 46.2; table forward B=3 S=5000 D=448 (120,
+//   surplus 15) 29.5 and 27.7.
+// One counter for all lane-blocks made the tickets a queue (11 ns each): 21.1 us
+// for the bf16 forward above.
+inline TileOrder tile_order(int64_t n_lb, int64_t n_tiles) {
+  constexpr int64_t kCusPerXcd = 32;
+  TileOrder o{};
+  o.grid = (unsigned)(n_lb * n_tiles);
+  if (n_lb % 8 == 0 || n_tiles == 1) return o;
+  o.spread = true;
+  const int64_t pad = (n_lb + 7) / 8 * 8, most = pad / 8 * n_tiles, surplus = most - n_lb * n_tiles / 8;
+  if (most <= kCusPerXcd || surplus <= 12 || surplus <= most / 16) {
+    o.grid = (unsigned)(pad * n_tiles);
+    o.n_slots = (int)pad;
+    o.by_slots = divisor(pad);
+    return o;
+  }
+  const int64_t q = n_lb / 8, r = n_lb % 8;
+  const uint64_t tickets = (uint64_t)(r * n_tiles + 7) / 8, per_xcd = (uint64_t)(q * n_tiles) + tickets;
+  o.grid = (unsigned)(8 * per_xcd);
+  o.ticket = q ? (unsigned)(((tickets << 32) + per_xcd - 1) / per_xcd) : 1u;
+  if (q) o.by_whole = divisor(q);
+  o.by_rest = divisor(r);
+  return o;
+}
+
 struct FwdParams {
   const void* x;
   void* out;
@@ -163,7 +272,8 @@ struct FwdParams {
   uint32_t hd_magic;           // n / hd = (umulhi(n, hd_magic) + n) >> hd_shift for 0 <= n < 2^31
   int hd_shift;
   int n_lbd;                   // lane-blocks per batch row = ceil(D / LANES)
-  int n_lb;                    // B * n_lbd; grid = n_lb * n_tiles
+  int n_lb;                    // B * n_lbd
+  TileOrder order;
   int n_tiles;                 // ceil(S / TILE)
   float lam_shift, lam_min, lam_max;
   int clamp_out;
@@ -254,6 +364,7 @@ struct LutScanParams : V10FixedParams {
   uint32_t hd_magic;           // division by hd (div_magic)
   int hd_shift;
   int n_lbd, n_lb, n_tiles;
+  TileOrder order;
   int wsh;                     // log2 of the look-back words per thread
   int clamp_at;                // tile that holds the first clamp boundary
   unsigned poll_limit;
@@ -295,17 +406,6 @@ struct EngineParams {
   int B, S, D;
   float eps;
 };
-
-// Multiplier and shift that divide by v (1 <= v < 2^31) for dividends
-// 0 <= n < 2^31: s = ceil(log2 v), m = floor(2^32 (2^s - v) / v) + 1
-// (Granlund and Montgomery, "Division by invariant integers using
-// multiplication", 1994, the round-up variant).
-inline void div_magic(uint32_t v, uint32_t* magic, int* shift) {
-  int s = 0;
-  while ((uint64_t(1) << s) < v) ++s;
-  *shift = s;
-  *magic = (uint32_t)((((uint64_t(1) << s) - v) << 32) / v + 1);
-}
 
 // Workspace layout helpers (bytes).
 size_t slot_words(bool dyn);

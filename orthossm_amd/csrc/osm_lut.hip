@@ -27,7 +27,7 @@ namespace {
 // to 0 would make it NaN.  Finite states do not notice 2^-149.
 constexpr float kTinyDecay = 1.401298464324817e-45f;
 
-template <class G, typename XT, int KP, bool LUT>
+template <class G, typename XT, int KP, bool LUT, bool SPREAD>
 __global__ void __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 lut_fwd_kernel(const LutScanParams p) {
   constexpr int R = G::R, LPT = G::LPT;
@@ -39,7 +39,11 @@ lut_fwd_kernel(const LutScanParams p) {
 
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles, p.wsh);
+  TileInfo ti = tile_info<G, SPREAD>(p.order, p.hdr, p.n_lb, p.n_lbd, p.n_tiles, p.wsh);
+  if (SPREAD && ti.pad) {
+    skip_block(p.hdr, tags, ti);
+    return;
+  }
   const int t_tile = ti.tile * G::TILE;
   const int d0 = ti.lbd * kLanes + q.lt * LPT;
   const bool lane_ok = d0 < p.D;
@@ -175,7 +179,7 @@ lut_fwd_kernel(const LutScanParams p) {
     look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A64, p.hdr, p.poll_limit,
                                kTinyDecay);
   }
-  finish_complete(p.hdr, tags.epoch, fin_prev);
+  finish_complete<SPREAD>(p.hdr, tags.epoch, fin_prev);
   if (at_clamp && !ti.is_last && q.wave == 0) {
     float s = L.carry[q.wl];
     for (int g = 0; g < G::NTG; ++g) {
@@ -230,14 +234,18 @@ lut_fwd_kernel(const LutScanParams p) {
   }
 }
 
+template <class G, typename XT, bool LUT, int KP>
+hipError_t launch_kp(const LutScanParams& p, hipStream_t stream) {
+  with_order(p.order, [&](auto spread) {
+    hipLaunchKernelGGL((lut_fwd_kernel<G, XT, KP, LUT, decltype(spread)::value>), dim3(p.order.grid),
+                       dim3(G::THREADS), 0, stream, p);
+  });
+  return hipGetLastError();
+}
+
 template <class G, typename XT, bool LUT>
 hipError_t launch_g(const LutScanParams& p, int kpad, hipStream_t stream) {
-  const dim3 grid((unsigned)p.n_lb * (unsigned)p.n_tiles), block(G::THREADS);
-  if (kpad == 4)
-    hipLaunchKernelGGL((lut_fwd_kernel<G, XT, 4, LUT>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((lut_fwd_kernel<G, XT, 8, LUT>), grid, block, 0, stream, p);
-  return hipGetLastError();
+  return kpad == 4 ? launch_kp<G, XT, LUT, 4>(p, stream) : launch_kp<G, XT, LUT, 8>(p, stream);
 }
 
 template <typename XT, bool LUT>

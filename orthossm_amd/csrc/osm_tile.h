@@ -102,7 +102,7 @@ __device__ __forceinline__ MonoLoad<KP, G> mono_issue(const FwdParams& p, const 
       // out-of-range offset): a branch here would make the compiler convert
       // each value inside it and so wait for every load on the spot, before
       // the caller's bulk loads are issued.
-      // (every tile of the lane-block, all on one XCD, reads them)
+      // (every tile of the lane-block reads them)
       const int k = j + 2 * i;
       m.cm[n][i] = load_f32_shared(a.c, k < p.K ? vc : kOffOOB, (uint32_t)k * a.sc);
     }

@@ -252,7 +252,7 @@ __device__ __forceinline__ float wave_sum_tg(float v) {
 }
 
 // Two workgroups (4 waves per SIMD) per CU: at most 128 VGPRs.
-template <class G, bool DYN, bool SOFT, typename XT, typename OT, int KP>
+template <class G, bool DYN, bool SOFT, typename XT, typename OT, int KP, bool SPREAD>
 __global__ void __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 cheby_ema_ttt_kernel(const FwdParams p) {
   constexpr int R = G::R;
@@ -278,7 +278,11 @@ cheby_ema_ttt_kernel(const FwdParams p) {
 
   const ThreadPos q = thread_pos<G>();
   const Tags tags = launch_tags(p.hdr);
-  const TileInfo ti = tile_info<G>(blockIdx.x, p.n_lb, p.n_lbd, p.n_tiles);
+  const TileInfo ti = tile_info<G, SPREAD>(p.order, p.hdr, p.n_lb, p.n_lbd, p.n_tiles);
+  if (SPREAD && ti.pad) {
+    skip_block(p.hdr, tags, ti);
+    return;
+  }
   const TileAddr a = tile_addr<G, DYN, XT, OT>(p, q, ti);
   // This wave's monomial coefficient (wave w holds coefficient w of the 64
   // lanes), formed once per launch by ttt_mono_prep or, without a table
@@ -543,7 +547,7 @@ cheby_ema_ttt_kernel(const FwdParams p) {
     for (int w = 0; w < G::WAVES; ++w) acc += sh_ur.red[w][v][q.wl];
     part[(size_t)v * kLanes + q.wl] = ks_w * acc;
   }
-  finish_block(p.hdr, tags.epoch);
+  finish_block<SPREAD>(p.hdr, tags.epoch);
 }
 
 // The scaled monomial coefficients of every lane-block, as the forward forms
@@ -670,8 +674,10 @@ hipError_t launch_all(const FwdParams& p0, float* grad, hipStream_t stream) {
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  const unsigned grid = (unsigned)p.n_lb * (unsigned)p.n_tiles;
-  hipLaunchKernelGGL((cheby_ema_ttt_kernel<G, DYN, SOFT, XT, OT, KP>), dim3(grid), dim3(G::THREADS), 0, stream, p);
+  with_order(p.order, [&](auto spread) {
+    hipLaunchKernelGGL((cheby_ema_ttt_kernel<G, DYN, SOFT, XT, OT, KP, decltype(spread)::value>), dim3(p.order.grid),
+                       dim3(G::THREADS), 0, stream, p);
+  });
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (p.n_tiles <= kDirectTiles) {

@@ -119,3 +119,28 @@ def test_chains_across_xcds(dev, B, S, H, hd, dyn):
     wx, wc, _ = oracle_backward(inp, go.cpu().numpy(), out_saved=a[0].cpu().numpy())
     assert_close_grad(a[4].cpu(), wx, what="grad_x")
     assert_close_grad(a[5].cpu(), wc, what="grad_coeffs")
+
+
+def test_launches_on_several_streams(dev):
+    """Launches that wait across XCDs and hold more blocks than the chip has
+    places for, on four streams at once: each equals the launch alone, and no
+    wait gives up."""
+    from orthossm_amd.ops import cheby_ema_lut_forward
+    inp = to_dev(inputs(3, 9000, 8, 50, 8, seed=5), dev)
+    args = (inp["x"], inp["coeffs"], inp["damping"], inp["lam"])
+    go = torch.randn(3, 9000, 400, generator=torch.Generator().manual_seed(6)).to(dev)
+    out = cheby_ema_forward(*args)
+    calls = (lambda: (cheby_ema_forward(*args),), lambda: cheby_ema_ttt(*args),
+             lambda: cheby_ema_backward(*args, out, go)[:2], lambda: cheby_ema_lut_forward(inp["x"], inp["coeffs"], n_heads=8))
+    want = [f() for f in calls]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in calls]
+    for _ in range(3):
+        got = [None] * len(calls)
+        for i in range(12):
+            with torch.cuda.stream(streams[i % 4]):
+                got[i % 4] = calls[(i + i // 4) % 4]()
+        torch.cuda.synchronize()
+        for i in range(4):
+            assert_same(got[i], want[(i + 10) % 4])
+    assert ops.workspace_faults() == []

@@ -120,7 +120,8 @@ typedef enum osm_status {
                                       word is set and the outputs that depend
                                       on the missing value are NaN (out,
                                       ema_final, the TTT gradient, the
-                                      backward's gradients); every kernel
+                                      backward's gradients, the table
+                                      forward's out and ema_final); every kernel
                                       still exits normally */
 
 /* TTT target y */
@@ -427,7 +428,8 @@ int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* args, void* stream);
  * and gives the same results up to rounding; where the scan does not apply
  * (osm_lut_fwd_workspace_bytes gives 0: a decay outside [0.25, 1], a short
  * sequence of few lanes, or invalid arguments) it is osm_cheby_ema_lut_fwd,
- * and the workspace may be NULL. */
+ * and the workspace may be NULL.  Both also take the look-back's test flags,
+ * OSM_FLAG_TIMING_JITTER and OSM_FLAG_POLL_LIMIT_ZERO. */
 size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* args);
 int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* args, void* workspace, size_t workspace_bytes, void* stream);
 

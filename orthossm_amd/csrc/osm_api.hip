@@ -309,12 +309,15 @@ int run_empty(const osm_cheby_args* a, hipStream_t stream) {
 }
 
 // Validates the fixed-coefficient forward's arguments without touching the
-// GPU.  Returns OSM_OK or an error; B == 0 is valid (nothing to do).
-int check_lut(const osm_lut_fwd_args* a) {
+// GPU.  Returns OSM_OK or an error; B == 0 is valid (nothing to do).  ws: the
+// entry points with a look-back, which take its test flags.
+constexpr int kLookBackTests = OSM_FLAG_TIMING_JITTER | OSM_FLAG_POLL_LIMIT_ZERO;
+int check_lut(const osm_lut_fwd_args* a, bool ws) {
   if (!a) return fail(OSM_E_ARG, "args is NULL");
   if (a->abi_version != OSM_ABI_VERSION)
     return fail(OSM_E_ARG, "abi_version %d does not match library ABI %d", a->abi_version, OSM_ABI_VERSION);
-  if (a->flags & ~OSM_V10_USE_LUT) return fail(OSM_E_ARG, "unknown flag bits 0x%x", a->flags);
+  if (a->flags & ~(OSM_V10_USE_LUT | (ws ? kLookBackTests : 0)))
+    return fail(OSM_E_ARG, "unknown flag bits 0x%x", a->flags);
   if (a->B < 0 || a->S < 0 || a->H < 1 || a->hd < 1)
     return fail(OSM_E_SHAPE, "need B, S >= 0, H, hd >= 1 (B=%lld S=%lld H=%lld hd=%lld)", (long long)a->B,
                 (long long)a->S, (long long)a->H, (long long)a->hd);
@@ -394,6 +397,21 @@ osm::V10FixedParams lut_params(const osm_lut_fwd_args* a) {
   p.ty_ss = a->ty_stride_s;
   p.clamp_tile = (int)a->clamp_tile;
   return p;
+}
+
+// The forward by the walk of osm_v10.hip, arguments checked.
+int run_lut_walk(const osm_lut_fwd_args* a, void* stream) {
+  if (a->B == 0) return ok();
+  osm::V10FixedParams p = lut_params(a);
+  // Waves of 32 tokens with 8 lanes per workgroup, 16 with 16 lanes: the
+  // clamp boundaries fall between waves.
+  p.lanes = a->clamp_tile % 32 ? 16 : osm::v10_fixed_lanes(a->B, a->H, a->hd);
+  p.n_lg = (int)((a->hd + p.lanes - 1) / p.lanes);
+  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 64) return fail(OSM_E_SHAPE, "problem too large");
+  const hipError_t e = osm::launch_v10_fixed(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0, a->K <= 4 ? 4 : 8,
+                                             static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "fixed-coefficient forward launch");
+  return ok();
 }
 
 // Geometry of the scan (osm_lut.hip) for these arguments, or n_tiles = 0
@@ -749,32 +767,21 @@ int osm_v10_bwd(const osm_v10_bwd_args* a, void* stream) {
 }
 
 int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* a, void* stream) {
-  const int rc = check_lut(a);
-  if (rc != OSM_OK) return rc;
-  if (a->B == 0) return ok();
-  osm::V10FixedParams p = lut_params(a);
-  // Waves of 32 tokens with 8 lanes per workgroup, 16 with 16 lanes: the
-  // clamp boundaries fall between waves.
-  p.lanes = a->clamp_tile % 32 ? 16 : osm::v10_fixed_lanes(a->B, a->H, a->hd);
-  p.n_lg = (int)((a->hd + p.lanes - 1) / p.lanes);
-  if ((int64_t)p.B * p.H * p.n_lg >= (int64_t(1) << 31) - 64) return fail(OSM_E_SHAPE, "problem too large");
-  const hipError_t e = osm::launch_v10_fixed(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0, a->K <= 4 ? 4 : 8,
-                                             static_cast<hipStream_t>(stream));
-  if (e != hipSuccess) return hip_fail(e, "fixed-coefficient forward launch");
-  return ok();
+  const int rc = check_lut(a, false);
+  return rc == OSM_OK ? run_lut_walk(a, stream) : rc;
 }
 
 size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* a) {
-  if (check_lut(a) != OSM_OK) return 0;
+  if (check_lut(a, true) != OSM_OK) return 0;
   const Geometry geo = lut_scan_shape(a);
   return geo.n_tiles ? osm::fwd_workspace_bytes(geo.n_lb, geo.n_tiles, geo.lanes, false) : 0;
 }
 
 int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t workspace_bytes, void* stream) {
-  int rc = check_lut(a);
+  int rc = check_lut(a, true);
   if (rc != OSM_OK) return rc;
   const Geometry geo = lut_scan_shape(a);
-  if (!geo.n_tiles) return osm_cheby_ema_lut_fwd(a, stream);
+  if (!geo.n_tiles) return run_lut_walk(a, stream);
   const size_t need = osm::fwd_workspace_bytes(geo.n_lb, geo.n_tiles, geo.lanes, false);
   rc = check_ws(geo, OSM_OP_FWD, (int)a->K, workspace, workspace_bytes);
   if (rc != OSM_OK) return rc;
@@ -792,7 +799,8 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   p.order = osm::tile_order(geo.n_lb, geo.n_tiles);
   p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
-  p.poll_limit = osm::kSpinLimit;
+  p.jitter = (a->flags & OSM_FLAG_TIMING_JITTER) ? 1 : 0;
+  p.poll_limit = (a->flags & OSM_FLAG_POLL_LIMIT_ZERO) ? 0u : osm::kSpinLimit;
   const hipError_t e = osm::launch_lut_scan(p, a->x_dtype, (a->flags & OSM_V10_USE_LUT) != 0,
                                             osm::FwdShape{geo.tile, geo.lanes, geo.lpt}, geo.kpad, st);
   if (e != hipSuccess) return hip_fail(e, "fixed-coefficient scan launch");

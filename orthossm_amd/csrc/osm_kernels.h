@@ -367,6 +367,7 @@ struct LutScanParams : V10FixedParams {
   TileOrder order;
   int wsh;                     // log2 of the look-back words per thread
   int clamp_at;                // tile that holds the first clamp boundary
+  int jitter;                  // as in FwdParams
   unsigned poll_limit;
 };
 

@@ -27,6 +27,11 @@ namespace {
 // to 0 would make it NaN.  Finite states do not notice 2^-149.
 constexpr float kTinyDecay = 1.401298464324817e-45f;
 
+// The clamp of a state; NaN (a look-back wait gave up) stays NaN.
+__device__ __forceinline__ float clamp_state(float s) {
+  return s == s ? __builtin_amdgcn_fmed3f(s, -1.0f, 1.0f) : s;
+}
+
 template <class G, typename XT, int KP, bool LUT, bool SPREAD>
 __global__ void __launch_bounds__(G::THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 lut_fwd_kernel(const LutScanParams p) {
@@ -165,17 +170,21 @@ lut_fwd_kernel(const LutScanParams p) {
   const bool ckpt = ti.is_ckpt;
   ti.is_ckpt = ckpt || at_clamp;
   float pA, pB[LPT], aggA, aggB;
+  jitter(p.jitter, tags.epoch, 0);
   const float run_A = __builtin_fmaxf(pow_n<R>(mu), kTinyDecay);
   tile_scan<G, false>(L, q, ti, tags, run_A, Bv, pA, pB, aggA, aggB, ls);
   {
     const int dc = ti.lbd * kLanes + carry_lane<G>(q);
-    const float init_c =
-        p.ema_init && q.wave == 0 && dc < p.D ? p.ema_init[(int64_t)ti.b * p.init_sb + dc] : 0.0f;
+    float init_c = p.ema_init && q.wave == 0 && dc < p.D ? p.ema_init[(int64_t)ti.b * p.init_sb + dc] : 0.0f;
+    // A NaN state gives -1 from every clamp, as -inf does, which stands for it
+    // here: a NaN carry then comes only from a look-back wait that gave up.
+    init_c = init_c == init_c ? init_c : -__builtin_inff();
     const double tile_A64 = __builtin_fmax(pow_n_f64<G::TILE>((double)mu), (double)kTinyDecay);
     const float tile_A = (float)tile_A64;
     LookBack<G, false> lbk;
     look_back_issue<G, false>(lbk, q, ti, ls, p.wsh, ti.tile > p.clamp_at ? p.clamp_at + 1 : 0);
     ti.is_ckpt = ckpt && !at_clamp;   // the clamped tile's state is published below
+    jitter(p.jitter, tags.epoch, 1);
     look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A64, p.hdr, p.poll_limit,
                                kTinyDecay);
   }
@@ -184,8 +193,9 @@ lut_fwd_kernel(const LutScanParams p) {
     float s = L.carry[q.wl];
     for (int g = 0; g < G::NTG; ++g) {
       s = __builtin_fmaf(L.A[g][q.wl / LPT], s, L.B[g][q.wl]);
-      if (g == g_clamp) s = __builtin_amdgcn_fmed3f(s, -1.0f, 1.0f);
+      if (g == g_clamp) s = clamp_state(s);
     }
+    jitter(p.jitter, tags.epoch, 2);
     publish(ls.at(ti.tile, q.wl), tags.pre, s);
   }
 
@@ -200,15 +210,14 @@ lut_fwd_kernel(const LutScanParams p) {
 #pragma unroll
       for (int i = 0; i < LPT; ++i) {
         s[i] = __builtin_fmaf(L.A[g][q.lt], s[i], L.B[g][q.lt * LPT + i]);
-        if (g == g_clamp) s[i] = __builtin_amdgcn_fmed3f(s[i], -1.0f, 1.0f);
+        if (g == g_clamp) s[i] = clamp_state(s[i]);
       }
   } else {
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      s[i] = __builtin_fmaf(pA, L.carry[q.lt * LPT + i], pB[i]);
-      lost |= s[i] != s[i];   // only a look-back wait that gave up leaves this
-    }
+    for (int i = 0; i < LPT; ++i) s[i] = __builtin_fmaf(pA, L.carry[q.lt * LPT + i], pB[i]);
   }
+#pragma unroll
+  for (int i = 0; i < LPT; ++i) lost |= s[i] != s[i];
   const Rsrc orr = rows(p.out, p.o_sb, p.o_ss, 4);
   const uint32_t vo = lane_off(p.o_ss, 4), so_step = (uint32_t)(p.o_ss * 4);
   const int r_last = p.S - 1 - (t_tile + q.tg * R);
@@ -223,7 +232,7 @@ lut_fwd_kernel(const LutScanParams p) {
     for (int i = 0; i < LPT; ++i) {
       s[i] = __builtin_fmaf(mu, s[i], w[r][i]);
       o[i] = __builtin_amdgcn_fmed3f(s[i], -1.0f, 1.0f);
-      o[i] = lost ? s[i] : o[i];
+      if (lost) o[i] = clamp_state(s[i]);
     }
     BufVec<float, LPT>::store(orr, vo, so, o);
     so = next_off(so, so_step);

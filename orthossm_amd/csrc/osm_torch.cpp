@@ -480,7 +480,7 @@ PyObject* run_v10_backward(PyObject* const* p) {
   return THPVariable_Wrap(gx);
 }
 
-// lut_forward(x, coeffs, n_heads, mu, ema_init, use_lut, lut, clamp_tile,
+// lut_forward(x, coeffs, n_heads, mu, ema_init, flags, lut, clamp_tile,
 // want_x_norm, want_tanh_y): None, or (out, x_norm | None, tanh_y | None, ema_final).
 PyObject* run_lut(PyObject* const* p) {
   const at::Tensor *xp = plain(p[0]), *cp = plain(p[1]);
@@ -500,12 +500,11 @@ PyObject* run_lut(PyObject* const* p) {
     a.ema_init = fptr(*t);
     a.init_stride_b = t->stride(0);
   }
-  const bool use_lut = PyObject_IsTrue(p[5]) == 1;
-  if (use_lut) a.lut = fptr(THPVariable_Unpack(p[6]));   // the module's own table
+  a.flags = (int32_t)PyLong_AsLong(p[5]);
+  if (a.flags & OSM_V10_USE_LUT) a.lut = fptr(THPVariable_Unpack(p[6]));   // the module's own table
   const bool want_n = PyObject_IsTrue(p[8]) == 1, want_y = PyObject_IsTrue(p[9]) == 1;
   if (PyErr_Occurred()) return nullptr;
   a.abi_version = OSM_ABI_VERSION;
-  a.flags = use_lut ? OSM_V10_USE_LUT : 0;
   a.x = x.data_ptr();
   a.x_dtype = code(x);
   a.x_stride_b = x.stride(0);

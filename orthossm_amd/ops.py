@@ -43,8 +43,8 @@ def set_fault_check(on: bool) -> bool:
     return old
 
 
-# Test aid: with timing jitter on, the forward, TTT and backward launches
-# carry OSM_FLAG_TIMING_JITTER (every workgroup sleeps a pseudo-random time
+# Test aid: with timing jitter on, the forward, TTT, backward and table-forward
+# scan launches carry OSM_FLAG_TIMING_JITTER (every workgroup sleeps a pseudo-random time
 # before it publishes to the look-back); results must not change.
 _timing_jitter = False
 
@@ -56,8 +56,8 @@ def set_timing_jitter(on: bool) -> bool:
     return old
 
 
-# Test aid: with the poll limit at zero, the forward, TTT and backward
-# launches carry OSM_FLAG_POLL_LIMIT_ZERO: a look-back wait whose word is not
+# Test aid: with the poll limit at zero, the forward, TTT, backward and
+# table-forward scan launches carry OSM_FLAG_POLL_LIMIT_ZERO: a look-back wait whose word is not
 # yet published gives up at once (the fault word is set and the outputs that
 # depend on the missing value are NaN), as a wait that passes its poll limit
 # does.
@@ -155,12 +155,15 @@ def _fast():
     return None if _check_faults else _ext
 
 
+def _test_flags() -> int:
+    return (nat.FLAG_TIMING_JITTER if _timing_jitter else 0) | (nat.FLAG_POLL_LIMIT_ZERO if _poll_limit_zero else 0)
+
+
 def _flags(clamp: bool, nan_policy: str) -> int:
     if nan_policy not in ("zero_z", "zero_u"):
         raise ValueError("nan_policy must be 'zero_z' or 'zero_u'")
     return ((0 if clamp else nat.FLAG_NO_CLAMP) | (nat.FLAG_NAN_ZERO_U if nan_policy == "zero_u" else 0) |
-            (nat.FLAG_TIMING_JITTER if _timing_jitter else 0) |
-            (nat.FLAG_POLL_LIMIT_ZERO if _poll_limit_zero else 0))
+            _test_flags())
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int, op: int) -> torch.Tensor:
@@ -702,7 +705,8 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and \
             ema_final is None and coeffs.dim() == 4 and coeffs.shape[1] == n_heads:
         table = v10_tables(dev, n_heads, LUT_TERMS)[0] if use_lut else None
-        res = fast.lut_forward(x, coeffs, n_heads, ema_momentum, ema_init, use_lut, table, clamp_tile, want_x_norm,
+        res = fast.lut_forward(x, coeffs, n_heads, ema_momentum, ema_init,
+                               (nat.V10_USE_LUT if use_lut else 0) | _test_flags(), table, clamp_tile, want_x_norm,
                                want_tanh_y)
         if res is not None:
             return res
@@ -762,6 +766,7 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     # the tiles, which needs none.
     nbytes = 0 if capturing else lib.osm_lut_fwd_workspace_bytes(ctypes.byref(a))
     if nbytes:
+        a.flags |= _test_flags()
         ws = _workspace(dev, stream, nbytes, nat.OP_LUT)
         nat.check(lib.osm_cheby_ema_lut_fwd_ws(ctypes.byref(a), ctypes.c_void_p(ws.data_ptr()), ws.numel(),
                                                ctypes.c_void_p(stream)))

@@ -102,12 +102,17 @@ def _run_case(case, d, dev):
     if case == "ttt":
         out, grad = cheby_ema_ttt(d["x"], d["coeffs"], d["damping"], d["lam"], g=d.get("g"))
         return (out, grad), nat.OP_TTT
+    if case.startswith("lut"):
+        # the first clamp in the second tile, or past 32 tiles (a checkpoint of its own)
+        out, _, _, fin = ops.cheby_ema_lut_forward(d["x"], d["coeffs"], n_heads=8, ema_init=d["init"],
+                                                   clamp_tile=4208 if case == "lut_late_clamp" else 256)
+        return (out, fin), nat.OP_LUT
     out = d["out_saved"]
     gx, gc, gi = cheby_ema_backward(d["x"], d["coeffs"], d["damping"], d["lam"], out, d["go"], need_init=True)
     return (gx, gc, gi), nat.OP_BWD
 
 
-@pytest.mark.parametrize("case", ["fwd_static", "fwd_dynamic", "ttt", "bwd"])
+@pytest.mark.parametrize("case", ["fwd_static", "fwd_dynamic", "ttt", "bwd", "lut", "lut_late_clamp"])
 def test_poll_limit_zero_poisons_the_dependent_outputs(dev, case):
     """OSM_FLAG_POLL_LIMIT_ZERO (with the timing jitter, so that tiles
     publish late): a look-back word not yet published at its first read
@@ -122,6 +127,8 @@ def test_poll_limit_zero_poisons_the_dependent_outputs(dev, case):
     if case == "bwd":
         d["out_saved"] = cheby_ema_forward(d["x"], d["coeffs"], d["damping"], d["lam"])
         d["go"] = torch.randn(B, S, 512, generator=torch.Generator().manual_seed(61)).to(dev)
+    # states outside [-1, 1], infinite and NaN up to the table forward's first clamp
+    d["init"] = torch.tensor([0.5, 30.0, float("inf"), float("nan")], device=dev).repeat(B, 128)
     ref, op = _run_case(case, d, dev)
     ref = [t.clone() for t in ref]
     stream = torch.cuda.current_stream(dev).cuda_stream

@@ -89,6 +89,19 @@ def test_backward_bits_unchanged(dev):
     assert_same(a, b)
 
 
+@pytest.mark.parametrize("B,S,H,hd,clamp_tile", [
+    (2, 9000, 8, 64, 128),       # the clamp in the first tile
+    (1, 9000, 4, 64, 1040),      # four look-back words per thread, the clamp inside a group
+    (3, 6000, 7, 48, 2064),      # tiles drawn by ticket
+])
+def test_table_forward_bits_unchanged(dev, B, S, H, hd, clamp_tile):
+    d = to_dev(inputs(B, S, H, hd, 8, seed=S + H), dev)
+    init = torch.linspace(-3, 3, B * H * hd, device=dev).view(B, H * hd)
+    a, b = twice(lambda: ops.cheby_ema_lut_forward(d["x"], d["coeffs"], n_heads=H, ema_init=init, clamp_tile=clamp_tile,
+                                                   ema_momentum=0.999))
+    assert_same(a, b)
+
+
 @pytest.mark.parametrize("B,S,H,hd,dyn", [
     (1, 9000, 1, 64, False),     # one lane-block: its tiles rotate over all eight XCDs
     (3, 5000, 1, 48, True),      # three, of 48 lanes

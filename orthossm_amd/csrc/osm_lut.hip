@@ -175,10 +175,14 @@ lut_fwd_kernel(const LutScanParams p) {
   tile_scan<G, false>(L, q, ti, tags, run_A, Bv, pA, pB, aggA, aggB, ls);
   {
     const int dc = ti.lbd * kLanes + carry_lane<G>(q);
-    float init_c = p.ema_init && q.wave == 0 && dc < p.D ? p.ema_init[(int64_t)ti.b * p.init_sb + dc] : 0.0f;
-    // A NaN state gives -1 from every clamp, as -inf does, which stands for it
-    // here: a NaN carry then comes only from a look-back wait that gave up.
-    init_c = init_c == init_c ? init_c : -__builtin_inff();
+    // (past the first clamp no tile uses it.)  A NaN state gives -1 from every
+    // clamp, as -inf does, which stands for it here: a NaN carry then comes
+    // only from a look-back wait that gave up.
+    float init_c = 0.0f;
+    if (p.ema_init && ti.tile <= p.clamp_at && q.wave == 0 && dc < p.D) {
+      init_c = p.ema_init[(int64_t)ti.b * p.init_sb + dc];
+      init_c = init_c == init_c ? init_c : -__builtin_inff();
+    }
     const double tile_A64 = __builtin_fmax(pow_n_f64<G::TILE>((double)mu), (double)kTinyDecay);
     const float tile_A = (float)tile_A64;
     LookBack<G, false> lbk;
@@ -195,7 +199,6 @@ lut_fwd_kernel(const LutScanParams p) {
       s = __builtin_fmaf(L.A[g][q.wl / LPT], s, L.B[g][q.wl]);
       if (g == g_clamp) s = clamp_state(s);
     }
-    jitter(p.jitter, tags.epoch, 2);
     publish(ls.at(ti.tile, q.wl), tags.pre, s);
   }
 
@@ -224,23 +227,28 @@ lut_fwd_kernel(const LutScanParams p) {
   float* fin = ti.is_last && p.ema_final && lane_ok && r_last >= 0 && r_last < R
                    ? p.ema_final + (int64_t)ti.b * p.final_sb + d0
                    : nullptr;
-  uint32_t so = 0;
+  auto replay = [&](auto nan_c) {
+    uint32_t so = 0;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    float o[LPT];
+    for (int r = 0; r < R; ++r) {
+      float o[LPT];
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      s[i] = __builtin_fmaf(mu, s[i], w[r][i]);
-      o[i] = __builtin_amdgcn_fmed3f(s[i], -1.0f, 1.0f);
-      if (lost) o[i] = clamp_state(s[i]);
+      for (int i = 0; i < LPT; ++i) {
+        s[i] = __builtin_fmaf(mu, s[i], w[r][i]);
+        o[i] = decltype(nan_c)::value ? clamp_state(s[i]) : __builtin_amdgcn_fmed3f(s[i], -1.0f, 1.0f);
+      }
+      BufVec<float, LPT>::store(orr, vo, so, o);
+      so = next_off(so, so_step);
+      if (fin && r == r_last) {
+#pragma unroll
+        for (int i = 0; i < LPT; ++i) fin[i] = o[i];
+      }
     }
-    BufVec<float, LPT>::store(orr, vo, so, o);
-    so = next_off(so, so_step);
-    if (fin && r == r_last) {
-#pragma unroll
-      for (int i = 0; i < LPT; ++i) fin[i] = o[i];
-    }
-  }
+  };
+  if (lost)
+    replay(std::true_type{});
+  else
+    replay(std::false_type{});
 }
 
 template <class G, typename XT, bool LUT, int KP>

@@ -427,7 +427,8 @@ int osm_cheby_ema_lut_fwd(const osm_lut_fwd_args* args, void* stream);
  * of one workgroup walking each group of lanes.  Takes the same arguments
  * and gives the same results up to rounding; where the scan does not apply
  * (osm_lut_fwd_workspace_bytes gives 0: a decay outside [0.25, 1], a short
- * sequence of few lanes, or invalid arguments) it is osm_cheby_ema_lut_fwd,
+ * sequence of few lanes, an output in the memory of ema_init or, other than
+ * element for element, of x, or invalid arguments) it is osm_cheby_ema_lut_fwd,
  * and the workspace may be NULL.  Both also take the look-back's test flags,
  * OSM_FLAG_TIMING_JITTER and OSM_FLAG_POLL_LIMIT_ZERO. */
 size_t osm_lut_fwd_workspace_bytes(const osm_lut_fwd_args* args);

@@ -414,9 +414,49 @@ int run_lut_walk(const osm_lut_fwd_args* a, void* stream) {
   return ok();
 }
 
+// Bytes that [B,S,D] rows of `size` bytes an element lie in; none for a NULL.
+struct Span {
+  uintptr_t lo = 0, hi = 0;
+  Span(const void* p, int64_t sb, int64_t ss, int64_t B, int64_t S, int64_t D, int size) {
+    if (!p || B < 1 || S < 1) return;
+    lo = (uintptr_t)p;
+    hi = lo + (uintptr_t)((B - 1) * sb + (S - 1) * ss + D) * (uintptr_t)size;
+  }
+  bool meets(const Span& o) const { return lo < o.hi && o.lo < hi; }
+};
+
+// Whether an output of the table forward lies in memory that it reads: the
+// initial state, or x other than element for element.  The walk reads a lane
+// group's state before it writes any of its lanes, and its rows in order; the
+// scan's tiles read the state at any time before the last one ends.
+bool lut_in_place(const osm_lut_fwd_args* a) {
+  const int64_t D = a->H * a->hd;
+  const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
+  const Span x(a->x, a->x_stride_b, a->x_stride_s, a->B, a->S, D, xs);
+  const Span init(a->ema_init, a->init_stride_b, 0, a->B, 1, D, 4);
+  struct {
+    float* p;
+    int64_t sb, ss, rows;
+  } const outs[4] = {{a->out, a->out_stride_b, a->out_stride_s, a->S},
+                     {a->x_norm, a->xn_stride_b, a->xn_stride_s, a->S},
+                     {a->tanh_y, a->ty_stride_b, a->ty_stride_s, a->S},
+                     {a->ema_final, a->final_stride_b, 0, 1}};
+  for (const auto& o : outs) {
+    const Span s(o.p, o.sb, o.ss, a->B, o.rows, D, 4);
+    if (s.meets(init)) return true;
+    if (!s.meets(x)) continue;
+    // rows of one layout: element for element, or other columns of wider rows
+    const bool alike = xs == 4 && o.sb == a->x_stride_b && o.ss == a->x_stride_s && o.rows == a->S;
+    const int64_t shift = ((intptr_t)s.lo - (intptr_t)x.lo) / 4, by = shift < 0 ? -shift : shift;
+    if (!(alike && (shift == 0 || (by >= D && by <= o.ss - D)))) return true;
+  }
+  return false;
+}
+
 // Geometry of the scan (osm_lut.hip) for these arguments, or n_tiles = 0
 // where the walk of osm_v10.hip serves the call: a decay outside [0.25, 1] (a
-// negative one reverses the clamp, one above 1 lets later clamps bind), or a
+// negative one reverses the clamp, one above 1 lets later clamps bind),
+// outputs in place of inputs (lut_in_place), or a
 // sequence the walk does in one block on one round of workgroups: at most 256
 // tokens and 2048 lanes (256 workgroups of 8).  Measured on MI355X, K=8, walk
 // against scan: 6.4 and 7.9 us at B=1 S=256 D=512, 7.2 and 8.4 at B=4, 10.1
@@ -424,7 +464,7 @@ int run_lut_walk(const osm_lut_fwd_args* a, void* stream) {
 Geometry lut_scan_shape(const osm_lut_fwd_args* a) {
   Geometry geo;
   if (!(a->ema_momentum >= 0.25f && a->ema_momentum <= 1.0f) || a->B == 0) return geo;
-  if (a->S == 0 || (a->S <= 256 && a->B * a->H * a->hd <= 2048)) return geo;
+  if (a->S == 0 || (a->S <= 256 && a->B * a->H * a->hd <= 2048) || lut_in_place(a)) return geo;
   const int xs = a->x_dtype == OSM_F32 ? 4 : 2;
   auto pairs = [](const void* p, int size, int64_t sb, int64_t ss) {
     return !p || ((uintptr_t)p % (uintptr_t)(2 * size) == 0 && sb % 2 == 0 && ss % 2 == 0);

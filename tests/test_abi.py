@@ -310,6 +310,27 @@ def test_lut_fwd_argument_errors(kw, code):
     assert lib.osm_cheby_ema_lut_fwd(None, None) == -1
 
 
+@pytest.mark.parametrize("kw,scan", [
+    (dict(), True),                                                       # out in place of x, element for element
+    (dict(out=0x900000), True),
+    (dict(out=0x10000 + 4 * 64, out_stride_s=128, out_stride_b=512 * 128, x_stride_s=128, x_stride_b=512 * 128), True),
+    (dict(out=0x10000 + 4 * 48, out_stride_s=128, out_stride_b=512 * 128, x_stride_s=128, x_stride_b=512 * 128), False),
+    (dict(out=0x10000 - 4 * 64), False),                                  # a row back
+    (dict(x_dtype=1), False),                                             # a bf16 x under fp32 results
+    (dict(ema_init=0x900000, init_stride_b=64, ema_final=0x900000, final_stride_b=64), False),
+    (dict(ema_init=0x900000, init_stride_b=64, ema_final=0x900000 + 4 * 127, final_stride_b=64), False),
+    (dict(ema_init=0x900000, init_stride_b=64, ema_final=0x900000 + 4 * 128, final_stride_b=64), True),
+    (dict(ema_init=0x10000 + 4 * 511 * 64, init_stride_b=512 * 64), False),   # the last row of out
+    (dict(ema_init=0x900000, init_stride_b=64, x_norm=0x900000, xn_stride_s=64, xn_stride_b=512 * 64), False),
+])
+def test_lut_scan_is_kept_from_outputs_in_place_of_inputs(kw, scan):
+    """The scan's tiles read the initial state, and x, at different times: with
+    an output in the same memory the walk (no workspace) serves the call."""
+    base = dict(S=512, x_stride_b=512 * 64, out_stride_b=512 * 64, ema_momentum=0.9, K=8)
+    n = nat.load().osm_lut_fwd_workspace_bytes(ctypes.byref(_lut(**{**base, **kw})))
+    assert (n > 0) == scan
+
+
 def test_lut_fwd_empty_batch_is_a_no_op():
     # B = 0 returns before any pointer is looked at (no GPU work)
     lib = nat.load()

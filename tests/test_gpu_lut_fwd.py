@@ -142,6 +142,17 @@ def test_scan_and_walk_agree_around_the_first_clamp(dev, monkeypatch, B, S, H, h
         assert rel(s, w.double().cpu().numpy()) <= 2e-5
 
 
+def test_state_and_rows_in_place(dev):
+    """ema_final in ema_init's memory (a carry kept in one buffer), out in x's."""
+    x, c, init = (t.to(dev) for t in case(2, 3000, 4, 32, 8, seed=11, init_scale=0.5))
+    want = cheby_ema_lut_forward(x, c, n_heads=4, ema_init=init, ema_momentum=0.99)
+    state, rows = init.clone(), x.clone()
+    got = cheby_ema_lut_forward(rows, c, n_heads=4, ema_init=state, ema_momentum=0.99, ema_final=state, out=rows)
+    assert got[3] is state and got[0] is rows
+    for g, w in zip(got, want):
+        assert rel(g, w.double().cpu().numpy()) <= 2e-5
+
+
 def test_capture_without_a_workspace(dev):
     # a capture on a stream that has made no call yet
     x, c, init = (t.to(dev) for t in case(2, 700, 2, 32, 8, seed=3, init_scale=0.5))

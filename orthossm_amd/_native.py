@@ -357,10 +357,11 @@ def load_ext():
     return _ext
 
 
-# The functions osm_torch takes by address, in the order of its init().
+# The functions osm_torch takes by address, in the order of its init() (the
+# last one the HIP runtime's, which the library links against).
 EXT_FUNCTIONS = ("osm_workspace_bytes", "osm_cheby_ema_fwd", "osm_cheby_ema_ttt", "osm_cheby_ema_bwd",
                  "osm_v10_chunked_ttt", "osm_v10_bwd", "osm_lut_fwd_workspace_bytes", "osm_cheby_ema_lut_fwd_ws",
-                 "osm_engine_scratch_bytes", "osm_engine_prologue")
+                 "osm_engine_scratch_bytes", "osm_engine_prologue", "hipStreamIsCapturing")
 
 
 def check(rc: int) -> None:

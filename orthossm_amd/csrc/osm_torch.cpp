@@ -36,6 +36,7 @@ struct Lib {
   decltype(&osm_cheby_ema_lut_fwd_ws) lut_ws;
   decltype(&osm_engine_scratch_bytes) engine_bytes;
   decltype(&osm_engine_prologue) engine;
+  int (*stream_is_capturing)(void* stream, int* status);   // hipStreamIsCapturing
 } lib;
 PyObject* raw_stream = nullptr;   // device index -> raw stream handle
 PyObject* ws_cache = nullptr;     // {(device index, stream, op): uint8 tensor}
@@ -101,16 +102,19 @@ bool stream_of(const at::Tensor& x, Ref* obj, void** stream) {
   return !PyErr_Occurred();
 }
 
-// The workspace of (device, stream, op), from the module's cache or made by
-// its _workspace; false with a Python error set.
-bool get_workspace(PyObject* x_obj, const at::Tensor& x, PyObject* stream, size_t need, int op, at::Tensor* ws) {
+// The workspace of (device, stream, op), from the module's cache or, where it
+// is to be made or a graph is to hold it, by its _workspace; false with a Python
+// error set.
+bool get_workspace(PyObject* x_obj, const at::Tensor& x, PyObject* stream, void* raw, size_t need, int op,
+                   at::Tensor* ws) {
   PyObject* key = Py_BuildValue("(iOi)", (int)x.get_device(), stream, op);
   if (!key) return false;
   PyObject* hit = PyDict_GetItemWithError(ws_cache, key);
   Py_DECREF(key);
   if (hit && THPVariable_Check(hit) && (size_t)THPVariable_Unpack(hit).numel() >= need) {
     *ws = THPVariable_Unpack(hit);
-    return true;
+    int status = 0;
+    if (lib.stream_is_capturing(raw, &status) == 0 && status == 0) return true;
   }
   if (PyErr_Occurred()) return false;
   PyObject* dev = PyObject_GetAttrString(x_obj, "device");
@@ -255,7 +259,7 @@ PyObject* run_forward(PyObject* const* p, bool ttt) {
   const int op = ttt ? OSM_OP_TTT : OSM_OP_FWD;
   const size_t need = lib.workspace_bytes(&c.a, op);
   if (need == 0) Py_RETURN_NONE;   // refused: the Python path says why
-  const bool have = get_workspace(p[0], x, s_obj.o, need, op, &ws);
+  const bool have = get_workspace(p[0], x, s_obj.o, stream, need, op, &ws);
   if (!have) return nullptr;
   int rc;
   {
@@ -315,7 +319,7 @@ PyObject* run_backward(PyObject* const* p) {
   b.gx_stride_s = gx.stride(1);
   if (need_c) b.grad_coeffs = fptr(gc);
   if (need_i) b.grad_init = fptr(gi);
-  const bool have = get_workspace(p[0], x, s_obj.o, need, OSM_OP_BWD, &ws);
+  const bool have = get_workspace(p[0], x, s_obj.o, stream, need, OSM_OP_BWD, &ws);
   if (!have) return nullptr;
   int rc;
   {
@@ -541,7 +545,7 @@ PyObject* run_lut(PyObject* const* p) {
   a.ema_final = fptr(fin);
   a.final_stride_b = fin.stride(0);
   const size_t need = lib.lut_bytes(&a);
-  if (need && !get_workspace(p[0], x, s_obj.o, need, kOpLut, &ws)) return nullptr;
+  if (need && !get_workspace(p[0], x, s_obj.o, stream, need, kOpLut, &ws)) return nullptr;
   int rc;
   {
     const NoGil nogil;
@@ -625,16 +629,16 @@ PyObject* py_v10_backward(PyObject*, PyObject* const* a, Py_ssize_t n) { return 
 PyObject* py_lut(PyObject*, PyObject* const* a, Py_ssize_t n) { return guarded<10>(a, n, run_lut); }
 PyObject* py_engine(PyObject*, PyObject* const* a, Py_ssize_t n) { return guarded<9>(a, n, run_engine); }
 
-// init(addresses of the ten library functions, raw_stream, ws_cache, workspace, check)
+// init(addresses of the eleven library functions, raw_stream, ws_cache, workspace, check)
 PyObject* py_init(PyObject*, PyObject* args) {
   PyObject *addr, *rs, *wc, *wf, *ck;
   if (!PyArg_ParseTuple(args, "O!OO!OO", &PyTuple_Type, &addr, &rs, &PyDict_Type, &wc, &wf, &ck)) return nullptr;
-  void* f[10];
-  if (PyTuple_GET_SIZE(addr) != 10) {
-    PyErr_SetString(PyExc_ValueError, "ten addresses are expected");
+  void* f[11];
+  if (PyTuple_GET_SIZE(addr) != 11) {
+    PyErr_SetString(PyExc_ValueError, "eleven addresses are expected");
     return nullptr;
   }
-  for (int i = 0; i < 10; ++i) f[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addr, i));
+  for (int i = 0; i < 11; ++i) f[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addr, i));
   if (PyErr_Occurred()) return nullptr;
   lib.workspace_bytes = reinterpret_cast<decltype(lib.workspace_bytes)>(f[0]);
   lib.fwd = reinterpret_cast<decltype(lib.fwd)>(f[1]);
@@ -646,6 +650,7 @@ PyObject* py_init(PyObject*, PyObject* args) {
   lib.lut_ws = reinterpret_cast<decltype(lib.lut_ws)>(f[7]);
   lib.engine_bytes = reinterpret_cast<decltype(lib.engine_bytes)>(f[8]);
   lib.engine = reinterpret_cast<decltype(lib.engine)>(f[9]);
+  lib.stream_is_capturing = reinterpret_cast<decltype(lib.stream_is_capturing)>(f[10]);
   PyObject** slots[4] = {&raw_stream, &ws_cache, &workspace, &check};
   PyObject* vals[4] = {rs, wc, wf, ck};
   for (int i = 0; i < 4; ++i) {

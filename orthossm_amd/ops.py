@@ -28,6 +28,10 @@ from . import _native as nat
 
 _ws_lock = threading.Lock()
 _ws_cache: dict[tuple[int, int, int], torch.Tensor] = {}
+# Workspaces whose address a captured graph holds: the keys whose current one
+# does, and those that a larger one has replaced since (see _workspace).
+_ws_in_graph: set[tuple[int, int, int]] = set()
+_ws_kept: list[tuple[tuple[int, int, int], torch.Tensor]] = []
 
 # With fault checks on (environment OSM_CHECK_FAULTS=1, or set_fault_check),
 # every launch that uses a workspace is followed by a read of the workspace's
@@ -102,7 +106,7 @@ def workspace_faults(reset: bool = True) -> list[tuple[tuple[int, int, int], int
     stream a workspace was made for may no longer exist).  ``reset`` clears
     the words it reports."""
     with _ws_lock:
-        items = list(_ws_cache.items())
+        items = list(_ws_cache.items()) + _ws_kept
     bad = []
     for key, ws in items:
         torch.cuda.synchronize(ws.device)
@@ -130,6 +134,17 @@ def _current_stream(dev: torch.device) -> int:
     if _raw_stream is not None:
         return _raw_stream(dev.index if dev.index is not None else torch.cuda.current_device())
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+# Whether the current stream of the current device is being captured.
+_current_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
+
+
+def _capturing(dev: torch.device) -> bool:
+    if dev.index is None or dev.index == torch.cuda.current_device():
+        return _current_capturing()
+    with torch.cuda.device(dev):
+        return _current_capturing()
 
 
 # The native launch path (csrc/osm_torch.cpp) and the library it was
@@ -170,15 +185,29 @@ def _workspace(device: torch.device, stream: int, nbytes: int, op: int) -> torch
     """Zero-initialised workspace reused per (device, stream, entry point).
     Calls on one stream are ordered, so they never overlap on a workspace;
     one workspace per entry point keeps its layout fixed across alternating
-    forward/backward calls (a layout change costs a clear)."""
+    forward/backward calls (a layout change costs a clear).
+
+    A graph holds the address of the workspace that its capture used, so that
+    one is never freed; the one that replaces it is at least twice its size, so
+    those kept stay smaller together than the one in use.  A capture that finds
+    none large enough gets memory of the graph, cleared in every replay."""
     key = (device.index, stream, op)
+    capturing = _capturing(device)
     with _ws_lock:
         ws = _ws_cache.get(key)
         if ws is None or ws.numel() < nbytes:
+            if capturing:
+                return torch.zeros(nbytes, dtype=torch.uint8, device=device)
             size = max(nbytes, 1 << 20)
+            if key in _ws_in_graph:
+                _ws_in_graph.discard(key)
+                _ws_kept.append((key, ws))
+                size = max(size, 2 * ws.numel())
             size = (size + (1 << 20) - 1) & ~((1 << 20) - 1)
             ws = torch.zeros(size, dtype=torch.uint8, device=device)
             _ws_cache[key] = ws
+        elif capturing:
+            _ws_in_graph.add(key)
         return ws
 
 
@@ -700,7 +729,7 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
     if x.device.type != "cuda":
         raise RuntimeError("orthossm_amd runs on a ROCm GPU only; x is on " + str(x.device))
     dev = x.device
-    capturing = torch.cuda.is_current_stream_capturing()
+    capturing = _capturing(dev)
     fast = None if capturing else _fast()
     if fast is not None and lut is None and out is None and x_norm is None and tanh_y is None and \
             ema_final is None and coeffs.dim() == 4 and coeffs.shape[1] == n_heads:
@@ -761,9 +790,7 @@ def cheby_ema_lut_forward(x: torch.Tensor, coeffs: torch.Tensor, *, n_heads: int
         a.tanh_y, a.ty_stride_b, a.ty_stride_s = tanh_y.data_ptr(), tanh_y.stride(0), tanh_y.stride(1)
     a.ema_final, a.final_stride_b = ema_final.data_ptr(), ema_final.stride(0)
     stream = _current_stream(dev)
-    # A graph would keep the address of a workspace that a later, larger call
-    # replaces, and share it with eager calls: a capture takes the walk over
-    # the tiles, which needs none.
+    # A capture takes the walk over the tiles, which needs no workspace.
     nbytes = 0 if capturing else lib.osm_lut_fwd_workspace_bytes(ctypes.byref(a))
     if nbytes:
         a.flags |= _test_flags()

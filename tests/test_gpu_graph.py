@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from helpers import inputs, to_dev
-from orthossm_amd import cheby_ema_backward, cheby_ema_forward, cheby_ema_ttt
+from orthossm_amd import cheby_ema_backward, cheby_ema_forward, cheby_ema_ttt, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -93,6 +93,56 @@ def test_backward_graph_replays_match_eager(dev):
         torch.cuda.synchronize()
         for got, w, what in zip((gx, gc, gi), want, ("grad_x", "grad_coeffs", "grad_init")):
             assert torch.equal(got, w), f"replay {i} {what}"
+
+
+def _three_calls(dev, seed):
+    """{name: call} of the forward, TTT and backward on one set of inputs, and
+    the same calls on a shape whose workspaces are many times larger."""
+    small, big = (to_dev(inputs(B, S, 8, 64, seed=seed), dev) for B, S in ((1, 2000), (8, 16384)))
+
+    def calls(d):
+        args = (d["x"], d["coeffs"], d["damping"], d["lam"])
+        out = cheby_ema_forward(*args)
+        go = torch.ones_like(out)
+        return dict(forward=lambda: (cheby_ema_forward(*args),), ttt=lambda: cheby_ema_ttt(*args),
+                    backward=lambda: cheby_ema_backward(*args, out, go, need_init=True))
+
+    return calls(small), calls(big)
+
+
+@pytest.mark.parametrize("name", ["forward", "ttt", "backward"])
+@pytest.mark.parametrize("warm", [True, False])
+def test_graph_outlives_the_workspace_of_its_stream(dev, name, warm):
+    """After a capture, eager calls on the capture stream grow that stream's
+    workspace and other tensors take what memory is free; the replays still
+    match and touch none of it.  Also for a capture with no call before it."""
+    small, big = _three_calls(dev, 41)
+    want = [t.clone() for t in small[name]()]
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        if warm:
+            small[name]()
+            stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            got = small[name]()
+        for i in range(3):
+            eager = big[name]() if i else small[name]()
+            filled = [torch.full((n,), 3.0, device=dev) for n in (1 << 18, 1 << 20, 1 << 22)]
+            for t in got:
+                t.fill_(float("nan"))
+            graph.replay()
+            stream.synchronize()
+            assert all((f == 3.0).all() for f in filled)
+            for g, w in zip(got, want):
+                assert torch.equal(g, w), f"replay {i}"
+            if i == 0:
+                for g, w in zip(eager, want):
+                    assert torch.equal(g, w)
+    kept = [ws.numel() for key, ws in ops._ws_kept if key[1] == stream.cuda_stream]
+    assert sum(kept) <= sum(ws.numel() for key, ws in ops._ws_cache.items() if key[1] == stream.cuda_stream)
+    assert ops.workspace_faults() == []
 
 
 def test_full_path_graph_replays_match_eager(dev):

@@ -583,22 +583,22 @@ PyObject* run_engine(PyObject* const* p) {
   void* stream;
   const c10::DeviceGuard guard(x.device());
   if (!stream_of(x, &s_obj, &stream)) return nullptr;
-  at::Tensor xn, scratch, small;
+  at::Tensor xn, scratch, gate, mu;
   int rc;
   {
     const NoGil nogil;
     xn = empty({a.B, a.S, a.D}, x, at::kFloat);
     scratch = empty({(int64_t)(lib.engine_bytes(a.B, a.S, a.D) / 4)}, x, at::kFloat);
-    small = empty({a.B + 1}, x, at::kFloat);
+    gate = empty({a.B, 1}, x, at::kFloat);
+    mu = empty({}, x, at::kFloat);
     a.x_normed = fptr(xn);
     a.scratch = fptr(scratch);
-    a.gate = fptr(small);
-    a.ema_momentum = fptr(small) + a.B;
+    a.gate = fptr(gate);
+    a.ema_momentum = fptr(mu);
     rc = lib.engine(&a, stream);
   }
   if (rc != OSM_OK) return fail_rc(rc);
-  return Py_BuildValue("(NNN)", THPVariable_Wrap(xn), THPVariable_Wrap(small.narrow(0, 0, a.B).view({a.B, 1})),
-                       THPVariable_Wrap(small.select(0, a.B)));
+  return Py_BuildValue("(NNN)", THPVariable_Wrap(xn), THPVariable_Wrap(gate), THPVariable_Wrap(mu));
 }
 
 // Runs a function under the argument count and the C++ exceptions of ATen.

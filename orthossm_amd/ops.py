@@ -684,8 +684,8 @@ def engine_prologue(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w1: 
     B, S, D = x.shape
     xn = torch.empty((B, S, D), device=dev, dtype=torch.float32)
     scratch = torch.empty(lib.osm_engine_scratch_bytes(B, S, D) // 4, device=dev, dtype=torch.float32)
-    small = torch.empty(B + 1, device=dev, dtype=torch.float32)
-    gate, mu = small[:B].view(B, 1), small[B]
+    gate = torch.empty((B, 1), device=dev, dtype=torch.float32)
+    mu = torch.empty((), device=dev, dtype=torch.float32)
     a = nat.EngineArgs()
     a.abi_version, a.eps = nat.ABI_VERSION, float(eps)
     a.B, a.S, a.D = B, S, D

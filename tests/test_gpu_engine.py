@@ -19,6 +19,7 @@ from oracle import v10_full as V
 
 from orthossm_amd import apply_cheby_rkv_v10
 from orthossm_amd import engine as E
+from orthossm_amd import ops
 from orthossm_amd.ops import cheby_ema_forward, head_momentum, v10_chunked_ttt
 from orthossm_amd.sdpc_kernel import v10_damping
 
@@ -246,6 +247,28 @@ def test_prologue_matches_module_calls(dev, B, S, D_):
         assert (xn - wn).abs().max() <= 2e-6 * wn.abs().max()
         wg = m.complexity_gate.double()(wn.mean(1))
         assert gate.shape == wg.shape and (gate - wg).abs().max() <= 1e-5
+
+
+@pytest.mark.parametrize("checks", [False, True])     # the native launch, and the Python one
+def test_prologue_results_are_tensors_of_their_own(dev, checks):
+    """gate and ema_momentum of a continued call, as a program may use them
+    after it: written in place with an operand that carries gradients, each
+    without touching the other."""
+    old = ops.set_fault_check(checks)
+    try:
+        m = make(dev, seed=3)
+        c = torch.randn(2, H, K, D // H, generator=torch.Generator().manual_seed(1)).to(dev) * 0.3
+        with torch.no_grad():
+            r = m(torch.randn(2, 64, D, device=dev), (c, torch.zeros_like(c)))
+    finally:
+        ops.set_fault_check(old)
+    assert not r.gate._is_view() and not r.ema_momentum._is_view()
+    mu, version = r.ema_momentum.clone(), r.ema_momentum._version
+    w = torch.ones((), device=dev, requires_grad=True)
+    r.gate.mul_(w)
+    r.gate.sum().backward()
+    assert torch.isfinite(w.grad)
+    assert torch.equal(r.ema_momentum, mu) and r.ema_momentum._version == version
 
 
 def test_fused_and_module_prologue_agree_on_every_route(dev):

@@ -10,7 +10,11 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sys
 import threading
+import warnings
+
+import torch
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libosm.so")
 
@@ -341,20 +345,33 @@ _ext = None
 
 
 def load_ext():
-    """The extension module ``osm_torch`` (csrc/osm_torch.cpp), imported once."""
+    """The extension module ``osm_torch`` (csrc/osm_torch.cpp), or None, with
+    one warning, where it is missing or was built for another torch or Python:
+    every launch then goes through ctypes, at more host time."""
     global _ext
     if _ext is None:
         with _lock:
             if _ext is None:
-                if not os.path.exists(EXT_PATH):
-                    raise ImportError(f"orthossm_amd: extension {EXT_PATH} is missing; build it with "
-                                      "`python -m orthossm_amd.build`.")
-                loader = importlib.machinery.ExtensionFileLoader("osm_torch", EXT_PATH)
-                spec = importlib.util.spec_from_file_location("osm_torch", EXT_PATH, loader=loader)
-                mod = importlib.util.module_from_spec(spec)
-                loader.exec_module(mod)
-                _ext = mod
-    return _ext
+                try:
+                    _ext = _import_ext()
+                except ImportError as e:
+                    _ext = False
+                    warnings.warn(f"orthossm_amd: launching through ctypes ({e}); `python -m orthossm_amd.build` "
+                                  "builds the extension for this torch and Python", RuntimeWarning, stacklevel=2)
+    return _ext or None
+
+
+def _import_ext():
+    if not os.path.exists(EXT_PATH):
+        raise ImportError(f"{EXT_PATH} is missing")
+    loader = importlib.machinery.ExtensionFileLoader("osm_torch", EXT_PATH)
+    spec = importlib.util.spec_from_file_location("osm_torch", EXT_PATH, loader=loader)
+    mod = importlib.util.module_from_spec(spec)
+    loader.exec_module(mod)
+    have = (torch.__version__.split("+")[0], sys.hexversion >> 16)
+    if mod.built_for != have:
+        raise ImportError(f"{EXT_PATH} was built for torch and Python {mod.built_for}, these are {have}")
+    return mod
 
 
 # The functions osm_torch takes by address, in the order of its init() (the

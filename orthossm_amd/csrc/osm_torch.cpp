@@ -18,6 +18,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "osm.h"
 
@@ -682,4 +683,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "osm_torch", nullptr, -1, methods, 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_osm_torch(void) { return PyModule_Create(&module); }
+// built_for: the torch version and the Python minor version of the build.
+PyMODINIT_FUNC PyInit_osm_torch(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddObject(m, "built_for", Py_BuildValue("(si)", TORCH_VERSION, PY_VERSION_HEX >> 16)) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -157,15 +157,17 @@ _DTYPE_CODE = {None: None, torch.float32: nat.F32, torch.bfloat16: nat.BF16}
 
 def _fast():
     """The native launch path, or None where the Python path has to run: with
-    fault checks on, or a library object that is not the loaded one."""
+    fault checks on, a library object that is not the loaded one, or without
+    the extension."""
     global _ext, _ext_for
     lib = nat.load()
     if _ext_for is not lib:
         if _raw_stream is None or not isinstance(lib, ctypes.CDLL):
             return None
         ext = nat.load_ext()
-        ext.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in nat.EXT_FUNCTIONS), _raw_stream,
-                 _ws_cache, _workspace, nat.check)
+        if ext is not None:
+            ext.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in nat.EXT_FUNCTIONS), _raw_stream,
+                     _ws_cache, _workspace, nat.check)
         _ext, _ext_for = ext, lib
     return None if _check_faults else _ext
 

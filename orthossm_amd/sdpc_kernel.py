@@ -45,8 +45,8 @@ import threading
 import torch
 import torch.nn as nn
 
-from .ops import (LUT_POINTS, LUT_TERMS, V10_LION_LAMBDA, cheby_ema, cheby_ema_forward, cheby_ema_lut_forward,
-                  chebyshev_lut_table, head_momentum, v10_chunked_ttt, v10_full_path)
+from .ops import (LUT_POINTS, LUT_TERMS, V10_LION_LAMBDA, _capturing, _current_stream, cheby_ema, cheby_ema_forward,
+                  cheby_ema_lut_forward, chebyshev_lut_table, head_momentum, v10_chunked_ttt, v10_full_path)
 
 # Points of the full path's half-table LUT and the number of Chebyshev terms
 # it holds (sdpc_kernel.py:58-59).
@@ -135,40 +135,44 @@ def v10_damping(n_heads: int, device=None) -> torch.Tensor:
     return 0.98 - 0.06 * h / n_heads
 
 
-# The fast path's per-head damping and lambda tensors, built once per
-# (device, heads) and (device, heads, momentum) instead of on every call (a
-# call with small inputs otherwise spends most of its host time building
-# them).  Entries are never dropped (a cached tensor may still be read by a
-# launch on another stream); past _CONST_CACHE_MAX entries new values are
-# built per call instead.
+# The fast path's per-head damping, and damping and lambda, built once per
+# (device, stream, heads) and (device, stream, heads, momentum) instead of on
+# every call (a call with small inputs otherwise spends most of its host time
+# building them).  The stream that built one has it ready; another might read
+# it before.  None is kept from a capture, whose kernels run in replays only.
+# Entries are never dropped (a graph may hold one); past _CONST_CACHE_MAX
+# entries new values are built per call instead.
 _const_lock = threading.Lock()
 _const_cache: dict = {}
 _CONST_CACHE_MAX = 64
 
 
+def _keep_constant(key, val, dev: torch.device):
+    """``val``, kept under ``key`` if there is room and no capture; or the entry
+    another thread has made."""
+    if dev.type == "cuda" and _capturing(dev):
+        return val
+    with _const_lock:
+        return _const_cache.setdefault(key, val) if len(_const_cache) < _CONST_CACHE_MAX else val
+
+
 def _fast_constants(n_heads: int, device: torch.device, ema_momentum):
     """(damping [H], lam [H]) fp32 on ``device`` for the fast path; a tensor
     ``ema_momentum`` (on the device, not read back) is expanded per call."""
-    dev = torch.device(device)
-    dkey = ("damping", dev, n_heads)
-    if isinstance(ema_momentum, torch.Tensor):
-        lkey = None
-    else:
-        lkey = ("lam", dev, n_heads, float(ema_momentum))
-    with _const_lock:
-        damping = _const_cache.get(dkey)
-        lam = _const_cache.get(lkey) if lkey is not None else None
-    if damping is not None and lam is not None:
-        return damping, lam
+    dev = device if type(device) is torch.device else torch.device(device)
+    stream = _current_stream(dev) if dev.type == "cuda" else 0
+    fixed = not isinstance(ema_momentum, torch.Tensor)
+    if fixed:
+        key = (dev, stream, n_heads, float(ema_momentum))
+        both = _const_cache.get(key)
+        if both is not None:
+            return both
+    dkey = (dev, stream, n_heads)
+    damping = _const_cache.get(dkey)
     if damping is None:
-        damping = v10_damping(n_heads, dev)
-    if lam is None:
-        lam = head_momentum(ema_momentum, n_heads, dev)
-    with _const_lock:
-        for key, val in ((dkey, damping), (lkey, lam)):
-            if key is not None and len(_const_cache) < _CONST_CACHE_MAX:
-                _const_cache.setdefault(key, val)
-    return damping, lam
+        damping = _keep_constant(dkey, v10_damping(n_heads, dev), dev)
+    both = damping, head_momentum(ema_momentum, n_heads, dev)
+    return _keep_constant(key, both, dev) if fixed else both
 
 
 def apply_cheby_rkv_v10(x, coeffs, momentum_buf, n_heads=4, base_lr=0.005, ema_momentum=0.9,

@@ -145,6 +145,47 @@ def test_graph_outlives_the_workspace_of_its_stream(dev, name, warm):
     assert ops.workspace_faults() == []
 
 
+def test_first_use_in_a_capture_leaves_later_eager_calls_right(dev):
+    """The engine's fast path with a carried state and the drop-in, first used
+    in a capture (seven heads, a momentum of its own): eager calls before any
+    replay, on the capture stream and on another, and the replays match."""
+    from orthossm_amd import ChebyContextPath, ChebyState, apply_cheby_rkv_v10
+    H, hd, S = 7, 12, 50
+    torch.manual_seed(1)
+    path = ChebyContextPath(H * hd, n_cheby_heads=H, max_degree=4, carry_ema=True).to(dev).eval()
+    x = torch.randn(2, S, H * hd, device=dev)
+    c = torch.randn(2, H, 4, hd, device=dev) * 0.3
+    state = ChebyState(c, torch.zeros_like(c), torch.full((2, H * hd), 0.2, device=dev))
+
+    def step():
+        with torch.no_grad():
+            path.total_tokens_seen.zero_()
+            r = path(x, state)
+            return r.out, apply_cheby_rkv_v10(x, c, None, n_heads=H, ema_momentum=0.8125)[0]
+
+    lam = path.ema_base.new_full((H,), 0.8125)
+    damp = torch.tensor([0.98 - 0.06 * h / H for h in range(H)], device=dev)
+    want = cheby_ema_forward(x, c, damp, lam, nan_policy="zero_u")
+    torch.cuda.synchronize()
+    cap, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=cap):
+        got = step()
+    eager = []
+    for s in (cap, other):
+        with torch.cuda.stream(s):
+            eager.append(step())
+    torch.cuda.synchronize()
+    for out, fast in eager:
+        torch.testing.assert_close(fast, want, rtol=1e-5, atol=1e-6)
+        assert torch.equal(out, eager[0][0])
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        for g, w in zip(got, eager[0]):
+            assert torch.equal(g, w)
+
+
 def test_full_path_graph_replays_match_eager(dev):
     from orthossm_amd.ops import v10_chunked_ttt
     gen = torch.Generator().manual_seed(36)

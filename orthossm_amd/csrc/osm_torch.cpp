@@ -559,17 +559,27 @@ PyObject* run_lut(PyObject* const* p) {
   return Py_BuildValue("(NNNN)", THPVariable_Wrap(out), on, oy, THPVariable_Wrap(fin));
 }
 
-// engine(x, norm_weight, eps, w1, b1, w2, b2, ema_base, tokens_seen), all as
-// the caller has checked them: (x_normed, gate, mu).
+// engine(x, norm_weight, eps, w1, b1, w2, b2, ema_base, tokens_seen): None, or
+// (x_normed, gate, mu).
 PyObject* run_engine(PyObject* const* p) {
-  const at::Tensor& x = THPVariable_Unpack(p[0]);
+  const at::Tensor* const xp = plain(p[0]);
+  if (!xp || !xp->is_cuda() || !is_f32(*xp) || !rows(*xp, *xp) || xp->numel() == 0) Py_RETURN_NONE;
+  const at::Tensor& x = *xp;
+  const int64_t D = x.size(2), sizes[6] = {D, D / 4 * D, D / 4, D / 4, 1, 1};
+  const int at[6] = {1, 3, 4, 5, 6, 7};   // norm_weight, w1, b1, w2, b2, ema_base
+  for (int i = 0; i < 6; ++i) {
+    const at::Tensor* t = plain(p[at[i]]);
+    if (!t || !f32_flat(*t, sizes[i], x)) Py_RETURN_NONE;
+  }
+  const at::Tensor* seen = plain(p[8]);
+  if (!seen || seen->scalar_type() != at::kLong || seen->numel() != 1 || seen->device() != x.device()) Py_RETURN_NONE;
   auto ptr = [&](int i) { return fptr(THPVariable_Unpack(p[i])); };
   osm_engine_args a{};
   if (!as_float(p[2], &a.eps)) Py_RETURN_NONE;
   a.abi_version = OSM_ABI_VERSION;
   a.B = x.size(0);
   a.S = x.size(1);
-  a.D = x.size(2);
+  a.D = D;
   a.x = fptr(x);
   a.x_stride_b = x.stride(0);
   a.x_stride_s = x.stride(1);
@@ -579,7 +589,7 @@ PyObject* run_engine(PyObject* const* p) {
   a.w2 = ptr(5);
   a.b2 = ptr(6);
   a.ema_base = ptr(7);
-  a.tokens_seen = static_cast<int64_t*>(THPVariable_Unpack(p[8]).data_ptr());
+  a.tokens_seen = static_cast<int64_t*>(seen->data_ptr());
   Ref s_obj;
   void* stream;
   const c10::DeviceGuard guard(x.device());

@@ -680,10 +680,21 @@ def engine_prologue(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, w1: 
     Returns (x_normed [B,S,D], gate [B,1], mu, a 0-d tensor)."""
     fast = _fast()
     if fast is not None:
-        return fast.engine(x, norm_weight, eps, w1, b1, w2, b2, ema_base, tokens_seen)
+        res = fast.engine(x, norm_weight, eps, w1, b1, w2, b2, ema_base, tokens_seen)
+        if res is not None:
+            return res
     lib = nat.load()
+    if x.dim() != 3 or x.dtype != torch.float32 or x.device.type != "cuda" or x.stride(2) != 1 or x.numel() == 0:
+        raise ValueError("x must be a non-empty [B,S,D] float32 tensor on a ROCm device with lane stride 1")
     dev = x.device
     B, S, D = x.shape
+    for name, t, n in (("norm_weight", norm_weight, D), ("w1", w1, D // 4 * D), ("b1", b1, D // 4), ("w2", w2, D // 4),
+                       ("b2", b2, 1), ("ema_base", ema_base, 1)):
+        if t.numel() != n:
+            raise ValueError(f"{name} must have {n} entries, got {t.numel()}")
+        _check_dest(t, t.shape, dev, name)
+    if tokens_seen.dtype != torch.int64 or tokens_seen.numel() != 1 or tokens_seen.device != dev:
+        raise ValueError(f"tokens_seen must be an int64 scalar on {dev}")
     xn = torch.empty((B, S, D), device=dev, dtype=torch.float32)
     scratch = torch.empty(lib.osm_engine_scratch_bytes(B, S, D) // 4, device=dev, dtype=torch.float32)
     gate = torch.empty((B, 1), device=dev, dtype=torch.float32)

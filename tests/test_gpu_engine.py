@@ -271,6 +271,23 @@ def test_prologue_results_are_tensors_of_their_own(dev, checks):
     assert torch.equal(r.ema_momentum, mu) and r.ema_momentum._version == version
 
 
+def test_prologue_refuses_what_its_kernels_do_not_take(dev):
+    x = torch.randn(2, 10, 64, device=dev)
+    good = [x, torch.ones(64, device=dev), 1e-6, torch.randn(16, 64, device=dev), torch.zeros(16, device=dev),
+            torch.randn(1, 16, device=dev), torch.zeros(1, device=dev), torch.tensor(0.9, device=dev),
+            torch.tensor(5, device=dev)]
+    ops.engine_prologue(*good)
+    for i, bad in ((0, x.cpu()), (0, x[0]), (0, x.bfloat16()), (0, x[:, :0]), (0, x.transpose(0, 2)),
+                   (1, torch.ones(32, device=dev)), (3, good[3].bfloat16()), (3, good[3].t()), (4, good[4][:8]),
+                   (5, good[5].cpu()), (7, torch.tensor(0.9, device=dev, dtype=torch.float64)),
+                   (8, torch.tensor(5, device=dev, dtype=torch.int32)), (8, torch.tensor(5))):
+        args = list(good)
+        args[i] = bad
+        with pytest.raises(ValueError):
+            ops.engine_prologue(*args)
+    assert good[8].item() == 15
+
+
 def test_fused_and_module_prologue_agree_on_every_route(dev):
     """A continued call with and without the fused prologue (a hook on the
     norm takes it off), carry included; with gradients enabled the modules run."""

@@ -177,17 +177,18 @@ class ChebyContextPath(nn.Module):
         and nothing attached that a module call would run (hooks, autocast,
         tracing, forward-mode gradients).  Looked at afresh on every call."""
         if (torch.is_grad_enabled() or type(x) is not torch.Tensor or x.dtype is not torch.float32 or not x.is_cuda or
-                x.numel() == 0 or x.shape[0] > 65535 or x.shape[2] % 4 or x.shape[2] > ENGINE_MAX_D or
+                x.numel() == 0 or x.shape[0] > 65535 or x.shape[1] >= 1 << 30 or x.shape[2] % 4 or x.shape[2] > ENGINE_MAX_D or
                 x.stride(2) != 1 or x.stride(0) % 4 or x.stride(1) % 4 or x.data_ptr() % 16):
             return None
         if (torch.is_autocast_enabled() or torch.jit.is_tracing() or torch.compiler.is_compiling() or
                 forward_ad._current_level >= 0 or nn_module._global_forward_hooks or
                 nn_module._global_forward_pre_hooks):
             return None
-        norm, cg = self._modules["input_norm"], self._modules["complexity_gate"]
+        # (a program may have put anything in place of a submodule or buffer)
+        norm, cg = self._modules.get("input_norm"), self._modules.get("complexity_gate")
         if type(norm) is not nn.RMSNorm or type(cg) is not GatedComplexityPredictor:
             return None
-        net = cg._modules["net"]
+        net = cg._modules.get("net")
         if type(net) is not nn.Sequential or len(net) != 4:
             return None
         l1, act, l2, sig = net._modules.values()
@@ -206,7 +207,9 @@ class ChebyContextPath(nn.Module):
             if type(w) is not nn.Parameter or w.dtype is not torch.float32 or w.device != dev or \
                     w.shape != shape or not w.is_contiguous() or w.data_ptr() % 16:
                 return None
-        base, seen = self._buffers["ema_base"], self._buffers["total_tokens_seen"]
+        base, seen = self._buffers.get("ema_base"), self._buffers.get("total_tokens_seen")
+        if type(base) is not torch.Tensor or type(seen) is not torch.Tensor:
+            return None
         if base.dtype is not torch.float32 or seen.dtype is not torch.long or base.device != dev or \
                 seen.device != dev or base.numel() != 1 or seen.numel() != 1:
             return None

@@ -288,6 +288,30 @@ def test_prologue_refuses_what_its_kernels_do_not_take(dev):
     assert good[8].item() == 15
 
 
+def test_replaced_parts_take_the_module_calls(dev):
+    """A submodule or buffer that a program has put something else in place of."""
+    c = torch.randn(2, H, K, D // H, generator=torch.Generator().manual_seed(1)).to(dev) * 0.3
+    x = torch.randn(2, 64, D, device=dev)
+    state = (c, torch.zeros_like(c))
+    for swap in ("norm", "buffer"):
+        m = make(dev, seed=3)
+        with torch.no_grad():
+            want = m(x, state)
+        m.total_tokens_seen.zero_()
+        if swap == "norm":
+            norm = m.input_norm
+            del m.input_norm
+            m.input_norm = lambda t: norm(t)
+        else:
+            base = m.ema_base
+            del m.ema_base
+            m.ema_base = torch.nn.Parameter(base)
+        with torch.no_grad():
+            assert m._fused_weights(x) is None
+            got = m(x, state)
+        torch.testing.assert_close(got.out, want.out, rtol=1e-5, atol=2e-6)
+
+
 def test_fused_and_module_prologue_agree_on_every_route(dev):
     """A continued call with and without the fused prologue (a hook on the
     norm takes it off), carry included; with gradients enabled the modules run."""

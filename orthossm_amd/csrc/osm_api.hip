@@ -507,6 +507,12 @@ size_t osm_workspace_bytes(const osm_cheby_args* args, int op) {
   }
   Geometry geo;
   if (check_args(args, &geo, op, /*shapes_only=*/true) != OSM_OK) return 0;
+  // The TTT's short tiles give a shorter sequence more tiles than a longer one
+  // may have: room for the most that any B and S up to these have.
+  if (op == OSM_OP_TTT && !geo.empty) {
+    const int64_t t = (args->S + osm::TttTileSmall::TILE - 1) / osm::TttTileSmall::TILE;
+    geo.n_tiles = std::max(geo.n_tiles, (int)std::min<int64_t>(t, osm::kDirectTiles));
+  }
   return ws_bytes_for(geo, op, (int)args->K);
 }
 

@@ -92,6 +92,20 @@ def test_workspace_bytes_formula():
     assert lib.osm_workspace_bytes(ctypes.byref(a), 0) == 0
 
 
+@pytest.mark.parametrize("g", [0, 0x10000])
+def test_ttt_workspace_of_a_longer_sequence_serves_shorter_ones(g):
+    lib = nat.load()
+
+    def need(B, S):
+        return lib.osm_workspace_bytes(ctypes.byref(_args(B=B, S=S, H=4, hd=32, K=8, g=g)), 1)
+
+    lengths = [1, 128, 129, 192, 193, 2000, 4095, 4096, 4097, 4224, 4225, 5000, 6144, 6145, 8192, 20000]
+    for B in (1, 2, 5, 8, 16, 40, 130):
+        sizes = [need(B, S) for S in lengths]
+        assert sizes == sorted(sizes), B
+        assert all(need(B, S) >= need(max(B - 1, 1), S) for S in lengths)
+
+
 def test_workspace_bytes_without_pointers():
     """A shapes-only forward query with x or out NULL does not know their
     alignment and is sized for the one-lane geometry (128-token tiles), the

@@ -160,7 +160,7 @@ typedef struct osm_cheby_args {
   float lam_shift, lam_min, lam_max;
 
   const float* ema_init;    /* optional [B, H*hd] fp32 contiguous */
-  float* ema_final;         /* optional [B, H*hd] fp32 contiguous */
+  float* ema_final;         /* optional [B, H*hd] fp32 contiguous; may be ema_init */
 } osm_cheby_args;
 
 /*

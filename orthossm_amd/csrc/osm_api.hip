@@ -152,6 +152,24 @@ int check_args(const osm_cheby_args* a, Geometry* geo, int op, bool shapes_only 
   return OSM_OK;
 }
 
+// Bytes that [B,S,D] rows of `size` bytes an element lie in; none for a NULL.
+struct Span {
+  uintptr_t lo = 0, hi = 0;
+  Span(const void* p, int64_t sb, int64_t ss, int64_t B, int64_t S, int64_t D, int size) {
+    if (!p || B < 1 || S < 1) return;
+    lo = (uintptr_t)p;
+    hi = lo + (uintptr_t)((B - 1) * sb + (S - 1) * ss + D) * (uintptr_t)size;
+  }
+  bool meets(const Span& o) const { return lo < o.hi && o.lo < hi; }
+};
+
+// Whether a [B,D] state that a launch reads lies in memory that it writes: the
+// other state, or rows.
+bool in_place(const float* state, const float* other, const Span& rows, int64_t B, int64_t D) {
+  const Span s(state, D, 0, B, 1, D, 4);
+  return s.meets(Span(other, D, 0, B, 1, D, 4)) || s.meets(rows);
+}
+
 osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* ws) {
   osm::FwdParams p{};
   p.x = a->x;
@@ -184,7 +202,11 @@ osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* w
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
-  p.order = osm::tile_order(geo.n_lb, geo.n_tiles);
+  p.order = osm::tile_order(geo.n_lb, geo.n_tiles,
+                            in_place(a->ema_init, a->ema_final,
+                                     Span(a->out, a->out_stride_b, a->out_stride_s, a->B, a->S, a->H * a->hd,
+                                          a->out_dtype == OSM_F32 ? 4 : 2),
+                                     a->B, a->H * a->hd));
   p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.lam_shift = a->lam_shift;
   p.lam_min = a->lam_min;
@@ -413,17 +435,6 @@ int run_lut_walk(const osm_lut_fwd_args* a, void* stream) {
   if (e != hipSuccess) return hip_fail(e, "fixed-coefficient forward launch");
   return ok();
 }
-
-// Bytes that [B,S,D] rows of `size` bytes an element lie in; none for a NULL.
-struct Span {
-  uintptr_t lo = 0, hi = 0;
-  Span(const void* p, int64_t sb, int64_t ss, int64_t B, int64_t S, int64_t D, int size) {
-    if (!p || B < 1 || S < 1) return;
-    lo = (uintptr_t)p;
-    hi = lo + (uintptr_t)((B - 1) * sb + (S - 1) * ss + D) * (uintptr_t)size;
-  }
-  bool meets(const Span& o) const { return lo < o.hi && o.lo < hi; }
-};
 
 // Whether an output of the table forward lies in memory that it reads: the
 // initial state, or x other than element for element.  The walk reads a lane
@@ -958,6 +969,10 @@ int osm_cheby_ema_bwd(const osm_cheby_args* args, const osm_cheby_bwd_args* bwd,
   if (rc != OSM_OK) return rc;
   osm::BwdParams bp{};
   bp.f = make_params(args, geo, workspace);
+  bp.f.order = osm::tile_order(geo.n_lb, geo.n_tiles,
+                               in_place(bwd->grad_state, bwd->grad_init,
+                                        Span(bwd->grad_x, bwd->gx_stride_b, bwd->gx_stride_s, args->B, args->S, D, xs),
+                                        args->B, D));
   bp.f.partials = reinterpret_cast<float*>(static_cast<char*>(workspace) + ((slot_bytes + 255) / 256) * 256);
   bp.gout = bwd->grad_out;
   bp.go_sb = bwd->go_stride_b;

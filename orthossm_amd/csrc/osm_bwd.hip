@@ -306,9 +306,9 @@ cheby_ema_bwd_kernel(const BwdParams bp) {
     const float init_c =
         (bp.grad_state && q.wave < G::NSUB && dc < p.D) ? bp.grad_state[(int64_t)ti.b * p.D + dc] : 0.0f;
     LookBack<G, true> lbk;
-    look_back_issue<G, true>(lbk, q, ti, ls);
+    look_back_issue<G, true>(lbk, q, ti, ls, kWordsShift<G>, group_min<SPREAD>(p.order, ti));
     jitter(p.jitter, tags.epoch, 1);
-    look_back_finish<G, true>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, 0.0f, p.hdr, p.poll_limit);
+    look_back_finish<G, true, SPREAD>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, 0.0f, p.hdr, p.poll_limit);
   }
   float v = __builtin_fmaf(pA, L.carry[q.lt], pB[0]);
 

@@ -132,6 +132,7 @@ __device__ __forceinline__ TileInfo tile_info(const TileOrder& order, unsigned* 
   ti.lbd = ti.lb - ti.b * n_lbd;
   ti.is_last = ti.tile == n_tiles - 1;
   ti.is_ckpt = ((ti.tile + 1) & ((G::WPS << wsh) - 1)) == 0;
+  if constexpr (SPREAD) ti.is_ckpt |= order.lead && ti.tile == 0;
   return ti;
 }
 
@@ -258,7 +259,8 @@ __device__ __forceinline__ void look_back_issue(LookBack<G, DYN>& st, const Thre
 // AL: the type in which a thread's words compose; double where a launch may
 // choose several per thread (rounded once; in fp32 the longer composition
 // raised the error of a long carry chain by half).
-template <class G, bool DYN, typename AL>
+// LEAD: the first tile may be a checkpoint (TileOrder::lead).
+template <class G, bool DYN, bool LEAD, typename AL>
 __device__ __forceinline__ void look_back_finish(LookBack<G, DYN>& st, ChainLds<G>& L, const ThreadPos& q,
                                                  const TileInfo& ti, const Tags& tg, float aggA, float aggB,
                                                  const LaneSlots& ls, float init_carry, AL a_look,
@@ -301,6 +303,8 @@ __device__ __forceinline__ void look_back_finish(LookBack<G, DYN>& st, ChainLds<
     }
   } else if (q.wave < G::NSUB) {
     L.carry[carry_lane<G>(q)] = init_carry;
+    if (LEAD && ti.is_ckpt && !ti.is_last)
+      publish(ls.at(0, carry_lane<G>(q)), tg.pre, __builtin_fmaf(aggA, init_carry, aggB));
   }
   __syncthreads();
 }
@@ -363,6 +367,13 @@ __device__ __forceinline__ void finish_block(unsigned* hdr_words, unsigned epoch
 __device__ __forceinline__ void skip_block(unsigned* hdr_words, const Tags& tg, const TileInfo& ti) {
   if (ti.lb >= 0 && threadIdx.x == 0) raise_fault(hdr_words, fault_tag_of(tg.agg));
   finish_block<true>(hdr_words, tg.epoch);
+}
+
+// First tile of the look-back group of a tile after the first: its checkpoint
+// is the tile before.
+template <bool SPREAD>
+__device__ __forceinline__ int group_min(const TileOrder& order, const TileInfo& ti) {
+  return SPREAD && order.lead && ti.tile > 0 ? 1 : 0;
 }
 
 // Launches a kernel in the version of the launch's tile order: f gets

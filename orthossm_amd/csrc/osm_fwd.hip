@@ -297,9 +297,9 @@ cheby_ema_fwd_kernel(const FwdParams p) {
     AL a_look = 0;
     if constexpr (!DYN) a_look = (AL)pow_n_f64<G::TILE>((double)p.lam[dlk < p.D ? div_hd(dlk, p) : 0]);
     LookBack<G, DYN> lbk;
-    look_back_issue<G, DYN>(lbk, q, ti, ls, wsh);
+    look_back_issue<G, DYN>(lbk, q, ti, ls, wsh, group_min<SPREAD>(p.order, ti));
     jitter(p.jitter, tags.epoch, 1);
-    look_back_finish<G, DYN>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
+    look_back_finish<G, DYN, SPREAD>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
   }
   finish_complete<SPREAD>(p.hdr, tags.epoch, fin_prev);
 

@@ -174,6 +174,7 @@ struct TileOrder {
   bool spread;       // false: block v takes tile v / n_lb of slot v % n_lb
   unsigned ticket;   // spread: 0, or with tickets the share of ticket blocks as a fraction of 2^32
   int n_slots;       // spread, by index: blocks per tile row, a multiple of 8
+  bool lead;         // spread: the first tile alone reads the initial state and publishes its own end state
   Divisor by_slots, by_whole, by_rest;   // n_slots; with tickets n_lb / 8 and n_lb % 8
 };
 struct TileSlot {
@@ -228,12 +229,18 @@ __host__ __device__ __forceinline__ TileSlot spread_slot(const TileOrder& o, uns
 //   surplus 15) 29.5 and 27.7.
 // One counter for all lane-blocks made the tickets a queue (11 ns each): 21.1 us
 // for the bf16 forward above.
-inline TileOrder tile_order(int64_t n_lb, int64_t n_tiles) {
+//
+// state_in_place: the final state may be written to the initial state's memory.
+// The tiles of the first look-back group read the initial state when they
+// resolve their carry, after they have published, so the last tile may be done
+// before them; with `lead` they take the first tile's published state instead.
+inline TileOrder tile_order(int64_t n_lb, int64_t n_tiles, bool state_in_place = false) {
   constexpr int64_t kCusPerXcd = 32;
   TileOrder o{};
   o.grid = (unsigned)(n_lb * n_tiles);
-  if (n_lb % 8 == 0 || n_tiles == 1) return o;
+  if (n_tiles == 1 || (n_lb % 8 == 0 && !state_in_place)) return o;
   o.spread = true;
+  o.lead = state_in_place;
   const int64_t pad = (n_lb + 7) / 8 * 8, most = pad / 8 * n_tiles, surplus = most - n_lb * n_tiles / 8;
   if (most <= kCusPerXcd || surplus <= 12 || surplus <= most / 16) {
     o.grid = (unsigned)(pad * n_tiles);

@@ -189,7 +189,7 @@ lut_fwd_kernel(const LutScanParams p) {
     look_back_issue<G, false>(lbk, q, ti, ls, p.wsh, ti.tile > p.clamp_at ? p.clamp_at + 1 : 0);
     ti.is_ckpt = ckpt && !at_clamp;   // the clamped tile's state is published below
     jitter(p.jitter, tags.epoch, 1);
-    look_back_finish<G, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A64, p.hdr, p.poll_limit,
+    look_back_finish<G, false, false>(lbk, L, q, ti, tags, tile_A, aggB, ls, init_c, tile_A64, p.hdr, p.poll_limit,
                                kTinyDecay);
   }
   finish_complete<SPREAD>(p.hdr, tags.epoch, fin_prev);

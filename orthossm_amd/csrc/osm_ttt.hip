@@ -423,9 +423,9 @@ cheby_ema_ttt_kernel(const FwdParams p) {
     const int dlk = ti.lbd * G::LANES + look_lane<G>(q);
     const float a_look = DYN ? 0.0f : sh_pw[1][look_lane<G>(q)];
     LookBack<G, DYN> lbk;
-    look_back_issue<G, DYN>(lbk, q, ti, ls);
+    look_back_issue<G, DYN>(lbk, q, ti, ls, kWordsShift<G>, group_min<SPREAD>(p.order, ti));
     jitter(p.jitter, tags.epoch, 1);
-    look_back_finish<G, DYN>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
+    look_back_finish<G, DYN, SPREAD>(lbk, L, q, ti, tags, aggA, aggB, ls, init_c, a_look, p.hdr, p.poll_limit);
   }
 
   float y_after[LPT];

@@ -23,8 +23,9 @@ SRC = r"""
 #include <stdio.h>
 #include <vector>
 #include "osm_kernels.h"
-static int check(int n_lb, int n_tiles) {
-  const osm::TileOrder o = osm::tile_order(n_lb, n_tiles);
+static int check_order(int n_lb, int n_tiles, bool state_in_place) {
+  const osm::TileOrder o = osm::tile_order(n_lb, n_tiles, state_in_place);
+  if (o.lead != (state_in_place && n_tiles > 1) || (o.lead && !o.spread)) return printf("FAIL lead n_lb=%d\n", n_lb);
   std::vector<long long> block((size_t)n_lb * n_tiles, -1);   // by index: who takes the tile
   std::vector<int> drawn(n_lb, 0);
   for (unsigned b = 0; b < o.grid; ++b) {
@@ -53,6 +54,7 @@ static int check(int n_lb, int n_tiles) {
   }
   return 0;
 }
+static int check(int n_lb, int n_tiles) { return check_order(n_lb, n_tiles, false) || check_order(n_lb, n_tiles, true); }
 int main() {
   for (int n_lb = 1; n_lb <= 70; ++n_lb)
     for (int n_tiles : {1, 2, 3, 7, 8, 9, 31, 32, 33, 40, 127, 512, 1000})

@@ -146,7 +146,7 @@ v10_bwd_kernel(const V10BwdParams p) {
   const int lbd = item % p.n_lbd;
   const int row = item / p.n_lbd;
   const int ch = row % p.n_chunks, b = row / p.n_chunks;
-  const int t0 = ch * p.chunk, t1 = min(t0 + p.chunk, p.S);
+  const int t0 = ch * p.chunk, t1 = t0 + min(p.chunk, p.S - t0);
   const int tid = threadIdx.x, lt = tid % G::TPR, tg = tid / G::TPR;
   const int d0 = lbd * LANES + lt * LPT;
   const float mu = p.mu_dev ? *p.mu_dev : p.mu;

@@ -22,6 +22,26 @@ from orthossm_amd.synthetic import make_inputs
 
 pytestmark = pytest.mark.gpu
 
+
+def test_full_path_backward_at_the_last_tokens_of_int32(dev):
+    """dL/dx of one lane over 2^31 - 200 tokens in chunks of 2^20: the last
+    chunk's end is past what a sum of its start and the chunk length holds.
+    x = z = 0, one linear coefficient, dL/dout = 1: dL/dx is (1-mu) gamma times
+    the sum of mu^i over the tokens left in the chunk."""
+    from orthossm_amd.ops import _v10_backward
+    S, chunk, mu = (1 << 31) - 200, 1 << 20, 0.9
+    n = (S + chunk - 1) // chunk
+    x = torch.zeros(1, S, 1, dtype=torch.bfloat16, device=dev)
+    out = torch.zeros(1, S, 1, device=dev)
+    hist = torch.zeros(n, 1, 1, 2, 1, device=dev)
+    hist[:, :, :, 1] = 1.0
+    gx, _ = _v10_backward(x, out, x, hist, torch.ones(1, device=dev).expand(1, S, 1), 1, mu, chunk, False)
+    left = torch.arange(3, 0, -1, dtype=torch.float64)
+    want = 0.98 * (1.0 - mu ** left)
+    for end in (S, S // chunk * chunk, chunk):
+        got = gx[0, end - 3:end, 0].double().cpu()
+        assert (got - want).abs().max() <= 2.0 ** -8 * want.max(), (end, got, want)
+
 S_LONG = 1 << 20
 
 

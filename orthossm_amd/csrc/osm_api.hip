@@ -493,7 +493,7 @@ Geometry lut_scan_shape(const osm_lut_fwd_args* a) {
   constexpr int64_t kCus = 256;
   const int tile = n_lb * tiles(osm::LutTile::TILE) >= kCus ? osm::LutTile::TILE : osm::LutTileSmall::TILE;
   const int64_t n_tiles = tiles(tile);
-  if (n_lb * n_tiles >= (int64_t(1) << 31)) return geo;
+  if (n_lb * n_tiles >= (int64_t(1) << 31) || a->S >= (int64_t(1) << 31) - tile) return geo;   // 32-bit token indices
   geo.n_lbd = (int)n_lbd;
   geo.n_lb = (int)n_lb;
   geo.n_tiles = (int)n_tiles;

@@ -345,6 +345,18 @@ def test_lut_scan_is_kept_from_outputs_in_place_of_inputs(kw, scan):
     assert (n > 0) == scan
 
 
+def test_lut_scan_ends_where_token_indices_would_pass_32_bits():
+    lib = nat.load()
+
+    def need(S):
+        return lib.osm_lut_fwd_workspace_bytes(ctypes.byref(_lut(
+            B=1, S=S, H=1, hd=1, ema_momentum=0.9, x_stride_s=1, x_stride_b=S, out=0x900000000000, out_stride_s=1,
+            out_stride_b=S)))
+
+    assert need(1 << 30) > 0 and need((1 << 31) - 129) > 0
+    assert need((1 << 31) - 128) == 0 and need((1 << 31) - 1) == 0
+
+
 def test_lut_fwd_empty_batch_is_a_no_op():
     # B = 0 returns before any pointer is looked at (no GPU work)
     lib = nat.load()

@@ -136,12 +136,14 @@ def _current_stream(dev: torch.device) -> int:
     return torch.cuda.current_stream(dev).cuda_stream
 
 
-# Whether the current stream of the current device is being captured.
+# Whether the current stream of the current device is being captured, and that
+# device (torch's C accessors where this torch has them, as above).
 _current_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing", torch.cuda.is_current_stream_capturing)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 
 
 def _capturing(dev: torch.device) -> bool:
-    if dev.index is None or dev.index == torch.cuda.current_device():
+    if dev.index is None or dev.index == _current_device():
         return _current_capturing()
     with torch.cuda.device(dev):
         return _current_capturing()

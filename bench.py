@@ -2,7 +2,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload W] [--no-others]
 
-Default workload: BASELINE configs[1] ("headline"): B=4, S=16384, D=512
+Default workload ("headline"): B=4, S=16384, D=512
 (H=8, hd=64), K=8, fp32, static per-head lambda.  One step = one pass of
 the fused operator over one batch held in HBM.  Inputs rotate over 4
 buffer sets (>1 GB) so the 256 MB Infinity Cache cannot serve them.
@@ -22,7 +22,7 @@ main kernel measured with rocprofv3's TCC->EA read and write request
 counters, by request size (profiles/hbm_traffic.json, written by
 ``--pmc-summary``).  ``cpu_baseline`` times the CPU restatement of the
 reference's PyTorch path (oracle/reference_form.py) on this host's cores:
-for the forward workloads BASELINE configs[0] and the workload in full,
+for the forward workloads B=1 S=2048 D=512 and the workload in full,
 otherwise one batch row; median of 3 runs after a warm-up.
 """
 from __future__ import annotations
@@ -96,8 +96,8 @@ def _median_time(run, reps: int = 3) -> float:
 
 def cpu_baseline(cfg):
     """The CPU restatement of the reference's PyTorch path on this host's
-    cores, median of 3 runs after one warm-up.  Forward workloads: BASELINE
-    configs[0] in full and the workload itself in full (the forward
+    cores, median of 3 runs after one warm-up.  Forward workloads:
+    B=1 S=2048 D=512 in full and the workload itself in full (the forward
     workloads at most 2^26 elements, a few seconds per run); the other
     workloads: one batch row of at most 16384 tokens."""
     from oracle import reference_form as RF
@@ -146,7 +146,7 @@ def cpu_baseline(cfg):
         "os_cpu_count": os.cpu_count(),
     }
     if forward_only and cfg.name != "cpu_ref":
-        # BASELINE configs[0] (B=1 S=2048 D=512), the reference's CPU-runnable case
+        # B=1 S=2048 D=512, the reference's CPU-runnable case
         c0 = CONFIGS["cpu_ref"]
         i0 = make_config_inputs(c0)
         t0 = _median_time(lambda: RF.forward(i0["x"], i0["coeffs"], i0["damping"], i0["lam"]))
@@ -363,7 +363,7 @@ def launch_figures(cfg, ms_per_step: float) -> dict:
 
 
 def other_workloads(skip: str, dev, stream, steps: int, warmup: int) -> dict:
-    """The other BASELINE workloads, each timed as the main one is (its own
+    """The other workloads, each timed as the main one is (its own
     warm-up, then ``steps`` steps between two events), on inputs drawn on
     the device, at most two buffer sets above 256 MB of x."""
     res = {}
@@ -540,7 +540,7 @@ def main():
         torch.cuda.synchronize()
         res["copy_calibration_bytes_each_way"] = xs[0].numel() * xs[0].element_size()
     if others:
-        # Each other BASELINE workload timed in the same run (100 warm-up
+        # Each other workload timed in the same run (100 warm-up
         # and 100 timed steps each), so that one run records all of them.
         del W, xs, outs, step
         torch.cuda.synchronize()

@@ -185,7 +185,7 @@ def test_backward_is_deterministic(dev):
 
 
 def test_backward_headline_linearity(dev):
-    # BASELINE configs[1] at full size: the backward is linear in
+    # B=4 S=16384 D=512 at full size: the backward is linear in
     # (dL/dout, dL/d ema_final), so bwd(g1) + bwd(g2) = bwd(g1 + g2).
     cfg = CONFIGS["headline"]
     inp = make_config_inputs(cfg)

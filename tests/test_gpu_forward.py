@@ -1,5 +1,5 @@
 """GPU parity of the fused forward (osm_cheby_ema_fwd through the C ABI)
-against the float64 oracle, at the BASELINE shapes and at edge cases."""
+against the float64 oracle, at the benchmark shapes and at edge cases."""
 import numpy as np
 import pytest
 import torch
@@ -179,7 +179,7 @@ def test_empty_sequence(dev):
 
 
 def test_headline_config_full_size(dev):
-    """configs[1]: B=4 S=16384 D=512 fp32, against the oracle at full size."""
+    """B=4 S=16384 D=512 fp32, against the oracle at full size."""
     inp = make_config_inputs(CONFIGS["headline"])
     out, fin = run(inp, dev, return_state=True)
     want, wfin = oracle_forward(inp)
@@ -188,7 +188,7 @@ def test_headline_config_full_size(dev):
 
 
 def test_streaming_config_full_size(dev):
-    """configs[2]: B=1 S=262144 as 16 chunks of 16384 with EMA carry == one
+    """B=1 S=262144 as 16 chunks of 16384 with EMA carry == one
     monolithic scan, and the monolithic scan == oracle."""
     cfg = CONFIGS["streaming"]
     inp = make_config_inputs(cfg)
@@ -209,7 +209,7 @@ def test_streaming_config_full_size(dev):
 
 
 def test_dynamic_config_full_size(dev):
-    """configs[3]: B=8 S=32768 D=1024 dynamic lambda, at full size: every
+    """B=8 S=32768 D=1024 dynamic lambda, at full size: every
     batch row (each an independent recurrence) is checked against the
     float64 oracle's C restatement (oracle/cheby_ema_c.c, pinned against the
     numpy oracle on the CPU), out and ema_final.  Measured on one MI355X box

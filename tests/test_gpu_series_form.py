@@ -26,7 +26,7 @@ pytestmark = pytest.mark.gpu
 
 
 def wide_inputs(B, S, H, hd, K, sigma, seed, dynamic=False, mixed=False, dtype=torch.float32):
-    """BASELINE-style inputs with c_k ~ N(0, sigma^2) for every k; with
+    """Benchmark-style inputs with c_k ~ N(0, sigma^2) for every k; with
     `mixed`, batch row 0 keeps the benchmark's N(0, 1/(k+1)^2)."""
     inp = inputs(B, S, H, hd, K, seed=seed, dynamic=dynamic, dtype=dtype)
     gen = torch.Generator().manual_seed(seed + 7)

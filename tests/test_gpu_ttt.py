@@ -33,7 +33,7 @@ def assert_grad(got, want, rtol=GRAD_RTOL):
 
 
 @pytest.mark.parametrize("B,S,H,hd,K,dyn,target", [
-    (1, 2048, 8, 64, 8, False, "x"),          # configs[0] shape
+    (1, 2048, 8, 64, 8, False, "x"),          # one short row
     (2, 1000, 8, 64, 8, True, "x"),
     (2, 777, 4, 32, 5, False, "softsign"),
     (1, 300, 3, 20, 8, True, "x"),            # partial lane-block
@@ -136,7 +136,7 @@ def test_ttt_deterministic(dev):
 
 
 def test_bf16_ttt_config_full_size(dev):
-    """configs[4]: B=16 S=65536 D=512, bf16 I/O, fp32 state, fused TTT, at
+    """B=16 S=65536 D=512, bf16 I/O, fp32 state, fused TTT, at
     full size: every batch row is compared with the float64 oracle's C
     restatement (oracle/cheby_ema_c.c, pinned against the numpy oracle on the
     CPU) run on that row with the loss mean over the whole batch: out (bf16,

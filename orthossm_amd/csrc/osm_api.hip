@@ -43,10 +43,11 @@ int ok() {
 // kFwdWords: 4 words (a checkpoint every 32 tiles) where few lane-blocks have
 // many tiles, so that the serial chain of checkpoints (~0.7 us each) is what
 // the launch waits for, else 1 (every 8 tiles), whose threads poll less.
-// Measured on MI355X, K=8, 1 word against 4: B=1 S=16384 D=256 16.8 and 11.0
-// us, S=65536 D=128 30.0 and 17.3, S=4096 D=256 8.5 and 7.4, S=16384 D=512 15.6
-// and 15.3 (8 lane-blocks); B=3 S=4000 D=384 (18) 11.2 and 11.4, dynamic
-// lambda B=3 S=6000 D=320 (15) 13.6 and 14.8.
+// Measured on MI355X, K=8, 1 word against 4: B=1 S=16384 D=256 18.1 and 12.3
+// us, S=65536 D=128 32.2 and 19.4, S=4096 D=256 8.5 and 7.3, S=16384 D=512 13.8
+// and 13.4 (8 lane-blocks), dynamic lambda S=30000 D=128 29.2 and 17.4, table
+// forward S=8192 D=128 18.9 and 11.7; B=3 S=4000 D=384 (18) 11.1 and 11.3,
+// dynamic lambda B=3 S=6000 D=320 (15) 14.7 and 14.9.
 int look_back_shift(int64_t n_lb, int64_t n_tiles) {
   return n_lb <= 8 && n_tiles >= 32 ? 2 : 0;
 }

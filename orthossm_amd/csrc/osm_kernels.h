@@ -67,7 +67,7 @@ using FwdTileSmall = TileGeo<2, 8, 8, 64, kFwdWords>;     // 128 tokens x 64 lan
 // coefficients take twice the registers.  Used only where the geometries
 // above do not apply.
 // (two versions of one shape: with room for kFwdWords words the many-tile
-// launches of 2-byte rows lose 1%: bf16 B=3 S=5001 D=400, 12.08 against 12.21 us)
+// launches of 2-byte rows lose 1%: bf16 B=3 S=5001 D=400, 12.8 against 12.9 us)
 using FwdTileGeneric = TileGeo<1, 8, 16, 64, 1>;             // 128 tokens x 64 lanes
 using FwdTileGenericFew = TileGeo<1, 8, 16, 64, kFwdWords>;  // few lane-blocks
 constexpr int kMaxTileRows = 512;              // bound on TILE (+1 row read past a tile)
@@ -357,9 +357,9 @@ struct V10FixedParams : V10Params {
 // The same forward as a single-pass scan over tiles (osm_lut.hip), chained by
 // the look-back: for 0.25 <= mu <= 1 and a caller's workspace.  128-token
 // tiles where they give every CU one, else 64 (a tile of 128 tokens holds
-// its CU's VALUs ~3.8 us): on MI355X, D=512 K=8, 8.5 against 10.5 us at B=4
-// S=512 (128 tiles of 128 tokens), 12.2 against 11.9 at B=2 S=2000 D=400
-// (224), 21.0 against 16.0 at B=2 S=4096 (512).  One lane per thread where
+// its CU's VALUs ~3.8 us): on MI355X, D=512 K=8, 64 tokens against 128, 9.4 and
+// 10.4 us at B=4 S=512 (128 tiles of 128 tokens), 12.0 and 12.1 at B=2 S=2000
+// D=400 (224), 21.3 and 15.2 at B=2 S=4096 (512).  One lane per thread where
 // rows are off two-element boundaries.
 using LutTile = TileGeo<2, 8, 8, 64, kFwdWords>;              // 128 tokens x 64 lanes
 using LutTileSmall = TileGeo<2, 8, 4, 64, kFwdWords>;         // 64 tokens

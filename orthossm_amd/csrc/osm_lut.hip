@@ -10,10 +10,10 @@
 // the first boundary publishes its state, clamped there, as a checkpoint, and
 // the tiles after it start their group from it.
 //
-// What bounds it: at large sizes HBM (16 bytes per element: 119 us at B=4
-// S=16384 D=512, 4.5 TB/s; the one-workgroup-per-lanes walk of osm_v10.hip
-// 234 us), at small ones the VALU work of one tile on one CU (~70
-// instructions per element) and the launch: 16.0 against 51.4 us at B=2
+// What bounds it: at large sizes HBM (16 bytes per element: 118 us at B=4
+// S=16384 D=512, 4.6 TB/s; the one-workgroup-per-lanes walk of osm_v10.hip
+// 234 us), at small ones the VALU work of one tile on one CU (65
+// instructions per element) and the launch: 15.5 against 51.4 us at B=2
 // S=4096 D=512, 8.0 against 8.7 at B=1 S=384.  The table gathers cost little
 // (15.1 us at B=2 S=4096 with the Clenshaw series in their place).
 #include "osm_tile.h"

@@ -203,7 +203,7 @@ osm::FwdParams make_params(const osm_cheby_args* a, const Geometry& geo, void* w
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
-  p.order = osm::tile_order(geo.n_lb, geo.n_tiles,
+  p.order = osm::tile_order(geo.n_lb, geo.n_tiles, geo.n_lbd,
                             in_place(a->ema_init, a->ema_final,
                                      Span(a->out, a->out_stride_b, a->out_stride_s, a->B, a->S, a->H * a->hd,
                                           a->out_dtype == OSM_F32 ? 4 : 2),
@@ -854,7 +854,7 @@ int osm_cheby_ema_lut_fwd_ws(const osm_lut_fwd_args* a, void* workspace, size_t 
   p.n_lbd = geo.n_lbd;
   p.n_lb = geo.n_lb;
   p.n_tiles = geo.n_tiles;
-  p.order = osm::tile_order(geo.n_lb, geo.n_tiles);
+  p.order = osm::tile_order(geo.n_lb, geo.n_tiles, geo.n_lbd);
   p.wsh = look_back_shift(geo.n_lb, geo.n_tiles);
   p.clamp_at = (int)((a->clamp_tile - 1) / geo.tile);
   p.jitter = (a->flags & OSM_FLAG_TIMING_JITTER) ? 1 : 0;
@@ -970,7 +970,7 @@ int osm_cheby_ema_bwd(const osm_cheby_args* args, const osm_cheby_bwd_args* bwd,
   if (rc != OSM_OK) return rc;
   osm::BwdParams bp{};
   bp.f = make_params(args, geo, workspace);
-  bp.f.order = osm::tile_order(geo.n_lb, geo.n_tiles,
+  bp.f.order = osm::tile_order(geo.n_lb, geo.n_tiles, geo.n_lbd,
                                in_place(bwd->grad_state, bwd->grad_init,
                                         Span(bwd->grad_x, bwd->gx_stride_b, bwd->gx_stride_s, args->B, args->S, D, xs),
                                         args->B, D));

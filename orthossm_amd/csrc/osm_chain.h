@@ -128,7 +128,7 @@ __device__ __forceinline__ TileInfo tile_info(const TileOrder& order, unsigned* 
     // (a drawn tile past the last: only where two launches share a workspace)
     ti.pad = ti.lb < 0 || (unsigned)ti.tile >= (unsigned)n_tiles;
   }
-  ti.b = ti.lb / n_lbd;
+  ti.b = SPREAD ? (int)order.by_row.of((unsigned)ti.lb) : ti.lb / n_lbd;
   ti.lbd = ti.lb - ti.b * n_lbd;
   ti.is_last = ti.tile == n_tiles - 1;
   ti.is_ckpt = ((ti.tile + 1) & ((G::WPS << wsh) - 1)) == 0;

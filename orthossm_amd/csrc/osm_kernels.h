@@ -176,6 +176,7 @@ struct TileOrder {
   int n_slots;       // spread, by index: blocks per tile row, a multiple of 8
   bool lead;         // spread: the first tile alone reads the initial state and publishes its own end state
   Divisor by_slots, by_whole, by_rest;   // n_slots; with tickets n_lb / 8 and n_lb % 8
+  Divisor by_row;    // spread: lane-blocks of a batch row
 };
 struct TileSlot {
   int tile;   // >= n_tiles: none; -1: the next of the lane-block, by its ticket counter
@@ -234,12 +235,13 @@ __host__ __device__ __forceinline__ TileSlot spread_slot(const TileOrder& o, uns
 // The tiles of the first look-back group read the initial state when they
 // resolve their carry, after they have published, so the last tile may be done
 // before them; with `lead` they take the first tile's published state instead.
-inline TileOrder tile_order(int64_t n_lb, int64_t n_tiles, bool state_in_place = false) {
+inline TileOrder tile_order(int64_t n_lb, int64_t n_tiles, int64_t n_lbd, bool state_in_place = false) {
   constexpr int64_t kCusPerXcd = 32;
   TileOrder o{};
   o.grid = (unsigned)(n_lb * n_tiles);
   if (n_tiles == 1 || (n_lb % 8 == 0 && !state_in_place)) return o;
   o.spread = true;
+  o.by_row = divisor(n_lbd);
   o.lead = state_in_place;
   const int64_t pad = (n_lb + 7) / 8 * 8, most = pad / 8 * n_tiles, surplus = most - n_lb * n_tiles / 8;
   if (most <= kCusPerXcd || surplus <= 12 || surplus <= most / 16) {

@@ -24,7 +24,7 @@ SRC = r"""
 #include <vector>
 #include "osm_kernels.h"
 static int check_order(int n_lb, int n_tiles, bool state_in_place) {
-  const osm::TileOrder o = osm::tile_order(n_lb, n_tiles, state_in_place);
+  const osm::TileOrder o = osm::tile_order(n_lb, n_tiles, 1, state_in_place);
   if (o.lead != (state_in_place && n_tiles > 1) || (o.lead && !o.spread)) return printf("FAIL lead n_lb=%d\n", n_lb);
   std::vector<long long> block((size_t)n_lb * n_tiles, -1);   // by index: who takes the tile
   std::vector<int> drawn(n_lb, 0);
